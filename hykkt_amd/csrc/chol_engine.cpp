@@ -182,7 +182,7 @@ void CholEngine::build_tasks()
   const int nlev = static_cast<int>(pl_.level_ptr.size()) - 1;
   lv_.assign(nlev, Level{});
   std::vector<int> eap, eacol, eacptr{0}, eacc, eaccol;
-  std::vector<int> potrf, trsm_sn, trsm_tr, trsm_tc, upd_sn, upd_tr, upd_tc;
+  std::vector<int> potrf, trsm_sn, trsm_tr, upd_sn, upd_tr, upd_tc;
   std::vector<int> syrk_sn, syrk_tr, syrk_tc, inv_sn, inv_step;
   struct Contrib {
     int t, c, r2;
@@ -321,7 +321,6 @@ void CholEngine::build_tasks()
         for (int t = 0; t < cdiv(f - (k0 + b), rows_unit); t++) {
           trsm_sn.push_back(s);
           trsm_tr.push_back(t);
-          trsm_tc.push_back(0);
         }
       }
       L.potrf[j].cnt = static_cast<int>(potrf.size()) - L.potrf[j].off;
@@ -411,7 +410,6 @@ void CholEngine::build_tasks()
   up(t_potrf_, potrf);
   up(t_trsm_sn_, trsm_sn);
   up(t_trsm_tr_, trsm_tr);
-  up(t_trsm_tc_, trsm_tc);
   up(t_upd_sn_, upd_sn);
   up(t_upd_tr_, upd_tr);
   up(t_upd_tc_, upd_tc);
@@ -598,9 +596,8 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt)
         });
       } else {
         timed(L.trsm[j].short_rows ? PK_DENSE_NT_SHORT : PK_DENSE_NT, L.trsm[j], [&] {
-          dev::dense_nt(cd_, L.trsm[j].cnt, t_trsm_sn_.p + L.trsm[j].off,
-                        t_trsm_tr_.p + L.trsm[j].off, t_trsm_tc_.p + L.trsm[j].off, 2, step, b,
-                        st_, L.trsm[j].short_rows);
+          dev::trsm_inv(cd_, L.trsm[j].cnt, t_trsm_sn_.p + L.trsm[j].off,
+                        t_trsm_tr_.p + L.trsm[j].off, step, b, st_, L.trsm[j].short_rows);
         });
       }
       if (rest_pending && upd_hi >= rest_lo) {

@@ -212,7 +212,7 @@ class CholEngine {
   // task lists
   std::vector<Level> lv_;
   DevBuf<int> t_ea_p_, t_ea_col_, t_ea_cptr_, t_ea_cc_, t_ea_ccol_;
-  DevBuf<int> t_potrf_, t_trsm_sn_, t_trsm_tr_, t_trsm_tc_, t_upd_sn_, t_upd_tr_, t_upd_tc_;
+  DevBuf<int> t_potrf_, t_trsm_sn_, t_trsm_tr_, t_upd_sn_, t_upd_tr_, t_upd_tc_;
   DevBuf<int> t_syrk_sn_, t_syrk_tr_, t_syrk_tc_;
   DevBuf<int> t_inv_sn_, t_inv_step_;
   int n_cu_ = 1;   // compute units: persistent-launch width

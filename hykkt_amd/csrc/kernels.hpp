@@ -256,15 +256,18 @@ void trsm(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr, 
 void inv_blocks(const CholDev& c, int ntasks, const int* task_sn, const int* task_step,
                 const Batch& b, hipStream_t st);
 
-// MFMA tile kernel over (supernode, tile row, tile col) tasks.  mode 0: trailing
-// panel update after block `step`; mode 1: U = -L21 L21^T; mode 2: TRSM of the
-// rows below block `step` with its inverted diagonal block; mode m >= 3: as
-// mode 0 by blocks step .. step+m-2.  short_rows: 32-row x 128-column tiles,
-// tile rows counted in 32-row units (modes 0, 2, 3+).  done: an event the
-// launch records on completion (nullptr: none).
+// MFMA update tiles over (supernode, tile row, tile col) tasks.  mode 0: trailing
+// panel update after block `step`; mode 1: U = -L21 L21^T; mode m >= 3: as mode 0
+// after blocks `step` .. `step`+m-2 (K = (m-1) blocks).  Tiles of 128 x 128, or
+// of 32 rows x 128 columns (short_rows; modes 0 and >= 3).  done: optional event
+// recorded by the launch's own completion.
 void dense_nt(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr,
               const int* task_tc, int mode, int step, const Batch& b, hipStream_t st,
               bool short_rows = false, hipEvent_t done = nullptr);
+// TRSM of the rows below blocks of at most 64 columns with their whole inverses,
+// in place (tasks as trsm()'s).
+void trsm_inv(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr, int step,
+              const Batch& b, hipStream_t st, bool short_rows);
 
 // Single-launch supernodal solves over the whole tree.  Work items are
 // 128-row blocks of the fronts, dispatched in a dependency-respecting order;

@@ -1,6 +1,6 @@
 // kernels_dense.hip -- dense FP64 kernels of the supernodal Cholesky on
-// gfx950: 128x128-tile NT-GEMM on the matrix cores (v_mfma_f64_16x16x4f64),
-// and the factorization + inversion of 128x128 diagonal blocks.
+// gfx950: NT-GEMM updates on the matrix cores (v_mfma_f64_16x16x4f64), and the
+// factorization + inversion of 128x128 diagonal blocks.
 //
 // MFMA f64 16x16x4 operand layout on gfx950 (lane l, 64 lanes):
 //   A operand: A[i = l%16][k = l/16];  B operand: B[k = l/16][j = l%16];
@@ -29,22 +29,6 @@ constexpr int BT = 128;        // tile edge (rows and columns of C)
 constexpr int KC = 16;         // K chunk staged in LDS
 constexpr int LDA_S = BT + 2;  // LDS row length (doubles)
 
-// Global loads and stores of factor data.  COH: device-scope relaxed atomics
-// (coherent across the XCDs' L2 caches), for data another workgroup of the
-// same launch produced or will consume.
-template <bool COH>
-__device__ __forceinline__ double ldg(const double* p)
-{
-  if constexpr (COH) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else return *p;
-}
-template <bool COH>
-__device__ __forceinline__ void stg(double* p, double v)
-{
-  if constexpr (COH) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else *p = v;
-}
-
 struct GemmArgs {
   const double* A;
   int64_t lda;
@@ -52,21 +36,15 @@ struct GemmArgs {
   int64_t ldb;
   double* C;
   int64_t ldc;
-  int M, N, K;       // C is M x N (tile-local bounds), K inner
-  double alpha, beta;
-  // pk > 0: C is the pk x pk lower triangle packed by columns and the tile
-  // sits at (pr0, pc0) in it; entries above the diagonal are not stored
-  int64_t pk = 0, pr0 = 0, pc0 = 0;
+  int M, N, K;   // C is M x N (tile-local bounds), K inner
 };
 
-// One TM x TN tile of C = beta*C + alpha*A*B^T with beta in {0, 1} and
-// alpha in {1, -1}.  256 threads: 4 waves in a WM x WN arrangement (2x2 for
-// 128x128 tiles, 1x4 for 32x128), each owning a QM x QN block of IM x JN
-// MFMA tiles.  The accumulators start from beta*C (all loads in flight at
-// once) and are stored once at the end; alpha is applied exactly to the
-// staged A values.  K is staged through LDS in chunks of KC, the next chunk's
-// global loads overlapping the current chunk's MFMAs.
-template <int TM, int TN, bool COH = false>
+// One TM x TN tile of C = A*B^T.  256 threads: 4 waves in a WM x WN
+// arrangement (2x2 for 128x128 tiles, 1x4 for 32x128), each owning a QM x QN
+// block of IM x JN MFMA tiles, stored once at the end.  K is staged through
+// LDS in chunks of KC, the next chunk's global loads overlapping the current
+// chunk's MFMAs.
+template <int TM, int TN>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, double* smem)
 {
   constexpr int WN = TM == TN ? 2 : 4, WM = 4 / WN;
@@ -80,24 +58,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, double* smem)
   const int wr = (wave / WN) * QM, wc = (wave % WN) * QN;
   d4 acc[IM][JN];
   // acc[i][j][v]: C row = wr + 16 i + lane%16, C col = wc + 16 j + 4 v + lane/16
-  if (g.beta != 0.0) {
 #pragma unroll
-    for (int i = 0; i < IM; i++) {
-      const int r = wr + i * 16 + (lane & 15);
+  for (int i = 0; i < IM; i++)
 #pragma unroll
-      for (int j = 0; j < JN; j++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int c = wc + j * 16 + 4 * v + (lane >> 4);
-          acc[i][j][v] = (r < g.M && c < g.N) ? ldg<COH>(g.C + c * g.ldc + r) : 0.0;
-        }
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < IM; i++)
-#pragma unroll
-      for (int j = 0; j < JN; j++) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-  }
+    for (int j = 0; j < JN; j++) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
 
   // staging assignment: thread t loads k = t/16, rows t%16 + 16 q (q < E): the
   // 16 lanes of a k write 16 consecutive LDS words (no bank conflicts)
@@ -108,19 +72,19 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, double* smem)
 #pragma unroll
     for (int q = 0; q < EA; q++) {
       const int r = sa + 16 * q;
-      ra[q] = (kk < g.K && r < g.M) ? ldg<COH>(g.A + kk * g.lda + r) : 0.0;
+      ra[q] = (kk < g.K && r < g.M) ? g.A[kk * g.lda + r] : 0.0;
     }
 #pragma unroll
     for (int q = 0; q < EB; q++) {
       const int r = sb + 16 * q;
-      rb[q] = (kk < g.K && r < g.N) ? ldg<COH>(g.B + kk * g.ldb + r) : 0.0;
+      rb[q] = (kk < g.K && r < g.N) ? g.B[kk * g.ldb + r] : 0.0;
     }
   };
   gload(0);
   for (int k0 = 0; k0 < g.K; k0 += KC) {
     __syncthreads();   // the previous chunk's fragments have been read
 #pragma unroll
-    for (int q = 0; q < EA; q++) As[sk * LA + sa + 16 * q] = g.alpha * ra[q];   // exact: alpha is +-1
+    for (int q = 0; q < EA; q++) As[sk * LA + sa + 16 * q] = ra[q];
 #pragma unroll
     for (int q = 0; q < EB; q++) Bs[sk * LB + sb + 16 * q] = rb[q];
     __syncthreads();
@@ -140,21 +104,6 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, double* smem)
           acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[j], fa[i], acc[i][j], 0, 0, 0);
     }
   }
-  if (g.pk > 0) {
-#pragma unroll
-    for (int i = 0; i < IM; i++) {
-      const int r = wr + i * 16 + (lane & 15);
-#pragma unroll
-      for (int j = 0; j < JN; j++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int c = wc + j * 16 + 4 * v + (lane >> 4);
-          const int64_t gr = g.pr0 + r, gc = g.pc0 + c;
-          if (r < g.M && c < g.N && gr >= gc) stg<COH>(g.C + packed_lower(gr, gc, g.pk), acc[i][j][v]);
-        }
-    }
-    return;
-  }
 #pragma unroll
   for (int i = 0; i < IM; i++) {
     const int r = wr + i * 16 + (lane & 15);
@@ -163,7 +112,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, double* smem)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const int c = wc + j * 16 + 4 * v + (lane >> 4);
-        if (r < g.M && c < g.N) stg<COH>(g.C + c * g.ldc + r, acc[i][j][v]);
+        if (r < g.M && c < g.N) g.C[c * g.ldc + r] = acc[i][j][v];
       }
   }
 }
@@ -184,79 +133,274 @@ __device__ __forceinline__ SnInfo sninfo(const CholDev& c, double* L, int s)
   return i;
 }
 
+// ------------------------------------------------------------- updates
+// Buffer descriptors over factor data: a uniform base, so a load costs one
+// 32-bit offset register, and a byte limit past which loads return 0 (word 3:
+// the gfx9-family raw-buffer setting).
+using rsrc_t = __amdgpu_buffer_rsrc_t;
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+constexpr uint32_t VIEW_MAX = 0x7fffffffu;
+constexpr uint32_t OFF_NONE = 0x80000000u;   // past every view: the load returns 0
+
+__device__ __forceinline__ int64_t uni64(int64_t v)
+{
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+  const uint32_t hi =
+      __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(v) >> 32));
+  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ __forceinline__ rsrc_t view(const double* base, int64_t bytes)
+{
+  const int64_t n = bytes < 0 ? 0 : (bytes > VIEW_MAX ? VIEW_MAX : bytes);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<double*>(base), 0, static_cast<uint32_t>(n),
+                                           0x00020000);
+}
+
+// Row (column) of group g's element m (0..15) within a wave's block of CNT
+// groups of 16: with an even CNT the groups come in pairs of interleaved rows,
+// so the two groups' values of a lane are adjacent in memory (one 16-byte
+// load or store instead of two of 8 bytes).
+template <int CNT>
+__device__ __forceinline__ constexpr int grow16(int g, int m)
+{
+  return CNT % 2 == 0 ? (g / 2) * 32 + 2 * m + (g & 1) : 16 * g + m;
+}
+
+// A lane's values of CNT groups of 16 rows of one matrix column (k), from the
+// view whose element (0, k) is at byte offset vo (the lane's row included).
+template <int CNT>
+__device__ __forceinline__ void frag_load(double (&v)[CNT], rsrc_t r, uint32_t vo)
+{
+  if constexpr (CNT % 2 == 0) {
+#pragma unroll
+    for (int g = 0; g < CNT; g += 2) {
+      const d2 t = __builtin_bit_cast(d2, __builtin_amdgcn_raw_buffer_load_b128(r, vo, g * 128, 0));
+      v[g] = t[0];
+      v[g + 1] = t[1];
+    }
+  } else {
+#pragma unroll
+    for (int g = 0; g < CNT; g++)
+      v[g] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, vo, g * 128, 0));
+  }
+}
+
 // mode 0: trailing panel update after block `step`   C = C - A A^T (K = block)
 // mode 1: update matrix U = -L21 L21^T                 (K = nc, U overwritten)
-// mode 2: TRSM L21(block) = A21 * Dinv^T               (K = block, in place)
 // mode m >= 3: as mode 0 after blocks `step` .. `step`+m-2 (K = m-1 blocks)
-// TM = 128: 128x128 tiles (all modes).  TM = 32: 32-row x 128-column tiles
-// (modes 0 and 2), four times as many workgroups for the short launches on
-// the critical path (the TRSM and the next-column update of a step with few
-// tiles).  System blockIdx.y.
-template <int TM>
-__global__ void __launch_bounds__(256, 2) k_dense_nt(CholDev c, const int* __restrict__ tsn,
-                                                  const int* __restrict__ ttr,
-                                                  const int* __restrict__ ttc, int mode, int step,
-                                                  Batch bt)
+//
+// Each wave holds a (16 IM) x (16 JN) block of C in accumulators and reads its
+// A and B fragments straight from global memory into registers, D K-steps (of
+// 4) ahead of the MFMAs that use them: no LDS, no barriers, so the waves of a
+// CU never wait for each other and the whole LDS stays free for the chain's
+// kernels (a diagonal block fits beside two update tiles).  A fragment read
+// by two waves of a tile comes from L1/L2 the second time.  The updates are
+// bound by the FP64 matrix cores: on a 12288 x 12288 C, K = 1024 / 512 / 256 /
+// 128 run at 72 / 68 / 60 / 47 TFLOP/s (LDS-staged with two barriers per 16
+// K-steps: 60 / 56 / 50 / 40; LDS double-buffered, one barrier: 67 / 64 / 57 /
+// 49); at small K the C traffic takes over.  D = 2 leaves the 128 x 128 tile
+// at two waves per SIMD with registers over for a diagonal block.
+//
+// Every C entry starts from its old value (modes 0, >= 3) or 0 and takes the
+// MFMAs of K in ascending order, whatever the tile shape.  Rows and columns of
+// a tile past the panel compute values that are not stored (their loads stay
+// in the panel, or return 0 past its end); K steps past K read 0 for both
+// operands.
+//
+// Four waves, WN of them along the columns, on TM rows; a tile's 128 columns are
+// split over gridDim.z workgroups of 16 JN WN columns.  System blockIdx.y.
+template <int TM, int IM, int JN, int WN, int D>
+__global__ void __launch_bounds__(256, 2)
+    k_dense_nt(CholDev c, const int* __restrict__ tsn, const int* __restrict__ ttr,
+               const int* __restrict__ ttc, int mode, int step, Batch bt)
 {
+  constexpr int QM = 16 * IM, QN = 16 * JN, TN = QN * WN;
+  static_assert(TM / QM * WN == 4, "four waves");
   // the 32-row launches are the factorization's critical chain: their waves
   // take issue priority over the trailing updates they share SIMDs with
   if constexpr (TM == 32) __builtin_amdgcn_s_setprio(3);
+  const int sy = batch_sys(bt);
+  if (sy < 0) return;
+  const int s = uni(tsn[blockIdx.x]), tr = uni(ttr[blockIdx.x]), tc = uni(ttc[blockIdx.x]);
+  const int nc = uni(c.sn_first[s + 1] - c.sn_first[s]);
+  const int nr = uni(c.rows_ptr[s + 1] - c.rows_ptr[s]);
+  const int f = nc + nr;
+  const double* Ls = batch_at(c.L, sy, bt) + uni64(c.l_off[s]);
+  // end of the views: the panel's last entry and the one after it (the second
+  // row of a pair; the storage goes on there)
+  const double* panel_end = Ls + static_cast<int64_t>(f) * nc + 1;
+  const int zc = static_cast<int>(blockIdx.z) * TN;
+  // this workgroup's rows and columns of the front (R0, C0), the first column
+  // of the K range and K; M, N: valid rows and columns
+  int R0, C0, ka, K, M, N;
+  if (mode == 1) {
+    R0 = nc + tr * TM;
+    C0 = nc + tc * BT + zc;
+    ka = 0;
+    K = nc;
+    M = min(TM, f - R0);
+    N = min(TN, f - C0);
+  } else {
+    ka = step * BT;
+    K = min(mode >= 3 ? (mode - 1) * BT : BT, nc - ka);
+    R0 = ka + K + tr * TM;
+    C0 = ka + K + tc * BT + zc;
+    M = min(TM, f - R0);
+    N = min(TN, nc - C0);
+  }
+  if (M <= 0 || N <= 0) return;
+  const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
+  const int m16 = lane & 15, q4 = lane >> 4;
+  const int wr = (wave / WN) * QM, wc = (wave % WN) * QN;
+  const uint32_t f8 = static_cast<uint32_t>(f) * 8u;
+
+  // fragments of K-step s: A(R0 + wr + row, ka + 4 s + q4), the same for B
+  double fa[D][IM], fb[D][JN];
+  const double* pa = Ls + static_cast<int64_t>(ka) * f + R0 + wr;
+  const double* pb = Ls + static_cast<int64_t>(ka) * f + C0 + wc;
+  const uint32_t va = q4 * f8 + grow16<IM>(0, m16) * 8u, vb = q4 * f8 + grow16<JN>(0, m16) * 8u;
+  const int64_t dk = 4 * static_cast<int64_t>(f);
+  auto load = [&](int d, bool in) {   // the next K-step into buffer d
+    frag_load<IM>(fa[d], view(pa, 8 * (panel_end - pa)), in ? va : OFF_NONE);
+    frag_load<JN>(fb[d], view(pb, 8 * (panel_end - pb)), in ? vb : OFF_NONE);
+    pa += dk;
+    pb += dk;
+  };
+#pragma unroll
+  for (int d = 0; d < D; d++) load(d, 4 * d + q4 < K);
+
+  // acc[i][j][v]: C row wr + grow16<IM>(i, m16), column wc + grow16<JN>(j, 4 v + q4)
+  d4 acc[IM][JN];
+  const double* Cp = Ls + static_cast<int64_t>(C0 + wc) * f + R0 + wr;
+  const uint32_t vc = grow16<JN>(0, q4) * f8 + grow16<IM>(0, m16) * 8u;
+  auto coff = [&](int j, int v) { return static_cast<uint32_t>(grow16<JN>(j, 4 * v)) * f8; };
+  if (mode != 1) {
+    const rsrc_t rc = view(Cp, 8 * (panel_end - Cp));
+#pragma unroll
+    for (int j = 0; j < JN; j++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        double t[IM];
+        frag_load<IM>(t, rc, vc + coff(j, v));
+#pragma unroll
+        for (int i = 0; i < IM; i++) acc[i][j][v] = t[i];
+      }
+  } else {
+#pragma unroll
+    for (int i = 0; i < IM; i++)
+#pragma unroll
+      for (int j = 0; j < JN; j++) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+  }
+
+  auto mm = [&](int d) {
+#pragma unroll
+    for (int i = 0; i < IM; i++)
+#pragma unroll
+      for (int j = 0; j < JN; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[d][j], -fa[d][i], acc[i][j], 0, 0, 0);
+  };
+  const int nk = (K + 3) / 4, kfull = K / 4;   // K-steps; those with all four columns
+  int k = 0;
+  for (; k + 2 * D <= kfull; k += D) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      mm(d);
+      load(d, true);
+    }
+  }
+  for (; k < nk; k += D) {
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      mm(d);
+      if (k + D < nk) load(d, 4 * (k + D + d) + q4 < K);
+    }
+  }
+
+  if (mode == 1) {
+    // U packed by columns, entries on or below its diagonal
+    double* U = batch_at(c.U, sy, bt) + uni64(c.u_off[s]);
+    const int gr0 = R0 - nc + wr, gc0 = C0 - nc + wc;
+    const bool whole = M == TM && N == TN && gr0 >= gc0 + QN;   // no entry to leave out
+#pragma unroll
+    for (int j = 0; j < JN; j++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int cl = grow16<JN>(j, 4 * v) + grow16<JN>(0, q4), gc = gc0 + cl;
+        double* col = U + packed_lower(gr0, gc, nr);   // row gr0 of column gc
+        if (whole) {
+#pragma unroll
+          for (int i = 0; i < IM; i++) col[grow16<IM>(i, m16)] = acc[i][j][v];
+        } else {
+#pragma unroll
+          for (int i = 0; i < IM; i++) {
+            const int r = grow16<IM>(i, m16);
+            if (wr + r < M && wc + cl < N && gr0 + r >= gc) col[r] = acc[i][j][v];
+          }
+        }
+      }
+    return;
+  }
+  double* Cw = const_cast<double*>(Cp);
+  const bool whole = M == TM && N == TN;
+#pragma unroll
+  for (int j = 0; j < JN; j++)
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const int cl = grow16<JN>(j, 4 * v) + grow16<JN>(0, q4);
+      double* col = Cw + static_cast<int64_t>(cl) * f;
+      if (whole) {
+        // pairs of rows: 16-byte stores (8-byte aligned, as the panel is)
+        if constexpr (IM % 2 == 0) {
+          typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+#pragma unroll
+          for (int i = 0; i < IM; i += 2)
+            *reinterpret_cast<d2u*>(col + grow16<IM>(i, m16)) = d2u{acc[i][j][v], acc[i + 1][j][v]};
+        } else {
+#pragma unroll
+          for (int i = 0; i < IM; i++) col[grow16<IM>(i, m16)] = acc[i][j][v];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < IM; i++) {
+          const int r = grow16<IM>(i, m16);
+          if (wr + r < M && wc + cl < N) col[r] = acc[i][j][v];
+        }
+      }
+    }
+}
+
+// TRSM below a diagonal block with its whole inverse (blocks of at most 64
+// columns), in place: L21(block) = A21 * Dinv^T (K = block).  TM rows per
+// tile (32 or 128).  The operands go through LDS (gemm_tile), so every read of
+// a tile comes before its stores.  System blockIdx.y.
+template <int TM>
+__global__ void __launch_bounds__(256, 2) k_trsm_inv(CholDev c, const int* __restrict__ tsn,
+                                                     const int* __restrict__ ttr, int step,
+                                                     Batch bt)
+{
+  if constexpr (TM == 32) __builtin_amdgcn_s_setprio(3);   // see k_dense_nt
   extern __shared__ double smem[];
   const int sy = batch_sys(bt);
   if (sy < 0) return;
   const SnInfo si = sninfo(c, batch_at(c.L, sy, bt), tsn[blockIdx.x]);
-  const int tr = ttr[blockIdx.x], tc = ttc[blockIdx.x];
+  const int k0 = step * BT;
+  const int b = min(BT, si.nc - k0);
+  const int R0 = k0 + b + ttr[blockIdx.x] * TM;
+  double* panel = si.Ls + static_cast<int64_t>(k0) * si.f;   // columns k0..k0+b
   GemmArgs g;
-  if (mode == 1) {
-    const double* L21 = si.Ls + si.nc;
-    const int R0 = tr * BT, C0 = tc * BT;
-    g.A = L21 + R0;
-    g.B = L21 + C0;
-    g.lda = g.ldb = si.f;
-    g.C = batch_at(c.U, sy, bt) + c.u_off[tsn[blockIdx.x]];   // packed lower triangle of U
-    g.ldc = si.nr;
-    g.pk = si.nr;
-    g.pr0 = R0;
-    g.pc0 = C0;
-    g.M = min(BT, si.nr - R0);
-    g.N = min(BT, si.nr - C0);
-    g.K = si.nc;
-    g.alpha = -1.0;
-    g.beta = 0.0;
-  } else {
-    const int k0 = step * BT;
-    // modes 3 and up: the update by blocks step .. step + mode - 2 together
-    const int b = min(mode >= 3 ? (mode - 1) * BT : BT, si.nc - k0);
-    const int cs = k0 + b;
-    double* panel = si.Ls + static_cast<int64_t>(k0) * si.f;   // columns k0..k0+b
-    if (mode != 2) {
-      const int R0 = cs + tr * TM, C0 = cs + tc * BT;
-      g.A = panel + R0;
-      g.B = panel + C0;
-      g.lda = g.ldb = si.f;
-      g.C = si.Ls + static_cast<int64_t>(C0) * si.f + R0;
-      g.ldc = si.f;
-      g.M = min(TM, si.f - R0);
-      g.N = min(BT, si.nc - C0);
-      g.K = b;
-      g.alpha = -1.0;
-      g.beta = 1.0;
-    } else {
-      const int R0 = cs + tr * TM;
-      g.A = panel + R0;
-      g.lda = si.f;
-      g.B = batch_at(c.dinv, sy, bt) + c.dinv_off[tsn[blockIdx.x]] +
-            static_cast<int64_t>(step) * BT * BT;
-      g.ldb = BT;
-      g.C = panel + R0;
-      g.ldc = si.f;
-      g.M = min(TM, si.f - R0);
-      g.N = b;
-      g.K = b;
-      g.alpha = 1.0;
-      g.beta = 0.0;
-    }
-  }
+  g.A = panel + R0;
+  g.lda = si.f;
+  g.B = batch_at(c.dinv, sy, bt) + c.dinv_off[tsn[blockIdx.x]] +
+        static_cast<int64_t>(step) * BT * BT;
+  g.ldb = BT;
+  g.C = panel + R0;
+  g.ldc = si.f;
+  g.M = min(TM, si.f - R0);
+  g.N = b;
+  g.K = b;
   if (g.M <= 0 || g.N <= 0) return;
   gemm_tile<TM, BT>(g, smem);
 }
@@ -522,7 +666,7 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
       int r, col;
       lower_entry<BK>(min(tid + u * 256, NL - 1), r, col);
       const bool in = r < b;
-      const double t = ldg<false>(D + (in ? r + static_cast<int64_t>(col) * si.f : 0));
+      const double t = D[in ? r + static_cast<int64_t>(col) * si.f : 0];
       v[u] = in ? t : (r == col ? 1.0 : 0.0);
     }
 #pragma unroll
@@ -635,7 +779,7 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
     const int e = tid + u * 256;
     lower_entry<BK>(min(e, NL - 1), r, col);
     const double lv = P[r][col];
-    if (e < NL && r < b) stg<false>(D + r + static_cast<int64_t>(col) * si.f, lv);
+    if (e < NL && r < b) D[r + static_cast<int64_t>(col) * si.f] = lv;
   }
 
   // ---- inverse: the 16x16 diagonal blocks (16 lanes each), then doubling ----
@@ -883,20 +1027,32 @@ __global__ void __launch_bounds__(256) k_trsm(CholDev c, const int* __restrict__
 
 }  // namespace
 
-size_t dense_nt_smem() { return 2 * KC * LDA_S * sizeof(double); }
+// Columns of a 32-row update tile per workgroup: see k_dense_nt's launch below.
+constexpr int SHORT_TN = 64;
+
 void dense_nt(const CholDev& c, int ntasks, const int* tsn, const int* ttr, const int* ttc,
               int mode, int step, const Batch& b, hipStream_t st, bool short_rows, hipEvent_t done)
 {
   if (ntasks <= 0 || b.count <= 0) return;
-  const dim3 grid(ntasks, b.count);
   // `done` rides on the launch itself (its completion signal), so no marker
   // of its own sits between this kernel and the next one of the stream
   if (short_rows)
-    hipExtLaunchKernelGGL(k_dense_nt<32>, grid, dim3(256), dense_nt_smem(), st, nullptr, done, 0,
-                          c, tsn, ttr, ttc, mode, step, b);
+    hipExtLaunchKernelGGL((k_dense_nt<32, 2, 1, 4, 8>), dim3(ntasks, b.count, BT / SHORT_TN),
+                          dim3(256), 0, st, nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
   else
-    hipExtLaunchKernelGGL(k_dense_nt<128>, grid, dim3(256), dense_nt_smem(), st, nullptr, done, 0,
-                          c, tsn, ttr, ttc, mode, step, b);
+    hipExtLaunchKernelGGL((k_dense_nt<128, 4, 4, 2, 2>), dim3(ntasks, b.count), dim3(256), 0, st,
+                          nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
+  HIPCHK(hipGetLastError());
+}
+
+void trsm_inv(const CholDev& c, int ntasks, const int* tsn, const int* ttr, int step,
+              const Batch& b, hipStream_t st, bool short_rows)
+{
+  if (ntasks <= 0 || b.count <= 0) return;
+  constexpr size_t SM = 2 * KC * LDA_S * sizeof(double);
+  const dim3 grid(ntasks, b.count);
+  if (short_rows) k_trsm_inv<32><<<grid, 256, SM, st>>>(c, tsn, ttr, step, b);
+  else k_trsm_inv<128><<<grid, 256, SM, st>>>(c, tsn, ttr, step, b);
   HIPCHK(hipGetLastError());
 }
 
