@@ -620,7 +620,8 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt)
         timed_on(st2_, PK_DENSE_NT, L.upd_rest[j], [&] {
           dev::dense_nt(cd_, L.upd_rest[j].cnt, t_upd_sn_.p + L.upd_rest[j].off,
                         t_upd_tr_.p + L.upd_rest[j].off, t_upd_tc_.p + L.upd_rest[j].off, umode,
-                        ustep, b, st2_, false, ev_rest_);
+                        ustep, b, st2_, false, ev_rest_,
+                        L.upd_rest[j].cnt * b.count <= 2 * n_cu_);   // all resident at once
         });
         rest_pending = true;
         rest_lo = std::min(rest_lo, upd_hi + 1);   // the rest starts after the columns just updated

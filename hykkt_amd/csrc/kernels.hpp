@@ -260,10 +260,11 @@ void inv_blocks(const CholDev& c, int ntasks, const int* task_sn, const int* tas
 // panel update after block `step`; mode 1: U = -L21 L21^T; mode m >= 3: as mode 0
 // after blocks `step` .. `step`+m-2 (K = (m-1) blocks).  Tiles of 128 x 128, or
 // of 32 rows x 128 columns (short_rows; modes 0 and >= 3).  done: optional event
-// recorded by the launch's own completion.
+// recorded by the launch's own completion.  alone: 128 x 128 tiles keep off a
+// compute unit that factors a 128-wide diagonal block.
 void dense_nt(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr,
               const int* task_tc, int mode, int step, const Batch& b, hipStream_t st,
-              bool short_rows = false, hipEvent_t done = nullptr);
+              bool short_rows = false, hipEvent_t done = nullptr, bool alone = false);
 // TRSM of the rows below blocks of at most 64 columns with their whole inverses,
 // in place (tasks as trsm()'s).
 void trsm_inv(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr, int step,

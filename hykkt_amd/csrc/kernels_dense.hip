@@ -1029,9 +1029,18 @@ __global__ void __launch_bounds__(256) k_trsm(CholDev c, const int* __restrict__
 
 // Columns of a 32-row update tile per workgroup: see k_dense_nt's launch below.
 constexpr int SHORT_TN = 64;
+// LDS that keeps an update tile off the compute unit of a 128-wide diagonal
+// block (130 of the 160 KB), for launches small enough to find room elsewhere:
+// FP64 VALU instructions wait for the matrix instructions of the waves they
+// share a SIMD with, and a diagonal block beside a tile takes 46 us instead of
+// 28.  A big trailing update keeps no LDS: its tiles fill every compute unit
+// for longer than the block would wait (5,000 buses: factor 3.47 -> 3.36 ms,
+// 10,000: 11.3 -> 11.16; with the LDS for every launch 20,000: 51.1 -> 51.9).
+constexpr size_t ALONE_LDS = 31 * 1024;
 
 void dense_nt(const CholDev& c, int ntasks, const int* tsn, const int* ttr, const int* ttc,
-              int mode, int step, const Batch& b, hipStream_t st, bool short_rows, hipEvent_t done)
+              int mode, int step, const Batch& b, hipStream_t st, bool short_rows, hipEvent_t done,
+              bool alone)
 {
   if (ntasks <= 0 || b.count <= 0) return;
   // `done` rides on the launch itself (its completion signal), so no marker
@@ -1040,8 +1049,8 @@ void dense_nt(const CholDev& c, int ntasks, const int* tsn, const int* ttr, cons
     hipExtLaunchKernelGGL((k_dense_nt<32, 2, 1, 4, 8>), dim3(ntasks, b.count, BT / SHORT_TN),
                           dim3(256), 0, st, nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
   else
-    hipExtLaunchKernelGGL((k_dense_nt<128, 4, 4, 2, 2>), dim3(ntasks, b.count), dim3(256), 0, st,
-                          nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
+    hipExtLaunchKernelGGL((k_dense_nt<128, 4, 4, 2, 2>), dim3(ntasks, b.count), dim3(256),
+                          alone ? ALONE_LDS : 0, st, nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
   HIPCHK(hipGetLastError());
 }
 
