@@ -31,7 +31,7 @@ inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 CholEngine::CholEngine(const Pattern& a, const CholOptions& opt, hipStream_t st) : st_(st)
 {
-  HIPCHK(hipStreamCreate(&st2_));   // default priority, like the solver's stream
+  pick_second_stream();
   // the two streams' events order work on this device only: a device-scope
   // release, no system-scope cache writeback when they are recorded
   HIPCHK(hipEventCreateWithFlags(&ev_main_, hipEventDisableTiming | hipEventReleaseToDevice));
@@ -97,6 +97,29 @@ CholEngine::CholEngine(const Pattern& a, const CholOptions& opt, hipStream_t st)
   cd_.dinv_off = dinv_off_.p;
   build_tasks();
   build_solve();
+}
+
+// The look-ahead needs its stream on another hardware queue than the solver's.
+// The runtime spreads streams over a few queues (4 by default) and, once all
+// are in use, may give both of a solver's streams the same one, which runs
+// their kernels one after the other: a 5,000-bus factorization took 4.37 ms
+// there, 3.36 on two queues.  So candidates are tried until one's kernel runs
+// while the solver's stream is busy; the rejected ones are kept until then
+// (their queue stays counted as used), at most as many as there are queues by
+// default.  Streams of default priority, like the solver's.
+void CholEngine::pick_second_stream()
+{
+  constexpr int TRIES = 4;
+  DevBuf<int> words;
+  words.alloc(2);
+  std::vector<hipStream_t> rejected;
+  for (int t = 0; t < TRIES; t++) {
+    HIPCHK(hipStreamCreate(&st2_));
+    if (t + 1 == TRIES || dev::streams_overlap(st_, st2_, words.p)) break;
+    rejected.push_back(st2_);
+    st2_ = nullptr;
+  }
+  for (hipStream_t s : rejected) (void)hipStreamDestroy(s);
 }
 
 CholEngine::Sizes CholEngine::sizes() const

@@ -186,6 +186,7 @@ class CholEngine {
   };
   void build_tasks();
   void build_solve();
+  void pick_second_stream();
 
   CholPlan pl_;
   hipStream_t st_;

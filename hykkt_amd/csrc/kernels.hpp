@@ -270,6 +270,12 @@ void dense_nt(const CholDev& c, int ntasks, const int* task_sn, const int* task_
 void trsm_inv(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr, int step,
               const Batch& b, hipStream_t st, bool short_rows);
 
+// Whether kernels of the two streams run at the same time: a kernel on `a` waits
+// (a bounded number of polls) for a word that one on `b` sets.  Streams that
+// share a hardware queue never do.  Synchronizes both; words: 2 ints of device
+// memory.
+bool streams_overlap(hipStream_t a, hipStream_t b, int* words);
+
 // Single-launch supernodal solves over the whole tree.  Work items are
 // 128-row blocks of the fronts, dispatched in a dependency-respecting order;
 // items synchronise on the values they exchange, whose buffers are filled

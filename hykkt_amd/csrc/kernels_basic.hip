@@ -790,10 +790,48 @@ __global__ void k_pivot_split(const int* __restrict__ pivot, int* __restrict__ o
   }
 }
 
+// words[0]: set by k_set_word; words[1]: what k_wait_word saw of it in at most
+// `polls` polls (about a microsecond each).
+__global__ void k_wait_word(int* words, int polls)
+{
+  int v = 0;
+  for (int i = 0; i < polls && v == 0; i++) {
+    v = __hip_atomic_load(words, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_s_sleep(16);
+  }
+  __hip_atomic_store(words + 1, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void k_set_word(int* word, int v)
+{
+  __hip_atomic_store(word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 }  // namespace
 
 // =================================================================== launchers
 #define LAUNCH_CHECK() HIPCHK(hipGetLastError())
+
+bool streams_overlap(hipStream_t a, hipStream_t b, int* words)
+{
+  constexpr int POLLS = 400;
+  // both kernels once before, so their code is loaded and the words are clear
+  k_set_word<<<1, 1, 0, b>>>(words, 0);
+  LAUNCH_CHECK();
+  HIPCHK(hipStreamSynchronize(b));
+  k_wait_word<<<1, 1, 0, a>>>(words, 1);
+  LAUNCH_CHECK();
+  HIPCHK(hipStreamSynchronize(a));
+  k_wait_word<<<1, 1, 0, a>>>(words, POLLS);
+  LAUNCH_CHECK();
+  k_set_word<<<1, 1, 0, b>>>(words, 1);
+  LAUNCH_CHECK();
+  HIPCHK(hipStreamSynchronize(a));
+  HIPCHK(hipStreamSynchronize(b));
+  int saw = 0;
+  HIPCHK(hipMemcpy(&saw, words + 1, sizeof(int), hipMemcpyDeviceToHost));
+  return saw != 0;
+}
 
 void fill(double* p, double v, int64_t n, const Batch& b, hipStream_t st)
 {
