@@ -25,7 +25,6 @@ namespace {
 constexpr int NB = 128;   // panel step, MFMA tile edge, solve block
 constexpr int SR = 32;    // rows of a short tile
 constexpr int GMAX = 8;   // most steps one grouped trailing update can cover
-constexpr int BWD_OWN_CHUNKS = 2;   // see build_solve
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 }  // namespace
 
@@ -446,49 +445,71 @@ void CholEngine::build_tasks()
 void CholEngine::build_solve()
 {
   const int ns = pl_.ns;
-  // top of the tree: supernodes wider than one block or with fronts taller
-  // than TOP_F rows, and all their ancestors; the rest is a forest closed
-  // under descendants
-  constexpr int TOP_F = 512;
+  // top of the tree: supernodes wider than FOREST_NC columns or with fronts
+  // taller than FOREST_F rows, and all their ancestors; the rest is a forest
+  // closed under descendants
   std::vector<char> top(ns, 0);
   for (int s = 0; s < ns; s++)
-    if (pl_.nc(s) > NB || pl_.nc(s) + pl_.nr(s) > TOP_F) top[s] = 1;
+    if (pl_.nc(s) > dev::FOREST_NC || pl_.nc(s) + pl_.nr(s) > dev::FOREST_F) top[s] = 1;
   for (int s = 0; s < ns; s++)
     if (top[s])
       for (int p = pl_.sn_parent[s]; p >= 0 && !top[p]; p = pl_.sn_parent[p]) top[p] = 1;
-  std::vector<int> fwd, bwd, fwd_top, bwd_top;
+  std::vector<int> fwd_top, bwd_top;
   solve_lower_[0] = solve_lower_[1] = 0.0;
   solve_n_[0] = solve_n_[1] = 0;
   for (int s = 0; s < ns; s++) {   // postorder: children first
-    std::vector<int>& f = top[s] ? fwd_top : fwd;
-    for (int b = 0; b < cdiv(pl_.nc(s), NB); b++) f.insert(f.end(), {s, 0, b});
-    for (int u = 0; u < cdiv(pl_.nr(s), NB); u++) f.insert(f.end(), {s, 1, u});
     const double nc = pl_.nc(s), nr = pl_.nr(s);
     solve_lower_[top[s]] += nc * (nc + 1) / 2 + nr * nc;
     solve_n_[top[s]] += pl_.nc(s);
+    if (!top[s]) continue;
+    for (int b = 0; b < cdiv(pl_.nc(s), NB); b++) fwd_top.insert(fwd_top.end(), {s, 0, b});
+    for (int u = 0; u < cdiv(pl_.nr(s), NB); u++) fwd_top.insert(fwd_top.end(), {s, 1, u});
   }
+  // forest items, by tree level (leaves first): a tall supernode, or up to four
+  // short ones of the level
+  std::vector<dev::ForestSn> fsn;
+  std::vector<int> fwd, bwd;
+  std::vector<int64_t> foff(ns + 1, 0), uvo(ns + 1, 0), dvo(ns + 1, 0);
+  for (int s = 0; s < ns; s++) {
+    foff[s + 1] = foff[s] + pl_.nc(s) + pl_.nr(s);
+    uvo[s + 1] = uvo[s] + pl_.nr(s);
+    dvo[s + 1] = dvo[s] + static_cast<int64_t>(cdiv(pl_.nc(s), NB)) * NB * NB;
+  }
+  for (size_t l = 0; l + 1 < pl_.level_ptr.size(); l++) {
+    int open = 0;   // waves left in the level's last item
+    for (int q = pl_.level_ptr[l]; q < pl_.level_ptr[l + 1]; q++) {
+      const int s = pl_.level_sn[q];
+      if (top[s]) continue;
+      const int i = static_cast<int>(fsn.size());
+      fsn.push_back(dev::ForestSn{pl_.sn_first[s], pl_.nc(s), pl_.nr(s), 0, pl_.l_off[s], dvo[s],
+                                  uvo[s], foff[s], pl_.rows_ptr[s], 0});
+      if (pl_.nc(s) + pl_.nr(s) > dev::FOREST_WAVE_F) {
+        // before the level's open item, which stays the last
+        fwd.insert(open > 0 ? fwd.end() - 4 : fwd.end(), {i, -2, -2, -2});
+      } else {
+        if (open == 0) {
+          fwd.insert(fwd.end(), {-1, -1, -1, -1});
+          open = 4;
+        }
+        fwd[fwd.size() - open] = i;
+        open--;
+      }
+    }
+  }
+  for (size_t k = fwd.size(); k >= 4; k -= 4)   // parents first
+    bwd.insert(bwd.end(), fwd.begin() + (k - 4), fwd.begin() + k);
   std::vector<int64_t> bpo(ns + 1, 0);
   for (int s = ns - 1; s >= 0; s--) {   // parents first: row chunks, then pivot blocks
-    std::vector<int>& b = top[s] ? bwd_top : bwd;
+    if (!top[s]) continue;
     const int np = cdiv(pl_.nc(s), NB), nu = cdiv(pl_.nr(s), NB);
-    if (!top[s] && nu <= BWD_OWN_CHUNKS) {
-      // a forest supernode (one block) with few row chunks: its pivot item
-      // forms the chunks' products itself, one dependency link instead of two
-      b.insert(b.end(), {s, 2, 0});
-      continue;
-    }
     for (int u = 0; u < nu; u++)
-      for (int k = 0; k < np; k++) b.insert(b.end(), {s, 0, u * np + k});
-    for (int k = np - 1; k >= 0; k--) b.insert(b.end(), {s, 1, k});
+      for (int k = 0; k < np; k++) bwd_top.insert(bwd_top.end(), {s, 0, u * np + k});
+    for (int k = np - 1; k >= 0; k--) bwd_top.insert(bwd_top.end(), {s, 1, k});
   }
-  for (int s = 0; s < ns; s++)
-    bpo[s + 1] = bpo[s] + static_cast<int64_t>(cdiv(pl_.nr(s), NB)) * pl_.nc(s);
+  for (int s = 0; s < ns; s++)   // the forest has no chunk partials
+    bpo[s + 1] = bpo[s] + (top[s] ? static_cast<int64_t>(cdiv(pl_.nr(s), NB)) * pl_.nc(s) : 0);
   // pull lists: front row of a parent <- entries of its children's update vectors
-  std::vector<int64_t> foff(ns + 1, 0);
-  for (int s = 0; s < ns; s++) foff[s + 1] = foff[s] + pl_.nc(s) + pl_.nr(s);
   std::vector<int> cnt(static_cast<size_t>(foff[ns]) + 1, 0);
-  std::vector<int64_t> uvo(ns + 1, 0);
-  for (int s = 0; s < ns; s++) uvo[s + 1] = uvo[s] + pl_.nr(s);
   for (int c = 0; c < ns; c++) {
     int p = pl_.sn_parent[c];
     if (p < 0) continue;
@@ -507,8 +528,11 @@ void CholEngine::build_solve()
     if (v.empty()) v.push_back(0);
     b.upload(v);
   };
-  sd_.n_fwd = static_cast<int>(fwd.size() / 3);
-  sd_.n_bwd = static_cast<int>(bwd.size() / 3);
+  sd_.n_fwd = static_cast<int>(fwd.size() / 4);
+  sd_.n_bwd = static_cast<int>(bwd.size() / 4);
+  if (fsn.empty()) fsn.push_back(dev::ForestSn{});
+  forest_.upload(fsn);
+  sd_.forest = forest_.p;
   sd_.n_fwd_top = static_cast<int>(fwd_top.size() / 3);
   sd_.n_bwd_top = static_cast<int>(bwd_top.size() / 3);
   upi(fwd_items_, fwd);
@@ -531,8 +555,7 @@ void CholEngine::build_solve()
   sd_.bpart_off = bpart_off_.p;
   sd_.err = flags_.p;
   sd_.ticket = flags_.p + 1;
-  grid_fwd_full_ = n_cu_ * dev::forest_blocks_per_cu();
-  sd_.grid_fwd = grid_fwd_full_;
+  forest_full_ = n_cu_ * dev::forest_blocks_per_cu();
   share_ = 1;
   n_bpart_ = bpo[ns];
   dev::fill_i(flags_.p, 0, 1, st_);
@@ -683,14 +706,12 @@ void CholEngine::set_sweep_share(int share)
   if (share == share_) return;
   share_ = share;
   if (share == 1) {
-    sd_.grid_fwd = grid_fwd_full_;
     sd_.cap_forest = sd_.cap_top = 0;
     return;
   }
   // the forest sweeps: their share of the 256-thread workgroups the device
   // holds; the top of the tree: of two 1024-thread workgroups per CU
-  sd_.grid_fwd = std::max(1, grid_fwd_full_ / share);
-  sd_.cap_forest = sd_.grid_fwd;
+  sd_.cap_forest = std::max(1, forest_full_ / share);
   sd_.cap_top = std::max(1, 2 * n_cu_ / share);
 }
 
@@ -716,8 +737,10 @@ void CholEngine::solve(double* x, const dev::Batch& bt)
     if ((part == 0 ? (fwd ? sd_.n_fwd : sd_.n_bwd) : (fwd ? sd_.n_fwd_top : sd_.n_bwd_top)) <= 0)
       return;
     if (pf) pf->begin(st_);
-    if (fwd) dev::solve_forward(cd_, sd_, x, ybuf_, part, b, st_);
-    else dev::solve_backward(cd_, sd_, ybuf_, x, part, b, st_);
+    if (fwd)
+      (part ? dev::solve_forward_top : dev::solve_forward_forest)(cd_, sd_, x, ybuf_, b, st_);
+    else
+      (part ? dev::solve_backward_top : dev::solve_backward_forest)(cd_, sd_, ybuf_, x, b, st_);
     if (pf)
       pf->end(kind, st_, 2.0 * solve_lower_[part] * b.count,
               8.0 * (solve_lower_[part] + 2.0 * solve_n_[part]) * b.count);

@@ -195,7 +195,7 @@ class CholEngine {
   Tuning tun_;
   bool pinned_ = false;
   int tcount_ = 1;   // systems per launch the task lists are shaped for
-  int grid_fwd_full_ = 1;   // the forward forest sweep's workgroups at full share
+  int forest_full_ = 1;   // workgroups of a forest sweep the device holds at once
   int share_ = 1;
   DevBuf<double> own_;   // owned storage (own)
   DevBuf<int> own_piv_;
@@ -220,6 +220,7 @@ class CholEngine {
   // solve items
   DevBuf<int> fwd_items_, bwd_items_, pull_ptr_, pull_src_, flags_;
   DevBuf<int64_t> bpart_off_;
+  DevBuf<dev::ForestSn> forest_;
   DevBuf<int> fwd_top_items_, bwd_top_items_;
   double* ybuf_ = nullptr;   // forward-sweep output (bound storage)
   int64_t n_bpart_ = 0;

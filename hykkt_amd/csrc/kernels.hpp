@@ -281,14 +281,30 @@ bool streams_overlap(hipStream_t a, hipStream_t b, int* words);
 // items synchronise on the values they exchange, whose buffers are filled
 // with a sentinel (fill_sentinel) before each sweep.  With several systems,
 // launch item i*count + k is item i of system k.
+constexpr int FOREST_NC = 32;   // most columns of a forest supernode
+constexpr int FOREST_F = 512;   // most front rows of one
+constexpr int FOREST_WAVE_F = 64;   // most front rows of one that takes one wave
+
+// What a sweep item needs to know of a forest supernode.
+struct ForestSn {
+  int a, nc, nr, pad;        // first column, columns, rows below them
+  int64_t l_off, dinv_off;   // panel, inverted diagonal block
+  int64_t uvec_off;          // its update vector in ubuf
+  int64_t front_off;         // its front rows in the pull_ptr index
+  int64_t rows_off;          // its rows in CholDev::rows
+  int64_t pad2;
+};
+
 struct SolveDev {
-  // Items of the small-supernode forest (fwd_items, bwd_items) and of the top
-  // of the tree (*_top) are separate launches: forward forest then top,
-  // backward top then forest.
-  const int* fwd_items;     // 3 ints per item: supernode, kind (0 pivot, 1 update), block
+  // Items of the small-supernode forest (fwd_items, bwd_items: 4 ints each, indices
+  // into `forest`; see kernels_forest.hip) and of the top of the tree (*_top: 3 ints
+  // per item) are separate launches: forward forest then top, backward top then
+  // forest.  Top items: supernode, kind, index (forward: 0 pivot, 1 update, block;
+  // backward: 0 row chunk, chunk * blocks + column block; 1 pivot, block).
+  const ForestSn* forest;
+  const int* fwd_items;
   int n_fwd;
-  const int* bwd_items;     // 3 ints per item: supernode, kind (0 row chunk, 1 pivot), index
-                            // (row chunk: chunk * blocks + column block; pivot: block)
+  const int* bwd_items;
   int n_bwd;
   const int* fwd_items_top;
   int n_fwd_top;
@@ -304,24 +320,27 @@ struct SolveDev {
   int* err;                 // 1: a wait hit its bound (sticky until the host clears it)
   int* ticket;              // 4 item counters (forward forest, forward top, backward top,
                             // backward forest), zeroed with the first sentinel fill of a solve
-  int grid_fwd;             // workgroups of the persistent forward forest sweep (resident at once)
   int cap_top = 0;          // most workgroups of a top-of-tree sweep launch (0: one per item)
-  int cap_forest = 0;       // most workgroups of a backward forest sweep launch (0: one per item)
+  int cap_forest = 0;       // most workgroups of a forest sweep launch (0: one per item)
 };
-// Workgroups of the forward forest sweep one compute unit holds at once.
+// Workgroups of a forest sweep one compute unit holds at once.
 int forest_blocks_per_cu();
 // p[i] = the sentinel, i < n (per system); zero4 (when not null): four ints set to 0
 void fill_sentinel(double* p, int64_t n, const Batch& b, hipStream_t st, int* zero4 = nullptr);
 // The same for three buffers (p_i[0..n_i)) in one launch.
 void fill_sentinel3(double* p0, int64_t n0, double* p1, int64_t n1, double* p2, int64_t n2,
                     const Batch& b, hipStream_t st, int* zero4 = nullptr);
-// L y = b (b, y internal order; y sentinel-filled, ubuf sentinel-filled).
-// part 0: the forest items, part 1: the top items.
-void solve_forward(const CholDev& c, const SolveDev& sd, const double* rhs, double* y, int part,
-                   const Batch& b, hipStream_t st);
-// L^T x = y (x and bpart sentinel-filled).
-void solve_backward(const CholDev& c, const SolveDev& sd, const double* y, double* x, int part,
-                    const Batch& b, hipStream_t st);
+// L y = b (b, y internal order; y sentinel-filled, ubuf sentinel-filled): the
+// forest, then the top of the tree.
+void solve_forward_forest(const CholDev& c, const SolveDev& sd, const double* rhs, double* y,
+                          const Batch& b, hipStream_t st);
+void solve_forward_top(const CholDev& c, const SolveDev& sd, const double* rhs, double* y,
+                       const Batch& b, hipStream_t st);
+// L^T x = y (x and bpart sentinel-filled): the top of the tree, then the forest.
+void solve_backward_top(const CholDev& c, const SolveDev& sd, const double* y, double* x,
+                        const Batch& b, hipStream_t st);
+void solve_backward_forest(const CholDev& c, const SolveDev& sd, const double* y, double* x,
+                           const Batch& b, hipStream_t st);
 
 }  // namespace dev
 }  // namespace hykkt
