@@ -587,12 +587,12 @@ void CholEngine::shift_diag(double delta, const dev::Batch& b)
   if (delta != 0.0) dev::add_at(cd_.L, diag_pos_.p, pl_.n, delta, b, st_);
 }
 
-void CholEngine::factor(double pivot_tol, const dev::Batch& bt)
+void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clear)
 {
   HYKKT_REQUIRE(cd_.L && bt.count <= cap_, HYKKT_E_STATE, "factor storage not bound");
   const dev::Batch b{bt.count, vs_, nullptr};
   cd_.pivot_tol = pivot_tol;
-  dev::fill_i(cd_.pivot, INT_MAX, b.count, st_);
+  if (!pivots_clear) dev::fill_i(cd_.pivot, INT_MAX, b.count, st_);
   Profiler* pf = prof_ && prof_->on() ? prof_ : nullptr;
   // Bracket one launch (skipped when it has no tasks, like the launchers);
   // charged with the work of all the systems it covers.

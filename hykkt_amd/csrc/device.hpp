@@ -149,8 +149,8 @@ class CholEngine {
   // Add `delta` to every diagonal entry of the assembled matrix.
   void shift_diag(double delta, const dev::Batch& b);
   // Factor the assembled matrices of b.count systems; pivot failures are
-  // recorded on the device.
-  void factor(double pivot_tol, const dev::Batch& b);
+  // recorded on the device (pivots_clear: its words are INT_MAX already).
+  void factor(double pivot_tol, const dev::Batch& b, bool pivots_clear = false);
   // First failing pivot (internal index) or -1 of each of `count` systems;
   // synchronizes the stream.
   std::vector<int> pivots(int count);

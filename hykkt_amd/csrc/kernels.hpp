@@ -70,10 +70,11 @@ void copy_in(int nsrc, double* const* dst, const double* const* src_tab, const i
 
 // ---------------------------------------------------------------- sparse
 // jd_vs = Ds-row-scaled Jd (skipped if jd_vs is null); ryd_s = ryd*ds + rs
-// (row_scale :490-509, add_vecs :310-317)
+// (row_scale :490-509, add_vecs :310-317).  word0, word1 (may be null): one int per
+// system each, set to INT_MAX.
 void row_scale(int d, const int* jd_rp, const double* jd_v, const double* ds,
                const double* ryd, const double* rs, double* jd_vs, double* ryd_s,
-               const Batch& b, hipStream_t st);
+               const Batch& b, hipStream_t st, int* word0 = nullptr, int* word1 = nullptr);
 // Row blocks of a CSR matrix for the LDS-staged SpMV: consecutive rows with
 // at most spmv_lds_entries() entries together (a longer row is a block of its
 // own); blocks[k] = first row of block k, blocks[nblk] = nrows.
@@ -113,6 +114,28 @@ void add_at(double* out, const int64_t* pos, int n, double delta, const Batch& b
 void ruiz_rowmax(int n, int totn, const int* h_rp, const double* h_v, const int* jt_rp,
                  const int* jt_map, const double* jt_v, const int* j_rp, const double* j_v,
                  double* scale, int* zero_row, const Batch& b, hipStream_t st);
+// One pass of the solver's Ruiz scaling over [H~ Jc^T; Jc], Jc^T's values read from
+// Jc's through jt_map: with scale_in, the last scale applied (h_v in place, j_src
+// -> j_dst, rhs1 in place, rhs2_src -> rhs2, max_d, which `first` starts); with
+// scale_out, the next scale formed from the scaled rows (and zero_row as above).
+// j_dst must not be j_src where both are given.
+struct RuizPass {
+  int n, m;
+  const int *h_rp, *h_ci;
+  double* h_v;
+  const int *jt_rp, *jt_ci, *jt_map, *j_rp, *j_ci;
+  const double* j_src;
+  double* j_dst;
+  const double* scale_in;
+  double* scale_out;
+  double* rhs1;
+  const double* rhs2_src;
+  double* rhs2;
+  double* max_d;
+  int first;
+  int* zero_row;
+};
+void ruiz_pass(const RuizPass& c, const Batch& b, hipStream_t st);
 // adapt_diag_scale (matrix_vector_ops.cu:146-186); jt_v_scaled may be null (Jt shares J).
 // first != 0: max_d is written as 1*scale (reset, :268-283, fused).
 void ruiz_scale(int n, int totn, const int* h_rp, const int* h_ci, double* h_v,

@@ -23,7 +23,7 @@ namespace hykkt {
 // Per-system arena slots (offsets in doubles from the system's base).
 struct Solver::Slots {
   int64_t in[IN_COUNT] = {}, gam = 0;
-  int64_t jd_vs = 0, ryd_s = 0, rx_til = 0, htil = 0, jcs = 0, ry_s = 0, max_d = 0, scale = 0;
+  int64_t jd_vs = 0, ryd_s = 0, rx_til = 0, htil = 0, jcs = 0, ry_s = 0, max_d = 0, scale = 0, scale2 = 0;
   int64_t jch_v = 0, jcth_v = 0, rxp = 0, tmp_n = 0, t1 = 0;
   int64_t cx = 0, cr = 0, cw = 0, cp = 0, cs = 0, schur = 0, sc = 0, part = 0;
   int64_t h0 = 0, cq = 0, cz = 0;
@@ -416,6 +416,7 @@ void Solver::analyze()
   z.ry_s = slot(m);
   z.max_d = slot(n + m);
   z.scale = slot(n + m);
+  z.scale2 = slot(n + m);
   z.jch_v = slot(S->nnz_jc);
   z.jcth_v = slot(S->nnz_jc);
   z.rxp = slot(n);
@@ -709,7 +710,7 @@ std::vector<int> Solver::run(int count, bool from_setters)
   // ---- compute_spgemm_htil (HykktSolver.cpp:289-337) ----
   if (S.has_jd) {
     dev::row_scale(d, S.jd_rp.p, in[IN_JD], in[IN_DS], in[IN_RYD], in[IN_RS], P(z.jd_vs),
-                   P(z.ryd_s), b, st_);
+                   P(z.ryd_s), b, st_, S.flag(FL_ZERO_ROW), S.flag(FL_PIVOT));
     timed(PK_SPMV, 2.0 * S.nnz_jd, spmv_bytes(n, d, S.nnz_jd, true, true, false), b, [&] {
       dev::spmv(n, S.jdt_rp.p, S.jdt_ci.p, S.jdt_map.p, in[IN_JD], 1.0, nullptr, P(z.ryd_s), 1.0,
                 in[IN_RX], P(z.rx_til), S.jdt_blk.p, S.jdt_nblk, b, st_);
@@ -721,19 +722,50 @@ std::vector<int> Solver::run(int count, bool from_setters)
   } else {
     dev::copy(P(z.rx_til), in[IN_RX], n, b, st_);
     dev::copy(P(z.htil), in[IN_H], S.nnz_h, b, st_);
+    dev::fill_i(S.flag(FL_ZERO_ROW), INT_MAX, count, st_);
+    dev::fill_i(S.flag(FL_PIVOT), INT_MAX, count, st_);
   }
-  dev::copy(P(z.jcs), in[IN_JC], S.nnz_jc, b, st_);
-  dev::copy(P(z.ry_s), in[IN_RY], m, b, st_);
 
-  // ---- compute_ruiz_scaling (HykktSolver.cpp:340-349; RuizClass.cpp:54-98) ----
-  if (opts.ruiz_its <= 0) dev::fill(P(z.max_d), 1.0, n + m, b, st_);
-  dev::fill_i(S.flag(FL_ZERO_ROW), INT_MAX, count, st_);
-  for (int it = 0; it < opts.ruiz_its; it++) {
-    dev::ruiz_rowmax(n, n + m, S.ht_rp.p, P(z.htil), S.jct_rp.p, S.jct_map.p, P(z.jcs), S.jc_rp.p,
-                     P(z.jcs), P(z.scale), S.flag(FL_ZERO_ROW), b, st_);
-    dev::ruiz_scale(n, n + m, S.ht_rp.p, S.ht_ci.p, P(z.htil), S.jct_rp.p, S.jct_ci.p, nullptr,
-                    S.jc_rp.p, S.jc_ci.p, P(z.jcs), P(z.scale), P(z.rx_til), P(z.ry_s),
-                    P(z.max_d), it == 0, b, st_);
+  // ---- compute_ruiz_scaling (HykktSolver.cpp:340-349; RuizClass.cpp:54-98):
+  // each pass applies the last sweep's scale and forms the next one's ----
+  if (opts.ruiz_its <= 0) {
+    dev::copy(P(z.jcs), in[IN_JC], S.nnz_jc, b, st_);
+    dev::copy(P(z.ry_s), in[IN_RY], m, b, st_);
+    dev::fill(P(z.max_d), 1.0, n + m, b, st_);
+  } else {
+    dev::RuizPass r{};
+    r.n = n;
+    r.m = m;
+    r.h_rp = S.ht_rp.p;
+    r.h_ci = S.ht_ci.p;
+    r.h_v = P(z.htil);
+    r.jt_rp = S.jct_rp.p;
+    r.jt_ci = S.jct_ci.p;
+    r.jt_map = S.jct_map.p;
+    r.j_rp = S.jc_rp.p;
+    r.j_ci = S.jc_ci.p;
+    r.j_src = in[IN_JC];
+    r.rhs1 = P(z.rx_til);
+    r.rhs2_src = in[IN_RY];
+    r.rhs2 = P(z.ry_s);
+    r.max_d = P(z.max_d);
+    r.zero_row = S.flag(FL_ZERO_ROW);
+    double* const scale[2] = {P(z.scale), P(z.scale2)};
+    // the passes in between alternate Jc's scaled values between jch_v (free
+    // until the factorization is done) and jcs, where the last one leaves them
+    double* const jbuf[2] = {P(z.jcs), P(z.jch_v)};
+    for (int k = 0; k <= opts.ruiz_its; k++) {
+      const bool last = k == opts.ruiz_its;
+      r.scale_in = k > 0 ? scale[(k - 1) & 1] : nullptr;
+      r.scale_out = last ? nullptr : scale[k & 1];
+      r.j_dst = k == 0 ? nullptr : jbuf[last ? 0 : (k & 1)];
+      r.first = k == 1;
+      dev::ruiz_pass(r, b, st_);
+      if (k > 0) {
+        r.j_src = r.j_dst;
+        r.rhs2_src = r.rhs2;
+      }
+    }
   }
 
   // ---- launch shapes of the factorization, once per pattern ----
@@ -745,7 +777,7 @@ std::vector<int> Solver::run(int count, bool from_setters)
   assemble_hgamma(b);
 
   // ---- compute_hgamma_factorization (HykktSolver.cpp:398-401) ----
-  ch.factor(opts.pivot_tol, b);
+  ch.factor(opts.pivot_tol, b, !(fresh && opts.autotune));   // the tuning runs record pivots, too
   HIPCHK(hipEventRecord(ev_[1], st_));
 
   // permuted Jc and Jc^T values (apply_permutation, HykktSolver.cpp:386-395)
