@@ -22,9 +22,10 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = "gfx950"
 
 HIP_SOURCES = {
-    # formation / Ruiz / SpMV / CG kernels: explicit fma only, so results are
+    # formation / Ruiz / SpMV / CG / residual kernels: explicit fma only, so results are
     # bit-identical to the CPU oracle's operation order
     "kernels_basic.hip": ["-ffp-contract=off"],
+    "kernels_pass.hip": ["-ffp-contract=off"],
     "kernels_chol.hip": [],
     "kernels_dense.hip": [],
     "kernels_trsv.hip": [],

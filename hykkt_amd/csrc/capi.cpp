@@ -20,7 +20,7 @@ struct hykkt_solver_s {
 struct hykkt_chol_s {
   hipStream_t st = nullptr;
   std::unique_ptr<hykkt::CholEngine> eng;
-  hykkt::DevBuf<double> vals, x;
+  hykkt::DevBuf<double> vals, x, x2;
   std::vector<int> post;
   int n = 0, nnz = 0;
   ~hykkt_chol_s()
@@ -707,6 +707,7 @@ int hykkt_chol_create(int n, int nnz, const int* rp, const int* ci, hykkt_chol* 
     c->eng->own(1);
     c->vals.alloc(std::max(1, nnz));
     c->x.alloc(std::max(1, n));
+    c->x2.alloc(std::max(1, n));
     c->post = c->eng->plan().post;
     c->n = n;
     c->nnz = nnz;
@@ -741,8 +742,8 @@ int hykkt_chol_solve(hykkt_chol c, const double* b, double* x)
     std::vector<double> t(n);
     for (int k = 0; k < n; k++) t[k] = b[c->post[k]];
     HIPCHK(hipMemcpyAsync(c->x.p, t.data(), n * sizeof(double), hipMemcpyHostToDevice, c->st));
-    c->eng->solve(c->x.p);
-    HIPCHK(hipMemcpyAsync(t.data(), c->x.p, n * sizeof(double), hipMemcpyDeviceToHost, c->st));
+    c->eng->solve(c->x.p, c->x2.p, hykkt::dev::Batch{1, c->eng->stride(), nullptr});
+    HIPCHK(hipMemcpyAsync(t.data(), c->x2.p, n * sizeof(double), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     HYKKT_REQUIRE(!c->eng->solve_error(), HYKKT_E_STATE,
                   "triangular-solve sweep exceeded its wait bound (results invalid)");
@@ -805,9 +806,9 @@ int hykkt_schur_cg(hykkt_chol c, int m, int n, const int* j_rp, const int* j_ci,
       }
       return bl;
     };
-    const std::vector<int> jb = blocks(Jh.rp, m), jtb = blocks(jt.at.rp, n);
-    DevBuf<int> jrp, jci, jtrp, jtci, jblk, jtblk, flg;
-    DevBuf<double> jv, jtv, t1, xv, r, w, p, s, bb, sc, part, gath;
+    const std::vector<int> jb = blocks(Jh.rp, m);
+    DevBuf<int> jrp, jci, jtrp, jtci, jblk, flg;
+    DevBuf<double> jv, jtv, t1, t2, xv, r, w, p, s, bb, sc, part, part2, out;
     auto upi = [](DevBuf<int>& d, const std::vector<int>& v) {
       if (v.empty()) d.upload(std::vector<int>{0});
       else d.upload(v);
@@ -823,18 +824,16 @@ int hykkt_schur_cg(hykkt_chol c, int m, int n, const int* j_rp, const int* j_ci,
     upi(jtci, jt.at.ci);
     upd(jtv, jthv);
     upi(jblk, jb);
-    upi(jtblk, jtb);
     upd(xv, std::vector<double>(x, x + m));
     upd(bb, std::vector<double>(b, b + m));
-    t1.alloc(std::max(1, n));
+    for (DevBuf<double>* q : {&t1, &t2}) q->alloc(std::max(1, n));
     for (DevBuf<double>* q : {&r, &w, &p, &s}) q->alloc(std::max(1, m));
-    sc.alloc(8);
-    part.alloc(hykkt::schur_partials(m, static_cast<int>(jb.size()) - 1));
-    gath.alloc(4);
+    sc.alloc(hykkt::dev::CG_SLOTS);
+    part.alloc(hykkt::dev::reduce_blocks(m));
+    part2.alloc(std::max<size_t>(jb.size(), 1));
+    out.alloc(hykkt::dev::FIN_SLOTS);
     flg.alloc(3);
     hykkt::SchurOps o;
-    o.m = m;
-    o.n = n;
     o.jh_rp = jrp.p;
     o.jh_ci = jci.p;
     o.jh_blk = jblk.p;
@@ -842,34 +841,33 @@ int hykkt_schur_cg(hykkt_chol c, int m, int n, const int* j_rp, const int* j_ci,
     o.jh_v = jv.p;
     o.jth_rp = jtrp.p;
     o.jth_ci = jtci.p;
-    o.jth_blk = jtblk.p;
-    o.jth_nblk = static_cast<int>(jtb.size()) - 1;
     o.jth_v = jtv.p;
     o.chol = c->eng.get();
     o.st = c->st;
-    o.t1 = t1.p;
-    o.x = xv.p;
-    o.r = r.p;
-    o.w = w.p;
-    o.p = p.p;
-    o.s = s.p;
-    o.sc = sc.p;
-    o.part = part.p;
-    o.live = flg.p;
-    o.iters = flg.p + 1;
-    o.status = flg.p + 2;
-    o.gath = gath.p;
+    o.v = hykkt::dev::CgVecs{m,       n,       xv.p,    r.p,  w.p,    p.p,    s.p,    t1.p,
+                             t2.p,    nullptr, nullptr, sc.p, part.p, part2.p, o.jh_nblk};
+    o.f = hykkt::dev::CgFlags{flg.p, flg.p + 1, flg.p + 2};
     // one system: its vectors are separate buffers, the factor the engine's
     const hykkt::dev::Batch one{1, c->eng->stride(), nullptr};
-    const std::vector<hykkt::CgResult> res =
-        hykkt::schur_cg_run(o, bb.p, tol, itmax, one, false, 1, 1);
+    hykkt::cg_start(o, bb.p, one, false);
+    std::vector<double> fin(hykkt::dev::FIN_SLOTS);
+    hykkt::dev::Finish fo{};
+    fo.out = out.p;
+    do {
+      hykkt::cg_iterate(o, 1, tol, itmax, one);
+      hykkt::dev::finish(fo, nullptr, o.v, o.k, tol, itmax, o.f, one, c->st);
+      HIPCHK(hipMemcpyAsync(fin.data(), out.p, fin.size() * sizeof(double), hipMemcpyDeviceToHost,
+                            c->st));
+      HIPCHK(hipStreamSynchronize(c->st));
+    } while (fin[hykkt::dev::FIN_LIVE] != 0.0 && o.k < itmax);
+    const hykkt::CgResult res = hykkt::cg_result(fin.data());
     HIPCHK(hipMemcpyAsync(x, xv.p, m * sizeof(double), hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     HYKKT_REQUIRE(!c->eng->solve_error(), HYKKT_E_STATE,
                   "triangular-solve sweep exceeded its wait bound (results invalid)");
-    if (iters) *iters = res[0].iters;
-    if (final_norm) *final_norm = res[0].final_norm;
-    return res[0].status;
+    if (iters) *iters = res.iters;
+    if (final_norm) *final_norm = res.final_norm;
+    return res.status;
   });
 }
 

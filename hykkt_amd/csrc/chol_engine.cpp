@@ -724,11 +724,25 @@ int CholEngine::solve_error()
   return h;
 }
 
-void CholEngine::solve(double* x, const dev::Batch& bt)
+dev::SweepFill CholEngine::sweep_fill(double* x) const
+{
+  dev::SweepFill f;
+  f.p[0] = ybuf_;
+  f.n[0] = pl_.n;
+  f.p[1] = x;
+  f.n[1] = pl_.n;
+  f.p[2] = sd_.ubuf;
+  f.n[2] = n_ubuf_;
+  f.p[3] = sd_.bpart;
+  f.n[3] = n_bpart_;
+  f.ticket = sd_.ticket;
+  return f;
+}
+
+void CholEngine::solve(const double* rhs, double* x, const dev::Batch& bt, bool filled)
 {
   const dev::Batch b{bt.count, vs_, bt.mask};
   Profiler* pf = prof_ && prof_->on() ? prof_ : nullptr;
-  const int64_t nu = n_ubuf_;
   // Algorithmic, per part of the tree: each sweep reads that part's factor
   // entries (lower trapezoids of its panels) once, 2 flops per entry, and
   // reads + writes its vector entries; charged for every system of the
@@ -738,20 +752,16 @@ void CholEngine::solve(double* x, const dev::Batch& bt)
       return;
     if (pf) pf->begin(st_);
     if (fwd)
-      (part ? dev::solve_forward_top : dev::solve_forward_forest)(cd_, sd_, x, ybuf_, b, st_);
+      (part ? dev::solve_forward_top : dev::solve_forward_forest)(cd_, sd_, rhs, ybuf_, b, st_);
     else
       (part ? dev::solve_backward_top : dev::solve_backward_forest)(cd_, sd_, ybuf_, x, b, st_);
     if (pf)
       pf->end(kind, st_, 2.0 * solve_lower_[part] * b.count,
               8.0 * (solve_lower_[part] + 2.0 * solve_n_[part]) * b.count);
   };
-  // forward: b in x -> y in ybuf; backward: y in ybuf -> x.  x holds b until
-  // the forward sweep is done, so it is filled after it; the other buffers
-  // (and the item counters) before it, in one launch.
-  dev::fill_sentinel3(ybuf_, pl_.n, sd_.ubuf, nu, sd_.bpart, n_bpart_, b, st_, sd_.ticket);
+  if (!filled) dev::fill_sentinel(sweep_fill(x), b, st_);
   sweep(PK_SOLVE_FWD_FOREST, 0, true);
   sweep(PK_SOLVE_FWD_TOP, 1, true);
-  dev::fill_sentinel(x, pl_.n, b, st_);
   sweep(PK_SOLVE_BWD_TOP, 1, false);
   sweep(PK_SOLVE_BWD_FOREST, 0, false);
 }

@@ -159,10 +159,11 @@ class CholEngine {
   // call (synchronizes the stream, clears the error word; solves in between
   // leave it set).
   int solve_error();
-  // Solve L L^T x = b in place for each system of b (its mask skips
-  // systems), x in internal (postordered) order, per system at x + k*b.vs.
-  void solve(double* x, const dev::Batch& b);
-  void solve(double* x) { solve(x, dev::Batch{1, vs_, nullptr}); }
+  // Solve L L^T x = rhs for each system of b (its mask skips systems), both in
+  // internal (postordered) order, per system at + k*b.vs; x is not rhs.  filled:
+  // sweep_fill(x)'s buffers were filled by a launch before.
+  void solve(const double* rhs, double* x, const dev::Batch& b, bool filled = false);
+  dev::SweepFill sweep_fill(double* x) const;
   // Device arrays of the assembly map (a's lower-triangle entries).
   const int* a_src() const { return a_src_.p; }
   const int64_t* a_dst() const { return a_dst_.p; }
@@ -229,57 +230,38 @@ class CholEngine {
 };
 
 // The Schur-complement operator S = Jh A^{-1} Jh^T with A factored by `chol`
-// (Jh: m x n, columns in the factor's internal order) and the CG workspace.
-// Per-system vectors are at their system-0 address + k * vs (the Batch);
-// the flag arrays hold one int per system.
+// (Jh: m x n, columns in the factor's internal order) and the CG on it
+// (SchurComplementConjugateGradient::solve, …ConjugateGradient.cpp:89-194).
+// Per-system vectors are at their system-0 address + k * vs (the Batch); the
+// flag arrays hold one int per system.  Every system's stopping test is taken
+// on the device, which then leaves that system alone.
 struct SchurOps {
-  int m = 0, n = 0;
   const int *jh_rp = nullptr, *jh_ci = nullptr, *jh_blk = nullptr;
   int jh_nblk = 0;
   const double* jh_v = nullptr;
-  const int *jth_rp = nullptr, *jth_ci = nullptr, *jth_blk = nullptr;
-  int jth_nblk = 0;
+  const int *jth_rp = nullptr, *jth_ci = nullptr;
   const double* jth_v = nullptr;
   CholEngine* chol = nullptr;
   hipStream_t st = nullptr;
-  double *t1 = nullptr;                                            // n
-  double *x = nullptr, *r = nullptr, *w = nullptr, *p = nullptr, *s = nullptr;   // m
-  double *sc = nullptr, *part = nullptr;   // 8 scalars; partials (max of both reductions)
-  // optional (n each): z = A^{-1} Jh^T x carried along with the iterate x
-  // (q the same image of the direction p), so the recovery needs no solve
-  double *tq = nullptr, *tz = nullptr;
-  int *live = nullptr, *iters = nullptr, *status = nullptr;   // per system
-  double* gath = nullptr;   // 4 doubles per system: the results packed for the readback
+  dev::CgVecs v{};   // v.q, v.z (optional): z = A^{-1} Jh^T x carried along with x
+  dev::CgFlags f{};
   Profiler* prof = nullptr;  // optional launch timing of the SpMVs
   int nnz = 0;               // entries of Jc
-  // optional pinned host memory of at least 4 doubles per system, for the
-  // live-flag checks and the results (pageable vectors otherwise)
-  double* pinned = nullptr;
-  // with pinned memory: leave the results' copy in flight and return them
-  // unfilled; cg_unpack(pinned, ...) fills them after the caller's next
-  // synchronization of the stream (one host round trip less per pass)
-  bool defer = false;
+  int k = 0;                 // updates since cg_start
 };
-// Partials a SchurOps needs per system.
-int schur_partials(int m, int jh_nblk);
+// The right-hand side b; v.x holds x0, unless x0_zero: then it is set to zero (and
+// r = b without a solve).  bt's mask: the systems taking part.
+void cg_start(SchurOps& o, const double* b, const dev::Batch& bt, bool x0_zero);
+// Up to `count` more iterations, o.k of itmax at most, for the live systems.
+// The stopping test of the last one is taken by the next call or by
+// dev::finish(.., o.k, ..).
+void cg_iterate(SchurOps& o, int count, double tol, int itmax, const dev::Batch& bt);
 
 struct CgResult {
   int iters = 0, status = 0;
   double final_norm = 0.0;
 };
-
-// SchurComplementConjugateGradient::solve (…ConjugateGradient.cpp:89-194)
-// on the device for the systems of `b` (its mask: the systems taking part):
-// ops.x holds x0 on entry and the solution on exit.  Every system's stopping
-// test (sqrt(r.r) < tol, or itmax iterations) is taken on the device, which
-// then leaves that system alone; the host reads the systems' live flags
-// only after `chunk` iterations and then after every `chunk_next`, so the
-// iterations in between run without a host round trip.  x0_zero: every x is
-// zero (r = b without a solve).  Returns per system (count entries).
-std::vector<CgResult> schur_cg_run(SchurOps& ops, const double* b, double tol, int itmax,
-                                   const dev::Batch& bt, bool x0_zero, int chunk,
-                                   int chunk_next = 1);
-// The results of a deferred schur_cg_run from its pinned memory.
-void cg_unpack(const double* pinned, std::vector<CgResult>& res);
+// From a system's FIN_SLOTS doubles of dev::finish().
+CgResult cg_result(const double* fin);
 
 }  // namespace hykkt

@@ -28,45 +28,36 @@ struct Batch {
 };
 inline Batch masked(const Batch& b, const int* m) { return Batch{b.count, b.vs, m}; }
 
+// The bit pattern a sweep's exchanged values hold until they are written: a
+// signalling-NaN payload no arithmetic result carries.
+constexpr uint64_t SWEEP_SENTINEL = 0x7ff4dead0badf00dull;
+// The buffers of one solve to fill with it before the sweeps (p[j], n[j] doubles
+// per system) and the sweeps' four item counters to zero; empty: nothing to do.
+struct SweepFill {
+  double* p[4] = {};
+  int64_t n[4] = {};
+  int* ticket = nullptr;
+};
+
 // ---------------------------------------------------------------- vectors
 void fill(double* p, double v, int64_t n, const Batch& b, hipStream_t st);
 // p[i] = v for i < n, one array (no batch)
 void fill_i(int* p, int v, int64_t n, hipStream_t st);
 void copy(double* dst, const double* src, int64_t n, const Batch& b, hipStream_t st);
-// dst[k] <- src[k] for each system k with keep[k] != 0 (both per-system)
-void copy_where(double* dst, const double* src, int64_t n, const int* keep, const Batch& b,
-                hipStream_t st);
-// dst[i] = src[map[i]]  (map_idx, permcheck.cu:12-19; map shared)
-void gather(double* dst, const double* src, const int* map, int64_t n, const Batch& b,
-            hipStream_t st);
 // dst[i] = src[map[i]] with 64-bit positions (one system)
 void gather64(double* dst, const double* src, const int64_t* map, int64_t n, hipStream_t st);
-// dst[i] = src[map[i]] * scale[i]
-void gather_scale(double* dst, const double* src, const int* map, const double* scale, int n,
-                  const Batch& b, hipStream_t st);
-// The recovery's two scaled results in one launch: dx[i] = (h0[map[i]] -
-// cz[map[i]]) * max_d[i] for i < n, dyc[i] = cx[i] * max_d[n + i] for i < m.
-void recover_xy(double* dx, const double* h0, const double* cz, const int* map,
-                const double* max_d, int n, double* dyc, const double* cx, int m, const Batch& b,
-                hipStream_t st);
 // y[i] *= s[i]  (vec_scale, matrix_vector_ops.cu:385-392)
 void vec_scale(double* y, const double* s, int n, const Batch& b, hipStream_t st);
-// out = a + b
-// out = a - b (per system)
-void sub(double* out, const double* a, const double* bv, int64_t n, const Batch& b,
-         hipStream_t st);
-// CG tracking: q = beta q + t, z += alpha q (alpha, beta from the CG scalars sc)
-void cg_track(int n, const double* sc, double* q, double* z, const double* t, const Batch& b,
-              hipStream_t st);
-void add(double* out, const double* a, const double* bv, int64_t n, const Batch& b,
-         hipStream_t st);
-// out[k*nslot + j] = base[k*vs + j] for j < nslot and each system k (b.count
-// systems, mask ignored): per-system scalars gathered for one readback.
-void collect(double* out, const double* base, int nslot, const Batch& b, hipStream_t st);
-// Per system k: the arrays src[k*nsrc + j] (j < nsrc, device pointers to
-// caller memory, lengths len[j]) copied to dst[j] + k*vs (arena slots).
-void copy_in(int nsrc, double* const* dst, const double* const* src_tab, const int64_t* len,
-             const Batch& b, hipStream_t st);
+// Caller memory into arena slots: for systems s < b.count, array j < COPY_ARRAYS of
+// system s from src[s * COPY_ARRAYS + j] (device pointers, len[j] doubles; null:
+// zeros if zero_null[j], else left alone) to dst[j] + s*vs, and scalar[s] to
+// dst_scalar + s*vs.  The pointers and scalars travel as kernel arguments,
+// COPY_SYSTEMS systems a launch: nothing is staged or copied ahead.  start (may be
+// null): event recorded as the first launch starts.
+constexpr int COPY_ARRAYS = 9, COPY_SYSTEMS = 16;
+void copy_in(double* const* dst, const int64_t* len, const bool* zero_null,
+             const double* const* src, double* dst_scalar, const double* scalar, const Batch& b,
+             hipStream_t st, hipEvent_t start = nullptr);
 
 // ---------------------------------------------------------------- sparse
 // jd_vs = Ds-row-scaled Jd (skipped if jd_vs is null); ryd_s = ryd*ds + rs
@@ -85,11 +76,16 @@ int spmv_lds_entries();
 // coalesced loads, then each row is summed by one thread in that order.
 // alpha_ps (may be null): per-system alpha (arena slot) instead of alpha.
 // dot_w (may be null): also dot_part[blk] = sum over the block's rows of
-// y_out[i] * dot_w[i] (per-system, for a fused w.r).
+// y_out[i] * dot_w[i] (per-system, for a fused w.r).  y_map (may be null): y_in is
+// read at y_map[i].  fill: sweep buffers to prepare on the way.
 void spmv(int nrows, const int* rp, const int* ci, const int* map, const double* v, double alpha,
           const double* alpha_ps, const double* x, double beta, const double* y_in,
           double* y_out, const int* blocks, int nblk, const Batch& b, hipStream_t st,
-          const double* dot_w = nullptr, double* dot_part = nullptr);
+          const double* dot_w = nullptr, double* dot_part = nullptr, const int* y_map = nullptr,
+          const SweepFill& fill = SweepFill{});
+// y = A x, the same sums, without row blocks planned ahead (64 rows a workgroup).
+void spmv_rows(int nrows, const int* rp, const int* ci, const double* v, const double* x, double* y,
+               const Batch& b, hipStream_t st);
 // out[p] = d_v[d_src[p]] (or 0) + alpha_p*acc, acc = sum fma(av[ta], bv[tb]) over terms of p
 void spgemm_values(int nnz_out, const int* d_src, const double* d_v, const int* term_ptr,
                    const int* ta, const int* tb, const double* av, const double* bv,
@@ -147,35 +143,20 @@ void ruiz_scale(int n, int totn, const int* h_rp, const int* h_ci, double* h_v,
 // ---------------------------------------------------------------- reductions
 // Block partial sums of a length-n reduction: reduce_blocks(n) blocks, a
 // function of n only (the same for every batch).
-int reduce_blocks(int64_t n);
-// Deterministic sum of a[i]*b[i] (bv == null: sum of a[i]); result to *out.
-// `part` needs reduce_blocks(n) doubles per system.
-void dot(int n, const double* a, const double* bv, double* part, double* out, const Batch& b,
-         hipStream_t st);
-// Up to DOTS_MAX such sums in two launches, out[k] per system for sum k
-// (same bits as dot() each); part needs the sum of their reduce_blocks(n[k])
-// doubles per system.  off is filled in by dots().
-constexpr int DOTS_MAX = 8;
-struct DotSet {
-  const double* a[DOTS_MAX];
-  const double* b[DOTS_MAX];
-  int n[DOTS_MAX];
-  int off[DOTS_MAX + 1];
-  int count = 0;
-};
-void dots(DotSet d, double* part, double* out, const Batch& b, hipStream_t st);
-// Per system k (b.count systems, stride b.vs between sc slots): sc[0], sc[1],
-// iters[k], status[k] as out[4k .. 4k+3].
-void cg_pack(double* out, const double* sc, const int* iters, const int* status, const Batch& b,
-             hipStream_t st);
-// out[0] = *w, then a[0..count) and bv[0..count) where not null.
-void collect_ints(int* out, const int* w, const int* a, const int* bv, int count, hipStream_t st);
-// The first stage of dot(): reduce_blocks(n) partials per system in part.
+__host__ __device__ inline int reduce_blocks_of(int64_t n)
+{
+  const int64_t g = (n + 255) / 256;
+  return static_cast<int>(g < 1 ? 1 : (g > 256 ? 256 : g));
+}
+inline int reduce_blocks(int64_t n) { return reduce_blocks_of(n); }
+// Deterministic partial sums of a[i]*b[i] in part: reduce_blocks(n) per system.
 void dot_partial(int n, const double* a, const double* bv, double* part, const Batch& b,
                  hipStream_t st);
 
 // ---------------------------------------------------------------- CG
-// CG scalars per system: sc[0]=gam [1]=gam1 [2]=delta [3]=alpha [4]=beta.
+// CG scalars per system: gam (r.r) and alpha of iteration k at the parity of k,
+// the last r.r.
+enum { CG_GAM = 0, CG_ALPHA = 2, CG_RR = 4, CG_SLOTS = 8 };
 // Per-system ints (one array each, indexed by system): live (1 while the
 // system iterates), iters, status.
 struct CgFlags {
@@ -183,48 +164,91 @@ struct CgFlags {
   int* iters;
   int* status;
 };
-// p = beta p + r; s = beta s + w; x += alpha p; r -= alpha s, and the block
-// partials of r.r in part (reduce_blocks(m) per system)
-void cg_update_dot(int m, const double* sc, double* p, double* s, double* x, double* r,
-                   const double* w, double* part, const Batch& b, hipStream_t st);
-// sc[slot] = sum of the np partials in part; with check (slot 1, iteration `it`): the
-// stopping test of SchurComplementConjugateGradient.cpp:164-170 -- sqrt(gam1)
-// < tol ends the system (iters it+1, status 0), it+1 == itmax ends it with
-// status 1.  With it < 0 (the start, slot 0): r.r == 0 ends it (iters 0).
-// With scalars (slot 2): then beta = gam1/gam, gam = gam1,
-// alpha = gam/(delta - beta gam/alpha) (:181-183), or alpha = gam/delta for
-// it < 0 (:143).
-void dot_final(int np, double* part, double* sc, int slot, bool check, bool scalars, int it,
-               double tol, int itmax, const CgFlags& f, const Batch& b, hipStream_t st);
+// The CG's vectors of system 0: x, r, w, p, s (m); t1, t2 (n, the solves' right-
+// hand side and solution); optionally q, z (n); scalars; partials of r.r
+// (reduce_blocks(m)) and of w.r (np2).
+struct CgVecs {
+  int m, n;
+  double *x, *r, *w, *p, *s, *t1, *t2, *q, *z, *sc, *part, *part2;
+  int np2;
+};
+// The flags of all b.count systems (live: those of b.mask); p = s = rhs, q = z =
+// 0 and, with x0_zero, x = 0, r = rhs and the partials of r.r.
+void cg_start(const CgVecs& c, const double* rhs, bool x0_zero, const CgFlags& f, const Batch& b,
+              hipStream_t st);
+// The stopping test after k updates, then t1 = Jh^T r and the sweeps' buffers filled.
+void cg_apply(const CgVecs& c, int k, double tol, int itmax, const int* jth_rp, const int* jth_ci,
+              const double* jth_v, const SweepFill& fill, const CgFlags& f, const Batch& b,
+              hipStream_t st);
+// Iteration k's update of x, r, p, s (and q, z) and the partials of r.r.
+void cg_update(const CgVecs& c, int k, const CgFlags& f, const Batch& b, hipStream_t st);
 
-// ---------------------------------------------------------------- recover / residual
-// Residual pieces, squares written per element for dot():
-//   n rows: r1 = rx - H dx - Jc^T dyc - Jd^T dyd   (Jc^T, Jd^T via transposes + maps)
-void resid_rows_n(int n, const int* h_rp, const int* h_ci, const double* h_v,
-                  const int* jct_rp, const int* jct_ci, const int* jct_map, const double* jc_v,
-                  const int* jdt_rp, const int* jdt_ci, const int* jdt_map, const double* jd_v,
-                  const double* rx, const double* dx, const double* dyc, const double* dyd,
-                  double* sq, double* e, const Batch& b, hipStream_t st);
-//   m rows: r3 = ry - Jc dx
-void resid_rows_m(int m, const int* jc_rp, const int* jc_ci, const double* jc_v, const double* ry,
-                  const double* dx, double* sq, double* e, const Batch& b, hipStream_t st);
-//   d rows: r2 = rs - (Ds ds - dyd), r4 = ryd - (Jd dx - ds)
-// e, e2, e4 (may be null): the signed residual rows, for iterative refinement.
-void resid_rows_d(int d, const int* jd_rp, const int* jd_ci, const double* jd_v, int has_jd,
-                  const double* ds, const double* rs, const double* ryd, const double* dx,
-                  const double* dsv, const double* dyd, double* sq2, double* sq4, double* e2,
-                  double* e4, const Batch& b, hipStream_t st);
-// ds = Jd dx - ryd (or -ryd); dyd = ds*Ds - rs
-void recover_d(int d, const int* jd_rp, const int* jd_ci, const double* jd_v, int has_jd,
-               const double* dx, const double* ryd, const double* ds_diag, const double* rs,
-               double* dsv, double* dyd, const Batch& b, hipStream_t st);
+// ---------------------------------------------------------------- pass
+// After the factorization: jh_v[i] = jcs[jh_map[i]], jth_v[i] = jcs[jth_map[i]]; ok = 0
+// and a zero solution for systems with a failing pivot, else ok = 1.  start
+// (may be null): event recorded as the launch starts.
+struct AfterFactor {
+  const int* pivot;
+  int* ok;
+  const double* jcs;
+  const int *jh_map, *jth_map;
+  double *jh_v, *jth_v;
+  int nnz, n, m, d;
+  double *dx, *dsv, *dyc, *dyd;
+};
+void after_factor(const AfterFactor& c, const Batch& b, hipStream_t st, hipEvent_t start = nullptr);
+// The solution of the 4x4 system from the CG's iterate: dx[i] = (h0[ipos[i]] -
+// z[ipos[i]]) max_d[i], dyc = x max_d[n..], dsv = Jd dx - ryd (has_jd = 0: -ryd), dyd =
+// dsv Ds - rs; base_* (may be null): added to the results.
+struct Recover {
+  int n, m, d, has_jd;
+  const double *h0, *z, *x, *max_d;
+  const int *ipos, *jd_rp, *jd_ci;
+  const double *jd_v, *ryd, *ds, *rs;
+  double *dx, *dsv, *dyc, *dyd;
+  const double *base_dx, *base_dsv, *base_dyc, *base_dyd;
+  int nbd;   // set by recover()
+};
+void recover(Recover c, const Batch& b, hipStream_t st, hipEvent_t start = nullptr);
+// Signed residual rows e_x = rx - H dx - Jc^T dyc - Jd^T dyd (ct_*, dt_*: the
+// transposes' patterns and their maps into the values), e_y = ry - Jc dx, e_s = rs -
+// (Ds ds - dyd), e_d = ryd - (Jd dx - ds), and partial sums of squares for
+// finish() (residual_partials() doubles per system).
+struct Residual {
+  int n, m, d, has_jd;
+  const int *h_rp, *h_ci, *ct_rp, *ct_ci, *ct_map, *dt_rp, *dt_ci, *dt_map, *jc_rp, *jc_ci, *jd_rp,
+      *jd_ci;
+  const double *h_v, *jc_v, *jd_v, *ds, *rx, *rs, *ry, *ryd, *dx, *dsv, *dyc, *dyd;
+  double *e_x, *e_s, *e_y, *e_d, *part;
+  int nbn, nbm, nbd, stride;   // set by residual()
+};
+int residual_partials(int n, int m, int d);
+void residual(Residual& c, const Batch& b, hipStream_t st);
+// What the host reads of a pass, per system: squared norms of residual rows 1, 3,
+// 2, 4 and of rx, rs, ry, ryd; the CG's r.r at exit, iterations, status and live
+// flag; the zero-row and pivot words (INT_MAX: none), the sweeps' error word.
+enum {
+  FIN_RES = 0, FIN_RR = 8, FIN_ITERS, FIN_STATUS, FIN_LIVE, FIN_ZERO_ROW, FIN_PIVOT, FIN_SWEEP_ERR,
+  FIN_SLOTS = 16
+};
+struct Finish {
+  double* out;   // FIN_SLOTS doubles per system, in memory the host can read
+  const int *zero_row, *pivot, *sweep_err;
+  const double* part;   // set by finish()
+  int np[8], stride;
+};
+// After k updates: the CG's stopping test, the residual's sums (r: of the launch
+// before; may be null) and out.  stop (may be null): event recorded at the end.
+void finish(Finish c, const Residual* r, const CgVecs& v, int k, double tol, int itmax,
+            const CgFlags& f, const Batch& b, hipStream_t st, hipEvent_t stop = nullptr);
+// dst[j] <- src[j] (n[j] doubles) for the systems with keep != 0 (null: all)
+struct Keep {
+  const double* src[4];
+  double* dst[4];
+  int n[4];
+};
+void keep_where(const Keep& c, const int* keep, const Batch& b, hipStream_t st);
 
-// ok[s] = (system s's factorization met no failing pivot); a system that
-// did gets a zero solution (dx n, dsv d, dyc m, dyd d).
-void pivot_split(const int* pivot, int* ok, int n, int m, int d, double* dx, double* dsv,
-                 double* dyc, double* dyd, const Batch& b, hipStream_t st);
-
-// ---------------------------------------------------------------- scratch
 // The allocation-free entry point's device scratch (noalloc.hip): its size
 // in bytes, and its address on the current device (taken once per device).
 size_t noalloc_scratch_bytes();
@@ -348,11 +372,8 @@ struct SolveDev {
 };
 // Workgroups of a forest sweep one compute unit holds at once.
 int forest_blocks_per_cu();
-// p[i] = the sentinel, i < n (per system); zero4 (when not null): four ints set to 0
-void fill_sentinel(double* p, int64_t n, const Batch& b, hipStream_t st, int* zero4 = nullptr);
-// The same for three buffers (p_i[0..n_i)) in one launch.
-void fill_sentinel3(double* p0, int64_t n0, double* p1, int64_t n1, double* p2, int64_t n2,
-                    const Batch& b, hipStream_t st, int* zero4 = nullptr);
+// The buffers of f filled with the sentinel, in a launch of its own.
+void fill_sentinel(const SweepFill& f, const Batch& b, hipStream_t st);
 // L y = b (b, y internal order; y sentinel-filled, ubuf sentinel-filled): the
 // forest, then the top of the tree.
 void solve_forward_forest(const CholDev& c, const SolveDev& sd, const double* rhs, double* y,

@@ -55,6 +55,7 @@
 
 #include <algorithm>
 
+#include "basic_dev.hpp"
 #include "sweep_dev.hpp"
 
 namespace hykkt {
@@ -98,25 +99,12 @@ __device__ __forceinline__ double sum_slices(const double (*part)[SB], int i)
   return a + b;
 }
 
-// Up to three buffers in one launch: element i of the concatenation
-// p0[0..n0) p1[0..n1) p2[0..n2) takes the sentinel.
-__global__ void k_fill_sentinel(double* __restrict__ p0, int64_t n0, double* __restrict__ p1,
-                                int64_t n1, double* __restrict__ p2, int64_t n2,
-                                int* __restrict__ zero4, Batch bt)
+__global__ void k_fill_sentinel(SweepFill f, Batch bt)
 {
-  if (zero4 && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 4)
-    __hip_atomic_store(zero4 + threadIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  clear_tickets(f.ticket);
   const int sy = batch_sys(bt);
   if (sy < 0) return;
-  p0 = batch_at(p0, sy, bt);
-  p1 = batch_at(p1, sy, bt);
-  p2 = batch_at(p2, sy, bt);
-  const int64_t n = n0 + n1 + n2;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double* p = i < n0 ? p0 + i : (i < n0 + n1 ? p1 + (i - n0) : p2 + (i - n0 - n1));
-    *p = __builtin_bit_cast(double, SENTINEL);
-  }
+  fill_sweep(f, sy, bt, blockIdx.x, gridDim.x);
 }
 
 // A slice of QW values, value k at byte offset vo + so0 + k*sstride of the
@@ -433,24 +421,12 @@ __global__ void __launch_bounds__(NT) k_solve_bwd(CholDev c, SolveDev sd,
 
 }  // namespace
 
-void fill_sentinel(double* p, int64_t n, const Batch& b, hipStream_t st, int* zero4)
+void fill_sentinel(const SweepFill& f, const Batch& b, hipStream_t st)
 {
-  fill_sentinel3(p, n, nullptr, 0, nullptr, 0, b, st, zero4);
-}
-
-void fill_sentinel3(double* p0, int64_t n0, double* p1, int64_t n1, double* p2, int64_t n2,
-                    const Batch& b, hipStream_t st, int* zero4)
-{
-  n0 = std::max<int64_t>(n0, 0);
-  n1 = std::max<int64_t>(n1, 0);
-  n2 = std::max<int64_t>(n2, 0);
-  const int64_t n = n0 + n1 + n2;
-  if ((n <= 0 && !zero4) || b.count <= 0) return;
-  int64_t g = (n + 255) / 256;
-  if (g > 65536) g = 65536;
-  if (g < 1) g = 1;
-  k_fill_sentinel<<<dim3(static_cast<unsigned>(g), b.count), 256, 0, st>>>(p0, n0, p1, n1, p2,
-                                                                             n2, zero4, b);
+  if (b.count <= 0) return;
+  int64_t n = 1;
+  for (int j = 0; j < 4; j++) n = std::max(n, f.n[j]);
+  k_fill_sentinel<<<dim3(nblocks(n), b.count), TPB, 0, st>>>(f, b);
   HIPCHK(hipGetLastError());
 }
 

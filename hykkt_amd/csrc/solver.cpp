@@ -6,8 +6,7 @@
 // pattern lives in one arena, system k's copy `stride` doubles after system
 // k-1's, so each launch covers all the systems of the batch (system
 // blockIdx.y) and a system's arithmetic is the same alone or in a batch.
-// The host reads back the CG live flags between chunks of iterations and
-// the residuals once per pass.
+// The host reads a pass's results once: the device writes them to pinned memory.
 #include "solver.hpp"
 
 #include <algorithm>
@@ -24,10 +23,10 @@ namespace hykkt {
 struct Solver::Slots {
   int64_t in[IN_COUNT] = {}, gam = 0;
   int64_t jd_vs = 0, ryd_s = 0, rx_til = 0, htil = 0, jcs = 0, ry_s = 0, max_d = 0, scale = 0, scale2 = 0;
-  int64_t jch_v = 0, jcth_v = 0, rxp = 0, tmp_n = 0, t1 = 0;
-  int64_t cx = 0, cr = 0, cw = 0, cp = 0, cs = 0, schur = 0, sc = 0, part = 0;
+  int64_t jch_v = 0, jcth_v = 0, rxp = 0, t1 = 0, t2 = 0;
+  int64_t cx = 0, cr = 0, cw = 0, cp = 0, cs = 0, schur = 0, sc = 0, part = 0, part2 = 0, rpart = 0;
   int64_t h0 = 0, cq = 0, cz = 0;
-  int64_t dx = 0, dsv = 0, dyc = 0, dyd = 0, sq_n = 0, sq_m = 0, sq_d2 = 0, sq_d4 = 0, res = 0;
+  int64_t dx = 0, dsv = 0, dyc = 0, dyd = 0;
   int64_t e_x = 0, e_s = 0, e_y = 0, e_d = 0, e_rxt = 0, e_ysc = 0, e_rxp = 0, e_schur = 0;
   int64_t e_cx = 0, c_dx = 0, c_dsv = 0, c_dyc = 0, c_dyd = 0;
   int64_t L = 0, U = 0, dinv = 0, y = 0, ubuf = 0, bpart = 0;
@@ -36,7 +35,6 @@ struct Solver::Slots {
 
 // per-system int flags, one array of `cap` each
 enum { FL_PIVOT = 0, FL_ZERO_ROW, FL_LIVE, FL_ACT, FL_KEEP, FL_CG_IT, FL_CG_ST, FL_OK, FL_COUNT };
-constexpr int RES_SLOTS = 8;
 
 struct Solver::Sym {
   int n = 0, m = 0, d = 0, nnz_h = 0, nnz_jc = 0, nnz_jd = 0, nnz_ds = 0;
@@ -65,26 +63,16 @@ struct Solver::Sym {
   int cap = 0;
   DevBuf<double> arena;
   DevBuf<int> flags;         // FL_COUNT arrays of cap ints
-  DevBuf<double> gath;       // cap * RES_SLOTS: per-system scalars gathered for a readback
-  DevBuf<double> gam_dev;    // cap gammas (staging for the copy into the arena)
-  DevBuf<const double*> tab; // cap * (IN_COUNT + 1) caller pointers for copy_in
-  HostBuf<double> readback;  // pinned: per-pass results copied back in one round trip
-  HostBuf<double> cg_host;   // pinned: the CG's live flags and results
-  // pinned staging of the gammas and the pointer table (inputs on the
-  // device), and the event after their copies
-  HostBuf<double> gam_h;
-  HostBuf<const double*> tab_h;
-  hipEvent_t up_done = nullptr;
+  // pinned: what the host reads of a pass (written by the device), and the
+  // per-system flags it sends
+  HostBuf<double> fin;
+  HostBuf<int> flag_host;
   int* flag(int which) { return flags.p + static_cast<int64_t>(which) * cap; }
   // the engine's second stream may still be zeroing the factor storage in
   // the arena (prezero_L): let it finish before the members are freed
   ~Sym()
   {
     if (chol) chol->quiesce();
-    if (up_done) {
-      (void)hipEventSynchronize(up_done);
-      (void)hipEventDestroy(up_done);
-    }
   }
 };
 
@@ -420,8 +408,8 @@ void Solver::analyze()
   z.jch_v = slot(S->nnz_jc);
   z.jcth_v = slot(S->nnz_jc);
   z.rxp = slot(n);
-  z.tmp_n = slot(n);
   z.t1 = slot(n);
+  z.t2 = slot(n);
   z.h0 = slot(n);
   z.cq = slot(n);
   z.cz = slot(n);
@@ -431,17 +419,14 @@ void Solver::analyze()
   z.cp = slot(m);
   z.cs = slot(m);
   z.schur = slot(m);
-  z.sc = slot(8);
-  z.part = slot(std::max(8 * 256, schur_partials(m, S->jch_nblk)));   // 8 residual sums
+  z.sc = slot(dev::CG_SLOTS);
+  z.part = slot(dev::reduce_blocks(m));
+  z.part2 = slot(S->jch_nblk);
+  z.rpart = slot(dev::residual_partials(n, m, d));
   z.dx = slot(n);
   z.dsv = slot(d);
   z.dyc = slot(m);
   z.dyd = slot(d);
-  z.sq_n = slot(n);
-  z.sq_m = slot(m);
-  z.sq_d2 = slot(d);
-  z.sq_d4 = slot(d);
-  z.res = slot(RES_SLOTS);
   z.e_x = slot(n);
   z.e_s = slot(d);
   z.e_y = slot(m);
@@ -466,9 +451,8 @@ void Solver::analyze()
   S->cap = cap_;
   S->arena.alloc(static_cast<size_t>(z.stride) * cap_);
   S->flags.alloc(static_cast<size_t>(FL_COUNT) * cap_);
-  S->gath.alloc(static_cast<size_t>(RES_SLOTS) * cap_ + cap_ + 1);   // + read_res's ints
-  S->gam_dev.alloc(static_cast<size_t>(cap_));
-  S->tab.alloc(static_cast<size_t>(IN_COUNT + 1) * cap_);
+  S->fin.ensure(static_cast<size_t>(dev::FIN_SLOTS) * cap_);
+  S->flag_host.ensure(2 * static_cast<size_t>(cap_));
   double* base = S->arena.p;
   S->chol->bind(CholEngine::Storage{base + z.L, base + z.U, base + z.dinv, base + z.y,
                                     base + z.ubuf, base + z.bpart, S->flags.p + FL_PIVOT * cap_},
@@ -495,45 +479,34 @@ void Solver::analyze()
 }
 
 // ------------------------------------------------------------------ values
-// Copy each system's values into its arena slots: one copy kernel over all
-// systems from device pointers, or host-to-device copies from host arrays.
+// Copy each system's values into its arena slots: a copy kernel over the systems
+// from device pointers, or host-to-device copies from host arrays.
 void Solver::upload_values(int count)
 {
   Sym& S = *sym_;
   const Slots& z = S.z;
   const dev::Batch b{count, z.stride, nullptr};
-  const int64_t len[IN_COUNT + 1] = {S.nnz_h, S.d, S.nnz_jc, S.nnz_jd, S.n, S.d, S.m, S.d, S.m, 1};
+  const int64_t len[IN_COUNT] = {S.nnz_h, S.d, S.nnz_jc, S.nnz_jd, S.n, S.d, S.m, S.d, S.m};
   bool any_y0 = false;
   std::vector<double> gam(count);
   for (int k = 0; k < count; k++) {
     gam[k] = sys_in_[k].gamma;
     any_y0 = any_y0 || sys_in_[k].v[IN_Y0] != nullptr;
   }
-  // a system without its own start y begins at zero
-  if (any_y0) dev::fill(P(z.in[IN_Y0]), 0.0, S.m, b, st_);
   if (opts.inputs_on_device) {
-    // the gammas and the pointer table go through pinned staging, so the
-    // copies need no wait here; the staging is refilled only once the
-    // previous execute's copies are done (normally long since)
-    if (!S.up_done) HIPCHK(hipEventCreateWithFlags(&S.up_done, hipEventDisableTiming));
-    else HIPCHK(hipEventSynchronize(S.up_done));
-    const size_t nt = static_cast<size_t>(IN_COUNT + 1) * count;
-    S.gam_h.ensure(count);
-    S.tab_h.ensure(nt);
-    for (int k = 0; k < count; k++) {
-      S.gam_h.p[k] = gam[k];
-      for (int j = 0; j < IN_COUNT; j++) S.tab_h.p[k * (IN_COUNT + 1) + j] = sys_in_[k].v[j];
-      S.tab_h.p[k * (IN_COUNT + 1) + IN_COUNT] = S.gam_dev.p + k;
+    static_assert(IN_COUNT == dev::COPY_ARRAYS, "one copy per input array");
+    double* dst[IN_COUNT];
+    bool zero[IN_COUNT] = {};
+    zero[IN_Y0] = any_y0;   // a system without its own start y begins at zero
+    std::vector<const double*> src(static_cast<size_t>(IN_COUNT) * count);
+    for (int j = 0; j < IN_COUNT; j++) {
+      dst[j] = P(z.in[j]);
+      for (int k = 0; k < count; k++) src[static_cast<size_t>(k) * IN_COUNT + j] = sys_in_[k].v[j];
     }
-    HIPCHK(hipMemcpyAsync(S.gam_dev.p, S.gam_h.p, sizeof(double) * count, hipMemcpyHostToDevice,
-                          st_));
-    HIPCHK(hipMemcpyAsync(S.tab.p, S.tab_h.p, sizeof(double*) * nt, hipMemcpyHostToDevice, st_));
-    HIPCHK(hipEventRecord(S.up_done, st_));
-    double* dst[IN_COUNT + 1];
-    for (int j = 0; j < IN_COUNT; j++) dst[j] = P(z.in[j]);
-    dst[IN_COUNT] = P(z.gam);
-    dev::copy_in(IN_COUNT + 1, dst, S.tab.p, len, b, st_);
+    dev::copy_in(dst, len, zero, src.data(), P(z.gam), gam.data(), b, st_, ev_[0]);
   } else {
+    HIPCHK(hipEventRecord(ev_[0], st_));
+    if (any_y0) dev::fill(P(z.in[IN_Y0]), 0.0, S.m, b, st_);
     for (int k = 0; k < count; k++) {
       double* base = P(static_cast<int64_t>(k) * z.stride);
       for (int j = 0; j < IN_COUNT; j++)
@@ -700,7 +673,6 @@ std::vector<int> Solver::run(int count, bool from_setters)
   const int n = S.n, m = S.m, d = S.d;
   const dev::Batch b{count, z.stride, nullptr};
   tune_ms_ = 0.f;
-  HIPCHK(hipEventRecord(ev_[0], st_));
   upload_values(count);
   bool any_y0 = false;
   for (int k = 0; k < count; k++) any_y0 = any_y0 || sys_in_[k].v[IN_Y0] != nullptr;
@@ -778,51 +750,62 @@ std::vector<int> Solver::run(int count, bool from_setters)
 
   // ---- compute_hgamma_factorization (HykktSolver.cpp:398-401) ----
   ch.factor(opts.pivot_tol, b, !(fresh && opts.autotune));   // the tuning runs record pivots, too
-  HIPCHK(hipEventRecord(ev_[1], st_));
 
-  // permuted Jc and Jc^T values (apply_permutation, HykktSolver.cpp:386-395)
-  dev::gather(P(z.jch_v), P(z.jcs), S.jch_map.p, S.nnz_jc, b, st_);
-  dev::gather(P(z.jcth_v), P(z.jcs), S.jcth_map.p, S.nnz_jc, b, st_);
+  // permuted Jc and Jc^T values (apply_permutation, HykktSolver.cpp:386-395).  A
+  // system whose factorization met a failing pivot (reported with status 1, as the
+  // reference's) gets a zero solution and skips the solve phase, so a batch does
+  // not run its CG to the iteration limit on a broken factor.
+  dev::AfterFactor af{};
+  af.pivot = S.flag(FL_PIVOT);
+  af.ok = S.flag(FL_OK);
+  af.jcs = P(z.jcs);
+  af.jh_map = S.jch_map.p;
+  af.jth_map = S.jcth_map.p;
+  af.jh_v = P(z.jch_v);
+  af.jth_v = P(z.jcth_v);
+  af.nnz = S.nnz_jc;
+  af.n = n;
+  af.m = m;
+  af.d = d;
+  af.dx = P(z.dx);
+  af.dsv = P(z.dsv);
+  af.dyc = P(z.dyc);
+  af.dyd = P(z.dyd);
+  dev::after_factor(af, b, st_, ev_[1]);
 
-  // ---- first pass: the reference's solve (HykktSolver.cpp:404-457) ----
-  // A system whose factorization met a failing pivot (reported with status 1,
-  // as the reference's) gets a zero solution and skips the solve phase, so a
-  // batch does not run its CG to the iteration limit on a broken factor.
-  dev::pivot_split(S.flag(FL_PIVOT), S.flag(FL_OK), n, m, d, P(z.dx), P(z.dsv), P(z.dyc),
-                   P(z.dyd), b, st_);
-  const dev::Batch bok = dev::masked(b, S.flag(FL_OK));
+  // ---- first pass: the reference's solve (HykktSolver.cpp:404-457) and its
+  // check_error (:846-930), with rows 2 and 4 ----
   // CG start y_host, or zero when none is bound (then no start-residual solve)
-  std::vector<CgResult> cg = solve_phase(Pass{z.rxp, z.schur, z.cx}, z.rx_til, z.ry_s,
-                                         z.in[IN_RS], z.in[IN_RYD], any_y0, z.dx, z.dsv, z.dyc,
-                                         z.dyd, bok, ev_[2], last_iters_);
-
-  // ---- check_error (HykktSolver.cpp:846-930) + rows 2 and 4 ----
-  residual(z.dx, z.dsv, z.dyc, z.dyd, true, b);
-  HIPCHK(hipEventRecord(ev_[3], st_));
-  std::vector<int> zrow(count), keep(count), act(count), piv(count);
-  std::vector<double> hr = read_res(count, &zrow, &piv);
-  cg_unpack(S.cg_host.p, cg);   // its copy finished with read_res's synchronization
-  int it_max = 0;
-  for (const CgResult& r : cg) it_max = std::max(it_max, r.iters);
-  last_iters_ = it_max;
+  const Solution sol{z.dx, z.dsv, z.dyc, z.dyd}, none{-1, -1, -1, -1};
+  solve_pass(Pass{z.rxp, z.schur, z.cx}, z.rx_til, z.ry_s, z.in[IN_RS], z.in[IN_RYD], any_y0, sol,
+             none, dev::masked(b, S.flag(FL_OK)), b, last_iters_, true);
+  std::vector<int> zrow(count), piv(count);
   std::vector<int> rc(count, HYKKT_OK);
   std::vector<double> nb(count);
+  auto fin = [&](int k) { return S.fin.p + static_cast<size_t>(k) * dev::FIN_SLOTS; };
+  int it_max = 0;
   for (int k = 0; k < count; k++) {
     hykkt_stats& st = st_k_[k];
-    const double* h = hr.data() + static_cast<size_t>(k) * RES_SLOTS;
+    const double* h = fin(k) + dev::FIN_RES;
+    const CgResult cg = cg_result(fin(k));
+    it_max = std::max(it_max, cg.iters);
     nb[k] = h[4] + h[5] + h[6] + h[7];
     st.resid2 = std::sqrt(h[0] + h[1]) / std::sqrt(nb[k]);
     st.resid4 = std::sqrt(h[0] + h[1] + h[2] + h[3]) / std::sqrt(nb[k]);
     st.resid4_first = st.resid4;
     st.refine_steps = 0;
-    st.cg_iters = cg[k].iters;
-    st.cg_status = cg[k].status;
-    st.cg_final_norm = cg[k].final_norm;
+    st.cg_iters = cg.iters;
+    st.cg_status = cg.status;
+    st.cg_final_norm = cg.final_norm;
+    zrow[k] = static_cast<int>(fin(k)[dev::FIN_ZERO_ROW]);
+    piv[k] = static_cast<int>(fin(k)[dev::FIN_PIVOT]);
+    if (piv[k] == INT_MAX) piv[k] = -1;
     st.pivot = piv[k];
     // matrix_vector_ops.cu:258-264 scales a zero row by 1/sqrt(0) = inf and
     // the solve turns to NaN; here it is an argument error of that system
     if (zrow[k] != INT_MAX) rc[k] = HYKKT_E_ARG;
   }
+  last_iters_ = it_max;
 
   // ---- iterative refinement on the 4x4 block KKT system (an addition: the
   // reference stops after one pass).  The signed residual rows go through the
@@ -830,19 +813,28 @@ std::vector<int> Solver::run(int count, bool from_setters)
   // Ruiz scaling max_d) and the same solve phase with a zero CG start; a
   // correction is kept only if it lowers resid4.  Each system decides for
   // itself, as it would alone; the pass covers the systems still refining. ----
-  std::vector<int> stopped(count, 0);
+  std::vector<int> act(count), stopped(count, 0);
+  int* const act_h = S.flag_host.p;
+  int* const keep_h = S.flag_host.p + S.cap;
   const Pass corr{z.e_rxp, z.e_schur, z.e_cx};
+  const Solution csol{z.c_dx, z.c_dsv, z.c_dyc, z.c_dyd};
+  bool refined = false;
   for (int pass = 0; pass < opts.refine_max; pass++) {
     int nact = 0;
     for (int k = 0; k < count; k++) {
       act[k] = (rc[k] == HYKKT_OK && piv[k] < 0 && !stopped[k] &&
                 st_k_[k].resid4 > opts.refine_tol) ? 1 : 0;
+      act_h[k] = act[k];
       nact += act[k];
     }
     if (nact == 0) break;
-    HIPCHK(hipMemcpyAsync(S.flag(FL_ACT), act.data(), sizeof(int) * count, hipMemcpyHostToDevice,
-                          st_));
-    const dev::Batch ba = dev::masked(b, S.flag(FL_ACT));
+    refined = true;
+    dev::Batch ba = b;
+    if (nact < count) {   // else every system takes part: no mask
+      HIPCHK(hipMemcpyAsync(S.flag(FL_ACT), act_h, sizeof(int) * count, hipMemcpyHostToDevice,
+                            st_));
+      ba = dev::masked(b, S.flag(FL_ACT));
+    }
     if (S.has_jd) {
       dev::row_scale(d, S.jd_rp.p, in[IN_JD], in[IN_DS], P(z.e_d), P(z.e_s), nullptr, P(z.ryd_s),
                      ba, st_);
@@ -859,56 +851,51 @@ std::vector<int> Solver::run(int count, bool from_setters)
     // the correction's right-hand side is small: its CG usually stops within
     // an iteration or two, so its first look at the live flags comes from
     // the last refinement pass, not the first pass
-    std::vector<CgResult> cgr =
-        solve_phase(corr, z.e_rxt, z.e_ysc, z.e_s, z.e_d, false, z.c_dx, z.c_dsv, z.c_dyc,
-                    z.c_dyd, ba, nullptr, last_ref_iters_);
-    dev::add(P(z.c_dx), P(z.c_dx), P(z.dx), n, ba, st_);
-    dev::add(P(z.c_dsv), P(z.c_dsv), P(z.dsv), d, ba, st_);
-    dev::add(P(z.c_dyc), P(z.c_dyc), P(z.dyc), m, ba, st_);
-    dev::add(P(z.c_dyd), P(z.c_dyd), P(z.dyd), d, ba, st_);
-    residual(z.c_dx, z.c_dsv, z.c_dyc, z.c_dyd, true, ba);
-    hr = read_res(count);
-    cg_unpack(S.cg_host.p, cgr);
+    solve_pass(corr, z.e_rxt, z.e_ysc, z.e_s, z.e_d, false, csol, sol, ba, ba, last_ref_iters_,
+               false);
     int rit = 0;
     for (int k = 0; k < count; k++)
-      if (act[k]) rit = std::max(rit, cgr[k].iters);
+      if (act[k]) rit = std::max(rit, cg_result(fin(k)).iters);
     last_ref_iters_ = rit;
     int nkeep = 0;
     for (int k = 0; k < count; k++) {
-      keep[k] = 0;
+      keep_h[k] = 0;
       if (!act[k]) continue;
-      const double* h = hr.data() + static_cast<size_t>(k) * RES_SLOTS;
+      const double* h = fin(k) + dev::FIN_RES;
       const double c4 = std::sqrt(h[0] + h[1] + h[2] + h[3]) / std::sqrt(nb[k]);
       if (!(c4 < st_k_[k].resid4)) {   // keep the better solution; its rows in e_* are stale
         stopped[k] = 1;
         continue;
       }
-      keep[k] = 1;
+      keep_h[k] = 1;
       nkeep++;
       st_k_[k].resid2 = std::sqrt(h[0] + h[1]) / std::sqrt(nb[k]);
       st_k_[k].resid4 = c4;
       st_k_[k].refine_steps++;
     }
     if (nkeep == 0) break;
-    HIPCHK(hipMemcpyAsync(S.flag(FL_KEEP), keep.data(), sizeof(int) * count,
-                          hipMemcpyHostToDevice, st_));
-    dev::copy_where(P(z.dx), P(z.c_dx), n, S.flag(FL_KEEP), b, st_);
-    dev::copy_where(P(z.dsv), P(z.c_dsv), d, S.flag(FL_KEEP), b, st_);
-    dev::copy_where(P(z.dyc), P(z.c_dyc), m, S.flag(FL_KEEP), b, st_);
-    dev::copy_where(P(z.dyd), P(z.c_dyd), d, S.flag(FL_KEEP), b, st_);
+    if (nkeep < count)
+      HIPCHK(hipMemcpyAsync(S.flag(FL_KEEP), keep_h, sizeof(int) * count, hipMemcpyHostToDevice,
+                            st_));
+    dev::Keep kp{{P(z.c_dx), P(z.c_dsv), P(z.c_dyc), P(z.c_dyd)},
+                 {P(z.dx), P(z.dsv), P(z.dyc), P(z.dyd)},
+                 {n, d, m, d}};
+    dev::keep_where(kp, nkeep < count ? S.flag(FL_KEEP) : nullptr, b, st_);
   }
-  HIPCHK(hipEventRecord(ev_[4], st_));
-  HIPCHK(hipEventSynchronize(ev_[4]));
+  if (refined) {
+    HIPCHK(hipEventRecord(ev_[4], st_));
+    HIPCHK(hipEventSynchronize(ev_[4]));
+  }
   prof.collect();
   // the factor is done with: zero its storage for the next execute now, on
   // the factorization's second stream, while the caller reads the results
   S.chol->prezero_L(count);
 
   float ms[4] = {};
-  HIPCHK(hipEventElapsedTime(&ms[0], ev_[0], ev_[4]));
+  HIPCHK(hipEventElapsedTime(&ms[0], ev_[0], ev_[refined ? 4 : 3]));
   HIPCHK(hipEventElapsedTime(&ms[1], ev_[0], ev_[1]));
   HIPCHK(hipEventElapsedTime(&ms[2], ev_[1], ev_[2]));
-  HIPCHK(hipEventElapsedTime(&ms[3], ev_[3], ev_[4]));
+  if (refined) HIPCHK(hipEventElapsedTime(&ms[3], ev_[3], ev_[4]));
   ms[0] -= tune_ms_;   // the autotuning runs sit between ev_[0] and ev_[1]
   ms[1] -= tune_ms_;
   for (int k = 0; k < count; k++) {
@@ -931,38 +918,40 @@ std::vector<int> Solver::run(int count, bool from_setters)
 }
 
 // setup_conjugate_gradient (HykktSolver.cpp:814-843), the Schur CG
-// (SchurComplementConjugateGradient.cpp:89-194) and recover_solution
-// (HykktSolver.cpp:410-457) for Ruiz-scaled right-hand sides rxt (n, natural
-// order) and ysc (m); rs, ryd are the unscaled d-rows used by the recovery.
-// All arguments are arena offsets; the systems of b (its mask) take part.
-std::vector<CgResult> Solver::solve_phase(const Pass& w, int64_t rxt, int64_t ysc, int64_t rs,
-                                          int64_t ryd, bool x0, int64_t dx, int64_t dsv,
-                                          int64_t dyc, int64_t dyd, const dev::Batch& b,
-                                          hipEvent_t after_cg, int iters_hint)
+// (SchurComplementConjugateGradient.cpp:89-194), recover_solution
+// (HykktSolver.cpp:410-457) and the residual rows, for Ruiz-scaled right-hand sides
+// rxt (n, natural order) and ysc (m); rs, ryd are the unscaled d-rows used by the
+// recovery.  All arguments are arena offsets; the systems of bs take part in the
+// solve, those of br in the recovery's and residual's results.
+//
+// The host looks at the systems once after as many iterations as the last pass
+// of the kind took (`hint`), or every cg_check_every: recovery, residual and the
+// results' launch are enqueued with them, as if every system stopped there, so
+// the usual pass has one host round trip and no iteration that nobody needs.  If
+// a system is still live, the CG goes on and they run again.
+void Solver::solve_pass(const Pass& w, int64_t rxt, int64_t ysc, int64_t rs, int64_t ryd, bool x0,
+                        const Solution& out, const Solution& base, const dev::Batch& bs,
+                        const dev::Batch& br, int hint, bool first)
 {
   Sym& S = *sym_;
   const Slots& z = S.z;
   const int n = S.n, m = S.m, d = S.d;
-  // r^x = r~x + gamma Jc^T ry in the factor's internal order
-  dev::gather(P(z.tmp_n), P(rxt), S.phat_d.p, n, b, st_);
+  CholEngine& ch = *S.chol;
+  // r^x = r~x + gamma Jc^T ry in the factor's internal order, A^{-1} r^x (kept for
+  // the recovery) and the Schur right-hand side Jc A^{-1} r^x - ry
   const double fl = 2.0 * S.nnz_jc;
-  const double by_t = spmv_bytes(n, m, S.nnz_jc, false, true, false);   // Jc^T x + y
-  const double by_j = spmv_bytes(m, n, S.nnz_jc, false, true, false);   // Jc x + y
-  timed(PK_SPMV, fl, by_t, b, [&] {
+  timed(PK_SPMV, fl, spmv_bytes(n, m, S.nnz_jc, false, true, false), bs, [&] {
     dev::spmv(n, S.jcth_rp.p, S.jcth_ci.p, nullptr, P(z.jcth_v), 0.0, P(z.gam), P(ysc), 1.0,
-              P(z.tmp_n), P(w.rxp), S.jcth_blk.p, S.jcth_nblk, b, st_);
+              P(rxt), P(w.rxp), S.jcth_blk.p, S.jcth_nblk, bs, st_, nullptr, nullptr, S.phat_d.p,
+              ch.sweep_fill(P(z.h0)));
   });
-  dev::copy(P(z.t1), P(w.rxp), n, b, st_);
-  S.chol->solve(P(z.t1), b);
-  dev::copy(P(z.h0), P(z.t1), n, b, st_);   // A^{-1} r^x, kept for the recovery
-  timed(PK_SPMV, fl, by_j, b, [&] {
-    dev::spmv(m, S.jch_rp.p, S.jch_ci.p, nullptr, P(z.jch_v), 1.0, nullptr, P(z.t1), -1.0,
-              P(ysc), P(w.schur), S.jch_blk.p, S.jch_nblk, b, st_);
+  ch.solve(P(w.rxp), P(z.h0), bs, true);
+  timed(PK_SPMV, fl, spmv_bytes(m, n, S.nnz_jc, false, true, false), bs, [&] {
+    dev::spmv(m, S.jch_rp.p, S.jch_ci.p, nullptr, P(z.jch_v), 1.0, nullptr, P(z.h0), -1.0,
+              P(ysc), P(w.schur), S.jch_blk.p, S.jch_nblk, bs, st_);
   });
 
   SchurOps ops;
-  ops.m = m;
-  ops.n = n;
   ops.jh_rp = S.jch_rp.p;
   ops.jh_ci = S.jch_ci.p;
   ops.jh_blk = S.jch_blk.p;
@@ -970,116 +959,113 @@ std::vector<CgResult> Solver::solve_phase(const Pass& w, int64_t rxt, int64_t ys
   ops.jh_v = P(z.jch_v);
   ops.jth_rp = S.jcth_rp.p;
   ops.jth_ci = S.jcth_ci.p;
-  ops.jth_blk = S.jcth_blk.p;
-  ops.jth_nblk = S.jcth_nblk;
   ops.jth_v = P(z.jcth_v);
-  ops.chol = S.chol.get();
+  ops.chol = &ch;
   ops.st = st_;
-  ops.t1 = P(z.t1);
-  ops.x = P(w.cx);
-  ops.r = P(z.cr);
-  ops.w = P(z.cw);
-  ops.p = P(z.cp);
-  ops.s = P(z.cs);
-  ops.sc = P(z.sc);
-  ops.part = P(z.part);
-  ops.live = S.flag(FL_LIVE);
-  ops.iters = S.flag(FL_CG_IT);
-  ops.status = S.flag(FL_CG_ST);
-  ops.gath = S.gath.p;
-  ops.tq = P(z.cq);
-  ops.tz = P(z.cz);
+  ops.v = dev::CgVecs{m,       n,       P(w.cx), P(z.cr), P(z.cw),   P(z.cp),    P(z.cs),
+                      P(z.t1), P(z.t2), P(z.cq), P(z.cz), P(z.sc),   P(z.part),  P(z.part2),
+                      S.jch_nblk};
+  ops.f = dev::CgFlags{S.flag(FL_LIVE), S.flag(FL_CG_IT), S.flag(FL_CG_ST)};
   ops.prof = &prof;
   ops.nnz = S.nnz_jc;
-  S.cg_host.ensure(4 * static_cast<size_t>(b.count));
-  ops.pinned = S.cg_host.p;
-  ops.defer = true;   // the results come back with the pass's residuals (cg_unpack)
-  if (x0) dev::copy(P(w.cx), P(z.in[IN_Y0]), m, b, st_);
-  else dev::fill(P(w.cx), 0.0, m, b, st_);
-  // the host looks at the live flags first after as many iterations as the
-  // last pass took (or every cg_check_every iterations when that is set)
-  const int chunk = opts.cg_check_every > 0 ? opts.cg_check_every : std::max(1, iters_hint);
-  const int chunk_next = opts.cg_check_every > 0 ? opts.cg_check_every : 1;
-  std::vector<CgResult> res =
-      schur_cg_run(ops, P(w.schur), opts.cg_tol, opts.cg_itmax, b, !x0, chunk, chunk_next);
-  if (after_cg) HIPCHK(hipEventRecord(after_cg, st_));
+  if (x0) dev::copy(P(w.cx), P(z.in[IN_Y0]), m, bs, st_);
+  cg_start(ops, P(w.schur), bs, !x0);
 
-  // recover_solution: dx = A^{-1} (r^x - Jc^T y) = A^{-1} r^x - A^{-1} Jc^T y, the
-  // second term carried along by the CG (no third solve)
-  dev::recover_xy(P(dx), P(z.h0), P(z.cz), S.ipos_d.p, P(z.max_d), n, P(dyc), P(w.cx), m, b,
-                  st_);
-  dev::recover_d(d, S.jd_rp.p, S.jd_ci.p, P(z.in[IN_JD]), S.has_jd ? 1 : 0, P(dx), P(ryd),
-                 P(z.in[IN_DS]), P(rs), P(dsv), P(dyd), b, st_);
-  return res;
-}
-
-// KKT residual of (dx, dsv, dyc, dyd) against the bound right-hand sides:
-// res[0..3] = squared norms of rows 1, 3, 2, 4; res[4..7] = squared norms of
-// rx, rs, ry, ryd.  rows: also keep the signed rows in e_x, e_y, e_s, e_d.
-void Solver::residual(int64_t dx, int64_t dsv, int64_t dyc, int64_t dyd, bool rows,
-                      const dev::Batch& b)
-{
-  Sym& S = *sym_;
-  const Slots& z = S.z;
-  const int n = S.n, m = S.m, d = S.d;
-  const double* in[IN_COUNT];
-  for (int j = 0; j < IN_COUNT; j++) in[j] = P(z.in[j]);
-  dev::resid_rows_n(n, S.h_rp.p, S.h_ci.p, in[IN_H], S.jct_rp.p, S.jct_ci.p, S.jct_map.p,
-                    in[IN_JC], S.has_jd ? S.jdt_rp.p : nullptr, S.jdt_ci.p, S.jdt_map.p, in[IN_JD],
-                    in[IN_RX], P(dx), P(dyc), P(dyd), P(z.sq_n), rows ? P(z.e_x) : nullptr, b, st_);
-  dev::resid_rows_m(m, S.jc_rp.p, S.jc_ci.p, in[IN_JC], in[IN_RY], P(dx), P(z.sq_m),
-                    rows ? P(z.e_y) : nullptr, b, st_);
-  dev::resid_rows_d(d, S.jd_rp.p, S.jd_ci.p, in[IN_JD], S.has_jd ? 1 : 0, in[IN_DS], in[IN_RS],
-                    in[IN_RYD], P(dx), P(dsv), P(dyd), P(z.sq_d2), P(z.sq_d4),
-                    rows ? P(z.e_s) : nullptr, rows ? P(z.e_d) : nullptr, b, st_);
-  // the eight squared norms in one launch pair (each the bits of its own dot)
-  dev::DotSet ds;
-  const double* sa[8] = {P(z.sq_n), P(z.sq_m), P(z.sq_d2), P(z.sq_d4),
-                         in[IN_RX], in[IN_RS], in[IN_RY], in[IN_RYD]};
-  const int sn[8] = {n, m, d, d, n, d, m, d};
-  for (int k = 0; k < 8; k++) {
-    ds.a[k] = sa[k];
-    ds.b[k] = k < 4 ? nullptr : sa[k];
-    ds.n[k] = sn[k];
+  dev::Recover rec{};
+  rec.n = n;
+  rec.m = m;
+  rec.d = d;
+  rec.has_jd = S.has_jd ? 1 : 0;
+  rec.h0 = P(z.h0);
+  rec.z = P(z.cz);
+  rec.x = P(w.cx);
+  rec.max_d = P(z.max_d);
+  rec.ipos = S.ipos_d.p;
+  rec.jd_rp = S.jd_rp.p;
+  rec.jd_ci = S.jd_ci.p;
+  rec.jd_v = P(z.in[IN_JD]);
+  rec.ryd = P(ryd);
+  rec.ds = P(z.in[IN_DS]);
+  rec.rs = P(rs);
+  rec.dx = P(out.dx);
+  rec.dsv = P(out.dsv);
+  rec.dyc = P(out.dyc);
+  rec.dyd = P(out.dyd);
+  if (base.dx >= 0) {
+    rec.base_dx = P(base.dx);
+    rec.base_dsv = P(base.dsv);
+    rec.base_dyc = P(base.dyc);
+    rec.base_dyd = P(base.dyd);
   }
-  ds.count = 8;
-  dev::dots(ds, P(z.part), P(z.res), b, st_);
-}
-
-std::vector<double> Solver::read_res(int count, std::vector<int>* zrow, std::vector<int>* piv)
-{
-  Sym& S = *sym_;
-  CholEngine& ch = *S.chol;
-  // one host round trip: the residual slots, the sweeps' error word and,
-  // with zrow / piv, each system's zero-row flag and first failing pivot,
-  // copied into pinned memory one after the other
-  const size_t nres = static_cast<size_t>(RES_SLOTS) * count;
-  const size_t words = 1 + (zrow ? count : 0) + (piv ? count : 0);
-  const size_t total = nres + (words + 1) / 2;
-  S.readback.ensure(total);
-  double* hres = S.readback.p;
-  int* hint = reinterpret_cast<int*>(S.readback.p + nres);
-  // everything gathered behind the residual slots on the device, one copy
-  dev::collect(S.gath.p, P(S.z.res), RES_SLOTS, dev::Batch{count, S.z.stride, nullptr}, st_);
-  dev::collect_ints(reinterpret_cast<int*>(S.gath.p + nres), ch.solve_error_dev(),
-                    zrow ? S.flag(FL_ZERO_ROW) : nullptr, piv ? ch.pivot_dev() : nullptr, count,
-                    st_);
-  HIPCHK(hipMemcpyAsync(hres, S.gath.p, sizeof(double) * total, hipMemcpyDeviceToHost, st_));
-  HIPCHK(hipStreamSynchronize(st_));
-  if (hint[0]) {
-    ch.clear_solve_error();
-    throw Error(HYKKT_E_STATE, "triangular-solve sweep exceeded its wait bound (results invalid)");
+  dev::Residual res{};
+  res.n = n;
+  res.m = m;
+  res.d = d;
+  res.has_jd = rec.has_jd;
+  res.h_rp = S.h_rp.p;
+  res.h_ci = S.h_ci.p;
+  res.ct_rp = S.jct_rp.p;
+  res.ct_ci = S.jct_ci.p;
+  res.ct_map = S.jct_map.p;
+  res.dt_rp = S.jdt_rp.p;
+  res.dt_ci = S.jdt_ci.p;
+  res.dt_map = S.jdt_map.p;
+  res.jc_rp = S.jc_rp.p;
+  res.jc_ci = S.jc_ci.p;
+  res.jd_rp = S.jd_rp.p;
+  res.jd_ci = S.jd_ci.p;
+  res.h_v = P(z.in[IN_H]);
+  res.jc_v = P(z.in[IN_JC]);
+  res.jd_v = P(z.in[IN_JD]);
+  res.ds = P(z.in[IN_DS]);
+  res.rx = P(z.in[IN_RX]);
+  res.rs = P(z.in[IN_RS]);
+  res.ry = P(z.in[IN_RY]);
+  res.ryd = P(z.in[IN_RYD]);
+  res.dx = rec.dx;
+  res.dsv = rec.dsv;
+  res.dyc = rec.dyc;
+  res.dyd = rec.dyd;
+  res.e_x = P(z.e_x);
+  res.e_s = P(z.e_s);
+  res.e_y = P(z.e_y);
+  res.e_d = P(z.e_d);
+  res.part = P(z.rpart);
+  dev::Finish fin{};
+  fin.out = S.fin.p;
+  fin.zero_row = S.flag(FL_ZERO_ROW);
+  fin.pivot = S.flag(FL_PIVOT);
+  fin.sweep_err = ch.solve_error_dev();
+  // algorithmic: the recovery's Jd dx; H, Jc twice and Jd twice of the residual
+  const double rec_by = spmv_bytes(d, n, S.nnz_jd, false, true, false);
+  const double res_fl = 2.0 * (S.nnz_h + 2.0 * S.nnz_jc + 2.0 * S.nnz_jd);
+  const double res_by = spmv_bytes(n, n, S.nnz_h, false, true, false) +
+                        spmv_bytes(n, m, S.nnz_jc, true, false, false) +
+                        spmv_bytes(n, d, S.nnz_jd, true, false, false) +
+                        spmv_bytes(m, n, S.nnz_jc, false, true, false) +
+                        spmv_bytes(d, n, S.nnz_jd, false, true, false);
+  int todo = opts.cg_check_every > 0 ? opts.cg_check_every : std::max(1, hint);
+  for (;;) {
+    cg_iterate(ops, todo, opts.cg_tol, opts.cg_itmax, bs);
+    timed(PK_SPMV, 2.0 * S.nnz_jd, rec_by, bs,
+          [&] { dev::recover(rec, bs, st_, first ? ev_[2] : nullptr); });
+    timed(PK_SPMV, res_fl, res_by, br, [&] { dev::residual(res, br, st_); });
+    dev::finish(fin, &res, ops.v, ops.k, opts.cg_tol, opts.cg_itmax, ops.f, br, st_,
+                first ? ev_[3] : nullptr);
+    HIPCHK(hipStreamSynchronize(st_));
+    bool live = false, bad = false;
+    for (int k = 0; k < br.count; k++) {
+      const double* h = S.fin.p + static_cast<size_t>(k) * dev::FIN_SLOTS;
+      live = live || h[dev::FIN_LIVE] != 0.0;
+      bad = bad || h[dev::FIN_SWEEP_ERR] != 0.0;
+    }
+    if (bad) {
+      ch.clear_solve_error();
+      throw Error(HYKKT_E_STATE, "triangular-solve sweep exceeded its wait bound (results invalid)");
+    }
+    if (!live || ops.k >= opts.cg_itmax) return;
+    todo = opts.cg_check_every > 0 ? opts.cg_check_every : 1;
   }
-  int at = 1;
-  if (zrow) {
-    zrow->assign(hint + at, hint + at + count);
-    at += count;
-  }
-  if (piv) {
-    piv->assign(hint + at, hint + at + count);
-    for (int& v : *piv) v = (v == INT_MAX) ? -1 : v;
-  }
-  return std::vector<double>(hres, hres + nres);
 }
 
 void Solver::get_solution(int k, double* dx, double* ds, double* dyc, double* dyd)

@@ -89,20 +89,14 @@ class Solver {
   struct Pass {
     int64_t rxp, schur, cx;
   };
-  std::vector<CgResult> solve_phase(const Pass& w, int64_t rxt, int64_t ysc, int64_t rs,
-                                    int64_t ryd, bool x0, int64_t dx, int64_t dsv, int64_t dyc,
-                                    int64_t dyd, const dev::Batch& b, hipEvent_t after_cg,
-                                    int iters_hint);
-  // Residual rows of (dx, dsv, dyc, dyd) (arena offsets) for the systems of
-  // b; rows: keep the signed rows for refinement.  Enqueues only; the eight
-  // squared norms of each system are at its `res` slot.
-  void residual(int64_t dx, int64_t dsv, int64_t dyc, int64_t dyd, bool rows, const dev::Batch& b);
-  // The res slots of `count` systems to the host in one round trip
-  // (synchronizes; throws if a sweep exceeded its wait bound); with zrow /
-  // piv, also each system's zero-row flag (INT_MAX: none) and first failing
-  // pivot (-1: none).
-  std::vector<double> read_res(int count, std::vector<int>* zrow = nullptr,
-                               std::vector<int>* piv = nullptr);
+  struct Solution {
+    int64_t dx, dsv, dyc, dyd;
+  };
+  // CG, recovery (into out, onto base unless its offsets are -1) and residual;
+  // synchronizes and leaves each system's FIN_SLOTS results in Sym::fin.
+  void solve_pass(const Pass& w, int64_t rxt, int64_t ysc, int64_t rs, int64_t ryd, bool x0,
+                  const Solution& out, const Solution& base, const dev::Batch& bs,
+                  const dev::Batch& br, int hint, bool first);
   double* P(int64_t off) const;   // system 0's address of an arena slot
   // Run the launch in fn bracketed for the profiler, charged with the work
   // of the b.count systems it covers.

@@ -43,9 +43,6 @@ __device__ __forceinline__ SysBufs sys_bufs(const CholDev& c, const SolveDev& sd
   return SysBufs{c.L + o, c.dinv + o, sd.ubuf + o, sd.bpart + o, in + o, out + o};
 }
 
-// Sentinel: a signalling-NaN payload no arithmetic result carries.
-constexpr uint64_t SENTINEL = 0x7ff4dead0badf00dull;
-
 __device__ __forceinline__ double xload(const double* p)
 {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -58,7 +55,7 @@ __device__ __forceinline__ void xstore(double* p, double v)
 
 __device__ __forceinline__ bool pending(double v)
 {
-  return __builtin_bit_cast(uint64_t, v) == SENTINEL;
+  return __builtin_bit_cast(uint64_t, v) == SWEEP_SENTINEL;
 }
 
 // The value at p once its producer has written it.  Gives up (sets *err,
