@@ -1,6 +1,8 @@
 // chol_engine.cpp -- host orchestration of the device multifrontal Cholesky.
 //
 // Numeric factorization, per tree level (leaves first):
+//   narrow supernodes (front_panel): children added, diagonal block, TRSM in one
+//   launch; the others:
 //   extend-add of the children's update matrices into the panels,
 //   blocked right-looking panel factorization in 128-column steps
 //     (factor + invert the diagonal block; TRSM of the rows below with the
@@ -8,8 +10,7 @@
 //      substitution with the inverses of the 16x16 diagonal blocks, the
 //      whole inverse formed after the level for the solves; MFMA update of
 //      the panel's trailing columns),
-//   U = -L21 L21^T on the matrix cores,
-//   extend-add of the children's update matrices into U.
+//   U = -L21 L21^T on the matrix cores plus the children's update matrices.
 // Solves: one forward and one backward sweep over the whole tree.
 #include <algorithm>
 #include <queue>
@@ -25,6 +26,7 @@ namespace {
 constexpr int NB = 128;   // panel step, MFMA tile edge, solve block
 constexpr int SR = 32;    // rows of a short tile
 constexpr int GMAX = 8;   // most steps one grouped trailing update can cover
+constexpr int U_SMALL_NC = 512;   // update matrices of at most so many columns take 64 x 64 tiles
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 }  // namespace
 
@@ -94,6 +96,7 @@ CholEngine::CholEngine(const Pattern& a, const CholOptions& opt, hipStream_t st)
   cd_.child_list = child_list_.p;
   cd_.sn_parent = sn_parent_.p;
   cd_.dinv_off = dinv_off_.p;
+  build_fronts();
   build_tasks();
   build_solve();
 }
@@ -186,6 +189,43 @@ CholEngine::~CholEngine()
   if (st2_) (void)hipStreamDestroy(st2_);
 }
 
+// The supernodes' records, and where each child's rows are among its parent's
+// front rows.
+void CholEngine::build_fronts()
+{
+  const int ns = pl_.ns;
+  std::vector<dev::ChildRec> rec(std::max<size_t>(pl_.child_list.size(), 1));
+  for (size_t t = 0; t < pl_.child_list.size(); t++) {
+    const int ch = pl_.child_list[t];
+    rec[t] = dev::ChildRec{pl_.u_off[ch], pl_.nr(ch), 0};
+  }
+  std::vector<dev::SnRec> sr(std::max(ns, 1));
+  std::vector<int> inv;
+  int64_t dinv = 0;
+  for (int s = 0; s < ns; s++) {
+    const int nc = pl_.nc(s), nr = pl_.nr(s), first = nc <= dev::FRONT_NC ? 0 : nc;
+    const int rows = nc + nr - first, nch = pl_.child_ptr[s + 1] - pl_.child_ptr[s];
+    const int64_t at = static_cast<int64_t>(inv.size()), off = at - first;
+    inv.resize(at + static_cast<int64_t>(nch) * rows, -1);
+    for (int t = 0; t < nch; t++) {
+      const int ch = pl_.child_list[pl_.child_ptr[s] + t];
+      for (int q = pl_.rows_ptr[ch]; q < pl_.rows_ptr[ch + 1]; q++)
+        if (pl_.rel[q] >= first)
+          inv[off + static_cast<int64_t>(t) * rows + pl_.rel[q]] = q - pl_.rows_ptr[ch];
+    }
+    sr[s] = dev::SnRec{pl_.sn_first[s], nc, nr, pl_.child_ptr[s], nch, rows, {0, 0},
+                       pl_.l_off[s], dinv, pl_.u_off[s], off};
+    dinv += static_cast<int64_t>(cdiv(nc, NB)) * NB * NB;
+  }
+  if (inv.empty()) inv.push_back(-1);
+  child_rec_.upload(rec);
+  sn_rec_.upload(sr);
+  inv_.upload(inv);
+  cd_.child_rec = child_rec_.p;
+  cd_.sn_rec = sn_rec_.p;
+  cd_.inv = inv_.p;
+}
+
 void CholEngine::build_tasks()
 {
   // Launch shapes (see Tuning), counted over the tcount_ systems a launch
@@ -206,6 +246,8 @@ void CholEngine::build_tasks()
   std::vector<int> eap, eacol, eacptr{0}, eacc, eaccol;
   std::vector<int> potrf, trsm_sn, trsm_tr, upd_sn, upd_tr, upd_tc;
   std::vector<int> syrk_sn, syrk_tr, syrk_tc, inv_sn, inv_step;
+  std::vector<int> fp_sn, fp_tile;
+  auto narrow = [&](int s) { return pl_.nc(s) <= dev::FRONT_NC; };
   struct Contrib {
     int t, c, r2;
   };
@@ -213,17 +255,18 @@ void CholEngine::build_tasks()
   for (int l = 0; l < nlev; l++) {
     Level& L = lv_[l];
     const int b0 = pl_.level_ptr[l], b1 = pl_.level_ptr[l + 1];
-    for (int part = 0; part < 2; part++) {
-      Launch& la = part == 0 ? L.ea_panel : L.ea_u;
+    {
+      Launch& la = L.ea_panel;
       la.off = static_cast<int>(eap.size());
       for (int q = b0; q < b1; q++) {
         const int p = pl_.level_sn[q], ncp = pl_.nc(p);
+        if (narrow(p)) continue;   // front_panel adds its children itself
         con.clear();
         for (int t = pl_.child_ptr[p]; t < pl_.child_ptr[p + 1]; t++) {
           const int c = pl_.child_list[t];
           for (int k = pl_.rows_ptr[c]; k < pl_.rows_ptr[c + 1]; k++) {
             int col = pl_.rel[k];
-            if ((part == 0) == (col < ncp)) con.push_back({col, c, k - pl_.rows_ptr[c]});
+            if (col < ncp) con.push_back({col, c, k - pl_.rows_ptr[c]});
           }
         }
         std::stable_sort(con.begin(), con.end(),
@@ -247,7 +290,24 @@ void CholEngine::build_tasks()
       la.cnt = static_cast<int>(eap.size()) - la.off;
     }
     int nsteps = 0;
-    for (int q = b0; q < b1; q++) nsteps = std::max(nsteps, cdiv(pl_.nc(pl_.level_sn[q]), NB));
+    for (int q = b0; q < b1; q++)
+      if (!narrow(pl_.level_sn[q]))
+        nsteps = std::max(nsteps, cdiv(pl_.nc(pl_.level_sn[q]), NB));
+    // narrow supernodes: one launch for the panel (its flops as a diagonal block's
+    // and a TRSM's; the children's entries and the panel read, the panel written)
+    L.front.off = static_cast<int>(fp_sn.size());
+    for (int q = b0; q < b1; q++) {
+      const int s = pl_.level_sn[q];
+      if (!narrow(s)) continue;
+      const double nc = pl_.nc(s), nr = pl_.nr(s);
+      L.front.flops += nc * nc * nc / 3 + nc * nc / 2 + nc / 6 + nr * nc * nc;
+      L.front.bytes += 16.0 * (nc * (nc + 1) / 2 + nr * nc);
+      for (int t = 0; t < std::max(1, cdiv(pl_.nr(s), NB)); t++) {
+        fp_sn.push_back(s);
+        fp_tile.push_back(t);
+      }
+    }
+    L.front.cnt = static_cast<int>(fp_sn.size()) - L.front.off;
     L.potrf.resize(nsteps);
     L.trsm.resize(nsteps);
     L.upd_next.resize(nsteps);
@@ -267,7 +327,7 @@ void CholEngine::build_tasks()
         for (int q = b0; q < b1; q++) {
           const int s = pl_.level_sn[q];
           const int nc = pl_.nc(s), f = nc + pl_.nr(s), k0 = j * NB;
-          if (k0 >= nc) continue;
+          if (k0 >= nc || narrow(s)) continue;
           const int cs = k0 + std::min(g * NB, nc - k0);
           const int rt = cdiv(f - cs, NB), ct = cdiv(nc - cs, NB);
           for (int tc = g; tc < ct; tc++) rest += rt - tc;
@@ -289,7 +349,7 @@ void CholEngine::build_tasks()
       for (int q = b0; q < b1; q++) {
         const int s = pl_.level_sn[q];
         const int nc = pl_.nc(s), f = nc + pl_.nr(s), k0 = j * NB;
-        if (k0 < nc) full_tiles += cdiv(f - (k0 + std::min(NB, nc - k0)), NB);
+        if (k0 < nc && !narrow(s)) full_tiles += cdiv(f - (k0 + std::min(NB, nc - k0)), NB);
       }
       const bool shrt = full_tiles * tc <= tun_.short_max;
       const int rows_unit = shrt ? SR : NB;
@@ -299,7 +359,7 @@ void CholEngine::build_tasks()
         const int s = pl_.level_sn[q];
         const int nc = pl_.nc(s), f = nc + pl_.nr(s);
         const int k0 = j * NB;
-        if (k0 >= nc) continue;
+        if (k0 >= nc || narrow(s)) continue;
         const int b = std::min(NB, nc - k0);
         potrf.push_back(s);
         L.potrf[j].maxb = std::max(L.potrf[j].maxb, b);
@@ -353,7 +413,7 @@ void CholEngine::build_tasks()
         for (int q = b0; q < b1; q++) {
           const int s = pl_.level_sn[q];
           const int nc = pl_.nc(s), f = nc + pl_.nr(s), k0 = j * NB;
-          if (k0 >= nc) continue;
+          if (k0 >= nc || narrow(s)) continue;
           if (G > 1 && !last && part == 1) continue;   // deferred to the group's update
           if (G > 1 && last) {
             // columns after the group's G blocks, K = all of them: the next G
@@ -389,12 +449,27 @@ void CholEngine::build_tasks()
         la.cnt = static_cast<int>(upd_sn.size()) - la.off;
       }
     }
+    // update matrices: tiles of 64 x 64, whose children's entries have four waves a
+    // SIMD in flight, unless K is long enough for the operand loads that a 128 x 128
+    // tile saves (10,000 buses, K = 404: 424 us against 510; K = 1,468: 1558 against
+    // 1512; levels of at most 32 columns: 14-250 us against 27-530)
+    L.small_u = true;
+    for (int q = b0; q < b1; q++)
+      if (pl_.nc(pl_.level_sn[q]) > U_SMALL_NC) L.small_u = false;
+    const int ut = L.small_u ? NB / 2 : NB;
     L.syrk.off = static_cast<int>(syrk_sn.size());
     for (int q = b0; q < b1; q++) {
-      const int s = pl_.level_sn[q], nt = cdiv(pl_.nr(s), NB);
+      const int s = pl_.level_sn[q], nt = cdiv(pl_.nr(s), ut);
       const double nr = pl_.nr(s), nc = pl_.nc(s), pairs = nr * (nr + 1) / 2;
       L.syrk.flops += 2.0 * nc * pairs;
       L.syrk.bytes += 8.0 * (nr * nc + pairs);
+      for (int t = pl_.child_ptr[s]; t < pl_.child_ptr[s + 1]; t++) {
+        const int ch = pl_.child_list[t];
+        double below = 0;   // the child's rows below s's columns
+        for (int k = pl_.rows_ptr[ch]; k < pl_.rows_ptr[ch + 1]; k++) below += pl_.rel[k] >= pl_.nc(s);
+        L.syrk.flops += below * (below + 1) / 2;
+        L.syrk.bytes += 8.0 * below * (below + 1) / 2;
+      }
       for (int tc = 0; tc < nt; tc++)
         for (int tr = tc; tr < nt; tr++) {
           syrk_sn.push_back(s);
@@ -410,7 +485,7 @@ void CholEngine::build_tasks()
       if (L.potrf[j].maxb <= 64) continue;
       for (int q = b0; q < b1; q++) {
         const int s = pl_.level_sn[q], nc = pl_.nc(s);
-        if (j * NB >= nc) continue;
+        if (j * NB >= nc || narrow(s)) continue;
         const double db = std::min(NB, nc - j * NB);
         inv_sn.push_back(s);
         inv_step.push_back(j);
@@ -429,6 +504,8 @@ void CholEngine::build_tasks()
   up(t_ea_cptr_, eacptr);
   up(t_ea_cc_, eacc);
   up(t_ea_ccol_, eaccol);
+  up(t_fp_sn_, fp_sn);
+  up(t_fp_tile_, fp_tile);
   up(t_potrf_, potrf);
   up(t_trsm_sn_, trsm_sn);
   up(t_trsm_tr_, trsm_tr);
@@ -604,6 +681,10 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
   };
   auto timed = [&](int kind, const Launch& la, auto&& launch) { timed_on(st_, kind, la, launch); };
   for (const Level& L : lv_) {
+    timed(PK_POTRF, L.front, [&] {
+      dev::front_panel(cd_, L.front.cnt, t_fp_sn_.p + L.front.off, t_fp_tile_.p + L.front.off, b,
+                       st_);
+    });
     timed(PK_EXTEND_ADD, L.ea_panel, [&] {
       dev::extend_add(cd_, L.ea_panel.cnt, t_ea_p_.p + L.ea_panel.off,
                       t_ea_col_.p + L.ea_panel.off, t_ea_cptr_.p + L.ea_panel.off, t_ea_cc_.p,
@@ -678,12 +759,8 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
       dev::inv_blocks(cd_, L.inv.cnt, t_inv_sn_.p + L.inv.off, t_inv_step_.p + L.inv.off, b, st_);
     });
     timed(PK_DENSE_NT, L.syrk, [&] {
-      dev::dense_nt(cd_, L.syrk.cnt, t_syrk_sn_.p + L.syrk.off, t_syrk_tr_.p + L.syrk.off,
-                    t_syrk_tc_.p + L.syrk.off, 1, 0, b, st_);
-    });
-    timed(PK_EXTEND_ADD, L.ea_u, [&] {
-      dev::extend_add(cd_, L.ea_u.cnt, t_ea_p_.p + L.ea_u.off, t_ea_col_.p + L.ea_u.off,
-                      t_ea_cptr_.p + L.ea_u.off, t_ea_cc_.p, t_ea_ccol_.p, b, st_);
+      dev::update_matrices(cd_, L.syrk.cnt, t_syrk_sn_.p + L.syrk.off, t_syrk_tr_.p + L.syrk.off,
+                           t_syrk_tc_.p + L.syrk.off, L.small_u, b, st_);
     });
   }
 }

@@ -179,12 +179,14 @@ class CholEngine {
     double flops = 0.0, bytes = 0.0;   // algorithmic, for the profiler
   };
   struct Level {
-    Launch ea_panel, ea_u, syrk, inv;
+    Launch front, ea_panel, syrk, inv;
+    bool small_u = false;   // update matrices in 64 x 64 tiles
     std::vector<Launch> potrf, trsm, upd_next, upd_rest;
     // per step: its position in its group of consecutive steps and the
     // group's size (1: the step updates after its own block; see build_tasks)
     std::vector<int> gpos, gsize;
   };
+  void build_fronts();
   void build_tasks();
   void build_solve();
   void pick_second_stream();
@@ -217,6 +219,10 @@ class CholEngine {
   DevBuf<int> t_potrf_, t_trsm_sn_, t_trsm_tr_, t_upd_sn_, t_upd_tr_, t_upd_tc_;
   DevBuf<int> t_syrk_sn_, t_syrk_tr_, t_syrk_tc_;
   DevBuf<int> t_inv_sn_, t_inv_step_;
+  DevBuf<int> t_fp_sn_, t_fp_tile_;
+  DevBuf<dev::ChildRec> child_rec_;
+  DevBuf<dev::SnRec> sn_rec_;
+  DevBuf<int> inv_;
   int n_cu_ = 1;   // compute units: persistent-launch width
   // solve items
   DevBuf<int> fwd_items_, bwd_items_, pull_ptr_, pull_src_, flags_;

@@ -255,11 +255,31 @@ size_t noalloc_scratch_bytes();
 void* noalloc_scratch();
 
 // ---------------------------------------------------------------- Cholesky
-// Offset of (r, c), r >= c, in an n x n lower triangle packed by columns.
-__host__ __device__ inline int64_t packed_lower(int64_t r, int64_t c, int64_t n)
+// Offset of (r, c), r >= c, in an n x n lower triangle packed by columns: c n - c
+// (c + 1) / 2 + r, with one 32 x 32 bit product.
+__host__ __device__ inline int64_t packed_lower(int r, int c, int n)
 {
-  return c * n - c * (c + 1) / 2 + r;
+  const uint32_t uc = static_cast<uint32_t>(c), m = 2u * static_cast<uint32_t>(n) - uc - 1u;
+  return static_cast<int64_t>((static_cast<uint64_t>(uc) * m) >> 1) + r;
 }
+
+// A child of a supernode, in child-list order: its update matrix and that one's size.
+struct ChildRec {
+  int64_t u_off;
+  int nr, pad;
+};
+// What a workgroup needs to know of a supernode.  Child t's row of its update matrix
+// at front row r, or -1: inv[inv_off + t * inv_rows + r] (the rows below the
+// supernode's columns; for at most FRONT_NC columns those, too).
+struct SnRec {
+  int a, nc, nr;      // first column, columns, rows below them
+  int child0, nch;    // its children in child_rec
+  int inv_rows;
+  int pad[2];
+  int64_t l_off, dinv_off, u_off, inv_off;
+};
+// Widest supernode that front_panel() takes.
+constexpr int FRONT_NC = 32;
 
 // The factor storage of system 0 (system k's at + k*vs, vs of the Batch).
 struct CholDev {
@@ -273,6 +293,9 @@ struct CholDev {
   const int* child_ptr;
   const int* child_list;
   const int* sn_parent;
+  const ChildRec* child_rec;   // by position in child_list
+  const SnRec* sn_rec;
+  const int* inv;              // see SnRec
   double* L;
   double* U;
   int* pivot;               // one int per system: first failing pivot (min), INT_MAX if none
@@ -304,14 +327,23 @@ void inv_blocks(const CholDev& c, int ntasks, const int* task_sn, const int* tas
                 const Batch& b, hipStream_t st);
 
 // MFMA update tiles over (supernode, tile row, tile col) tasks.  mode 0: trailing
-// panel update after block `step`; mode 1: U = -L21 L21^T; mode m >= 3: as mode 0
-// after blocks `step` .. `step`+m-2 (K = (m-1) blocks).  Tiles of 128 x 128, or
-// of 32 rows x 128 columns (short_rows; modes 0 and >= 3).  done: optional event
+// panel update after block `step`; mode m >= 3: after blocks `step` .. `step`+m-2
+// (K = (m-1) blocks).  Tiles of 128 x 128, or of 32 rows x 128 columns
+// (short_rows).  done: optional event
 // recorded by the launch's own completion.  alone: 128 x 128 tiles keep off a
 // compute unit that factors a 128-wide diagonal block.
 void dense_nt(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr,
               const int* task_tc, int mode, int step, const Batch& b, hipStream_t st,
               bool short_rows = false, hipEvent_t done = nullptr, bool alone = false);
+// The update matrices U = -L21 L21^T + the children's, tasks as above with tiles of
+// 128 x 128 (small: 64 x 64) entries of U.
+void update_matrices(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr,
+                     const int* task_tc, bool small, const Batch& b, hipStream_t st);
+// Supernodes of at most FRONT_NC columns: children's entries added to the panel,
+// diagonal block factored and inverted, L21 formed; tasks (supernode, tile of 128
+// rows below the columns; a supernode without such rows: one task).
+void front_panel(const CholDev& c, int ntasks, const int* task_sn, const int* task_tile,
+                 const Batch& b, hipStream_t st);
 // TRSM of the rows below blocks of at most 64 columns with their whole inverses,
 // in place (tasks as trsm()'s).
 void trsm_inv(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr, int step,

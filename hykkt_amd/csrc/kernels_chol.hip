@@ -34,7 +34,8 @@ __device__ __forceinline__ SnInfo sninfo(const CholDev& c, double* L, int s)
 }
 
 // ----------------------------------------------------------------- extend-add
-// One workgroup per parent front column and system.  Children are added one
+// One workgroup per column of a parent's panel and system (its update matrix takes
+// its children's in k_dense_nt).  Children are added one
 // after the other (fixed order => deterministic sums); within one child the
 // relative index map is injective.
 __global__ void __launch_bounds__(256) k_extend_add(CholDev c, const int* __restrict__ task_p,
@@ -46,19 +47,11 @@ __global__ void __launch_bounds__(256) k_extend_add(CholDev c, const int* __rest
   const int sy = batch_sys(b);
   if (sy < 0) return;
   double* const L = batch_at(c.L, sy, b);
-  double* const U = batch_at(c.U, sy, b);
+  const double* const U = batch_at(c.U, sy, b);
   const int t = blockIdx.x;
   const int p = task_p[t], col = task_col[t];
   const SnInfo ip = sninfo(c, L, p);
-  double* base;
-  int shift;
-  if (col < ip.nc) {
-    base = ip.Ls + static_cast<int64_t>(col) * ip.f;
-    shift = 0;
-  } else {
-    base = U + c.u_off[p] + packed_lower(0, col - ip.nc, ip.nr);   // rows >= col only
-    shift = -ip.nc;
-  }
+  double* const base = ip.Ls + static_cast<int64_t>(col) * ip.f;
   for (int k = cptr[t]; k < cptr[t + 1]; k++) {
     const int ch = cc[k], r2 = ccol[k];
     const int nrc = c.rows_ptr[ch + 1] - c.rows_ptr[ch];
@@ -74,7 +67,7 @@ __global__ void __launch_bounds__(256) k_extend_add(CholDev c, const int* __rest
       double sv[UNR], bv[UNR];
 #pragma unroll
       for (int u = 0; u < UNR; u++) {
-        ri[u] = relc[r1 + u * BS] + shift;
+        ri[u] = relc[r1 + u * BS];
         sv[u] = src[r1 + u * BS];
       }
 #pragma unroll
@@ -82,7 +75,7 @@ __global__ void __launch_bounds__(256) k_extend_add(CholDev c, const int* __rest
 #pragma unroll
       for (int u = 0; u < UNR; u++) base[ri[u]] = bv[u] + sv[u];
     }
-    for (; r1 < nrc; r1 += BS) base[relc[r1] + shift] += src[r1];
+    for (; r1 < nrc; r1 += BS) base[relc[r1]] += src[r1];
     __syncthreads();
   }
 }

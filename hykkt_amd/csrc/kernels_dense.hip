@@ -14,6 +14,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "batch_dev.hpp"
 #include "kernels.hpp"
@@ -188,8 +189,53 @@ __device__ __forceinline__ void frag_load(double (&v)[CNT], rsrc_t r, uint32_t v
   }
 }
 
+__device__ __forceinline__ int rl32(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
+__device__ __forceinline__ int64_t rl64(int v, int lane)
+{
+  const uint32_t lo = rl32(v, lane), hi = rl32(v, lane + 1);
+  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// Supernode s's record, wave-uniform: one load, a word per lane, instead of one
+// per field, each waited for.
+struct Sn {
+  int a, nc, nr, f, nch, stride;
+  int64_t l_off, dinv_off, u_off;
+  const ChildRec* rec;   // of its first child
+  const int* inv;        // of child 0, indexed by front row; child t's t * stride further
+};
+
+__device__ __forceinline__ Sn load_sn(const CholDev& c, int s, int lane)
+{
+  static_assert(sizeof(SnRec) == 64, "sixteen words");
+  const int w = reinterpret_cast<const int*>(c.sn_rec + s)[lane & 15];
+  Sn r;
+  r.a = rl32(w, 0);
+  r.nc = rl32(w, 1);
+  r.nr = rl32(w, 2);
+  r.f = r.nc + r.nr;
+  r.rec = c.child_rec + rl32(w, 3);
+  r.nch = rl32(w, 4);
+  r.stride = rl32(w, 5);
+  r.l_off = rl64(w, 8);
+  r.dinv_off = rl64(w, 10);
+  r.u_off = rl64(w, 12);
+  r.inv = c.inv + rl64(w, 14);
+  return r;
+}
+
+// The records of CG children from the t0-th on (past the last: the last one's),
+// one load: child g's in lanes 4 g .. 4 g + 3.
+template <int CG>
+__device__ __forceinline__ int child_words(const Sn& r, int t0, int lane)
+{
+  static_assert(sizeof(ChildRec) == 16 && CG <= 16, "four words a child");
+  const int g = min(lane >> 2, CG - 1);
+  return reinterpret_cast<const int*>(r.rec + min(t0 + g, r.nch - 1))[lane & 3];
+}
+
 // mode 0: trailing panel update after block `step`   C = C - A A^T (K = block)
-// mode 1: update matrix U = -L21 L21^T                 (K = nc, U overwritten)
+// mode 1: update matrix U = -L21 L21^T + children      (K = nc, U written)
 // mode m >= 3: as mode 0 after blocks `step` .. `step`+m-2 (K = m-1 blocks)
 //
 // Each wave holds a (16 IM) x (16 JN) block of C in accumulators and reads its
@@ -204,31 +250,39 @@ __device__ __forceinline__ void frag_load(double (&v)[CNT], rsrc_t r, uint32_t v
 // 49); at small K the C traffic takes over.  D = 2 leaves the 128 x 128 tile
 // at two waves per SIMD with registers over for a diagonal block.
 //
+// An update matrix takes its children's as the tile is finished, read once and
+// straight into the accumulators: a pass of its own over U, read and written again
+// per child, made the two 3190 us of a pass at 10,000 buses, now 2806 (eight systems
+// at 5,000: 2245 for the second pass alone, now 2319 in all).
+//
 // Every C entry starts from its old value (modes 0, >= 3) or 0 and takes the
 // MFMAs of K in ascending order, whatever the tile shape.  Rows and columns of
 // a tile past the panel compute values that are not stored (their loads stay
 // in the panel, or return 0 past its end); K steps past K read 0 for both
 // operands.
 //
-// Four waves, WN of them along the columns, on TM rows; a tile's 128 columns are
+// WN waves along the columns, TM / (16 IM) along the rows, on TM rows; a tile's 128 columns are
 // split over gridDim.z workgroups of 16 JN WN columns.  System blockIdx.y.
-template <int TM, int IM, int JN, int WN, int D>
-__global__ void __launch_bounds__(256, 2)
+// U: mode 1 (a kernel of its own, so that the others keep their registers).
+template <bool U, int TM, int IM, int JN, int WN, int D>
+__global__ void __launch_bounds__(TM / IM * WN * 4, TM / IM * WN / 32)
     k_dense_nt(CholDev c, const int* __restrict__ tsn, const int* __restrict__ ttr,
                const int* __restrict__ ttc, int mode, int step, Batch bt)
 {
   constexpr int QM = 16 * IM, QN = 16 * JN, TN = QN * WN;
-  static_assert(TM / QM * WN == 4, "four waves");
+  // mode 1: children whose indices, column quarters whose entries are in flight
+  constexpr int CG = IM * JN > 4 ? 1 : 4, VG = IM * JN > 4 ? 2 : 4;
+  static_assert(TM / QM * WN == 4 || TM / QM * WN == 8, "four or eight waves");
   // the 32-row launches are the factorization's critical chain: their waves
   // take issue priority over the trailing updates they share SIMDs with
   if constexpr (TM == 32) __builtin_amdgcn_s_setprio(3);
   const int sy = batch_sys(bt);
   if (sy < 0) return;
+  const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
   const int s = uni(tsn[blockIdx.x]), tr = uni(ttr[blockIdx.x]), tc = uni(ttc[blockIdx.x]);
-  const int nc = uni(c.sn_first[s + 1] - c.sn_first[s]);
-  const int nr = uni(c.rows_ptr[s + 1] - c.rows_ptr[s]);
-  const int f = nc + nr;
-  const double* Ls = batch_at(c.L, sy, bt) + uni64(c.l_off[s]);
+  const Sn sn = load_sn(c, s, lane);
+  const int nc = sn.nc, nr = sn.nr, f = sn.f;
+  const double* Ls = batch_at(c.L, sy, bt) + sn.l_off;
   // end of the views: the panel's last entry and the one after it (the second
   // row of a pair; the storage goes on there)
   const double* panel_end = Ls + static_cast<int64_t>(f) * nc + 1;
@@ -236,9 +290,9 @@ __global__ void __launch_bounds__(256, 2)
   // this workgroup's rows and columns of the front (R0, C0), the first column
   // of the K range and K; M, N: valid rows and columns
   int R0, C0, ka, K, M, N;
-  if (mode == 1) {
+  if (U) {
     R0 = nc + tr * TM;
-    C0 = nc + tc * BT + zc;
+    C0 = nc + tc * TN;
     ka = 0;
     K = nc;
     M = min(TM, f - R0);
@@ -252,7 +306,6 @@ __global__ void __launch_bounds__(256, 2)
     N = min(TN, nc - C0);
   }
   if (M <= 0 || N <= 0) return;
-  const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
   const int m16 = lane & 15, q4 = lane >> 4;
   const int wr = (wave / WN) * QM, wc = (wave % WN) * QN;
   const uint32_t f8 = static_cast<uint32_t>(f) * 8u;
@@ -277,7 +330,10 @@ __global__ void __launch_bounds__(256, 2)
   const double* Cp = Ls + static_cast<int64_t>(C0 + wc) * f + R0 + wr;
   const uint32_t vc = grow16<JN>(0, q4) * f8 + grow16<IM>(0, m16) * 8u;
   auto coff = [&](int j, int v) { return static_cast<uint32_t>(grow16<JN>(j, 4 * v)) * f8; };
-  if (mode != 1) {
+  // (the test of mode keeps this a block of its own, which the compiler does not
+  // interleave with its neighbours: their addresses beside the accumulators would
+  // spill)
+  if (!U && mode != 1) {
     const rsrc_t rc = view(Cp, 8 * (panel_end - Cp));
 #pragma unroll
     for (int j = 0; j < JN; j++)
@@ -319,24 +375,86 @@ __global__ void __launch_bounds__(256, 2)
     }
   }
 
-  if (mode == 1) {
+  // the lane's place anew, so that no address of the stores is formed before the
+  // loop and held in registers through it
+  int lm = m16, lq = q4;
+  asm volatile("" : "+v"(lm), "+v"(lq));
+  if constexpr (U) {
     // U packed by columns, entries on or below its diagonal
-    double* U = batch_at(c.U, sy, bt) + uni64(c.u_off[s]);
+    double* Us = batch_at(c.U, sy, bt) + sn.u_off;
     const int gr0 = R0 - nc + wr, gc0 = C0 - nc + wc;
+    // the children's update matrices, in the order of the child list: an entry
+    // (r, c) of the front takes child t's entry (inv(t, r), inv(t, c)) where it has
+    // both; the index loads of CG children are in flight together
+    const double* Ub = batch_at(c.U, sy, bt);
+    const int rlim = nr - gr0, clim = nr - gc0;   // rows, columns of the wave's block
+    for (int t0 = 0; t0 < sn.nch; t0 += CG) {
+      const int cw = child_words<CG>(sn, t0, lane);
+      int ia[CG][IM], ib[CG][JN][4];
+#pragma unroll
+      for (int g = 0; g < CG; g++) {
+        const bool in = t0 + g < sn.nch;
+        const int* iv = sn.inv + static_cast<int64_t>(min(t0 + g, sn.nch - 1)) * sn.stride + nc;
+#pragma unroll
+        for (int i = 0; i < IM; i++) {
+          const int r = grow16<IM>(i, lm);
+          const int x = iv[gr0 + min(r, max(rlim - 1, -gr0))];
+          ia[g][i] = in && r < rlim ? x : -1;
+        }
+#pragma unroll
+        for (int j = 0; j < JN; j++)
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            const int cl = grow16<JN>(j, 4 * v) + grow16<JN>(0, lq);
+            const int x = iv[gc0 + min(cl, max(clim - 1, -gc0))];
+            ib[g][j][v] = cl < clim ? x : 0x7fffffff;   // past every row
+            if (ib[g][j][v] < 0) ib[g][j][v] = 0x7fffffff;
+          }
+      }
+#pragma unroll
+      for (int g = 0; g < CG; g++) {
+        bool any = false;
+#pragma unroll
+        for (int i = 0; i < IM; i++) any = any || ia[g][i] >= 0;
+        if (!__builtin_amdgcn_ballot_w64(any)) continue;
+        const int n = rl32(cw, 4 * g + 2);
+        const double* uc = Ub + rl64(cw, 4 * g);
+#pragma unroll
+        for (int j = 0; j < JN; j++)
+#pragma unroll
+          for (int v0 = 0; v0 < 4; v0 += VG) {
+            double x[VG][IM];
+#pragma unroll
+            for (int v = 0; v < VG; v++) {
+              const int b = ib[g][j][v0 + v];
+              const double* col = uc + packed_lower(0, b < n ? b : 0, n);
+              // on or below the child's diagonal; the others read the column's first
+#pragma unroll
+              for (int i = 0; i < IM; i++) x[v][i] = col[ia[g][i] >= b ? ia[g][i] : (b < n ? b : 0)];
+            }
+#pragma unroll
+            for (int v = 0; v < VG; v++)
+#pragma unroll
+              for (int i = 0; i < IM; i++)
+                acc[i][j][v0 + v] = ia[g][i] >= ib[g][j][v0 + v] ? acc[i][j][v0 + v] + x[v][i]
+                                                                 : acc[i][j][v0 + v];
+          }
+      }
+    }
     const bool whole = M == TM && N == TN && gr0 >= gc0 + QN;   // no entry to leave out
 #pragma unroll
     for (int j = 0; j < JN; j++)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        const int cl = grow16<JN>(j, 4 * v) + grow16<JN>(0, q4), gc = gc0 + cl;
-        double* col = U + packed_lower(gr0, gc, nr);   // row gr0 of column gc
+        const int cl = grow16<JN>(j, 4 * v) + grow16<JN>(0, lq), gc = gc0 + cl;
+        double* col = Us + packed_lower(gr0, gc, nr);   // row gr0 of column gc
         if (whole) {
 #pragma unroll
-          for (int i = 0; i < IM; i++) col[grow16<IM>(i, m16)] = acc[i][j][v];
+          for (int i = 0; i < IM; i++) col[grow16<IM>(i, lm)] = acc[i][j][v];
         } else {
 #pragma unroll
           for (int i = 0; i < IM; i++) {
-            const int r = grow16<IM>(i, m16);
+            const int r = grow16<IM>(i, lm);
             if (wr + r < M && wc + cl < N && gr0 + r >= gc) col[r] = acc[i][j][v];
           }
         }
@@ -349,7 +467,7 @@ __global__ void __launch_bounds__(256, 2)
   for (int j = 0; j < JN; j++)
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      const int cl = grow16<JN>(j, 4 * v) + grow16<JN>(0, q4);
+      const int cl = grow16<JN>(j, 4 * v) + grow16<JN>(0, lq);
       double* col = Cw + static_cast<int64_t>(cl) * f;
       if (whole) {
         // pairs of rows: 16-byte stores (8-byte aligned, as the panel is)
@@ -357,15 +475,15 @@ __global__ void __launch_bounds__(256, 2)
           typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 #pragma unroll
           for (int i = 0; i < IM; i += 2)
-            *reinterpret_cast<d2u*>(col + grow16<IM>(i, m16)) = d2u{acc[i][j][v], acc[i + 1][j][v]};
+            *reinterpret_cast<d2u*>(col + grow16<IM>(i, lm)) = d2u{acc[i][j][v], acc[i + 1][j][v]};
         } else {
 #pragma unroll
-          for (int i = 0; i < IM; i++) col[grow16<IM>(i, m16)] = acc[i][j][v];
+          for (int i = 0; i < IM; i++) col[grow16<IM>(i, lm)] = acc[i][j][v];
         }
       } else {
 #pragma unroll
         for (int i = 0; i < IM; i++) {
-          const int r = grow16<IM>(i, m16);
+          const int r = grow16<IM>(i, lm);
           if (wr + r < M && wc + cl < N) col[r] = acc[i][j][v];
         }
       }
@@ -635,50 +753,15 @@ __device__ __forceinline__ void panel_tiles(double (*P)[BK + 1], int kb0, int np
   }
 }
 
-// Diagonal block `step` of supernode s, by one workgroup of 256 threads with
-// smem >= potrf_smem<BK>().  BK: padded block edge (32, 64 or 128) >= b.
-// FULL: the whole inverse; otherwise only the inverses of its 16x16 diagonal
-// blocks (the blocked TRSM's), the rest formed after the level (k_inv_blocks).
-template <int BK, bool FULL>
-__device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double* dinv, int* pivot,
-                                            int s, int step, double* smem)
+// The Cholesky factor of the BK x BK block in P's lower part (b columns of the
+// matrix, col0 the first, then the identity), in place; rd: the reciprocals of its
+// diagonal; *bad (shared, INT_MAX before): the first column whose pivot fails.
+// All threads of the workgroup, past a barrier at the end.
+template <int BK>
+__device__ __forceinline__ void potrf_factor(double (*P)[BK + 1], double* rd, int b, int col0,
+                                             double pivot_tol, int* bad, int tid, int lane,
+                                             int wave, int panels = BK / PW)
 {
-  constexpr int NPN = BK / PW;   // panels
-  const SnInfo si = sninfo(c, L, s);
-  const int k0 = step * BT;
-  if (k0 >= si.nc) return;
-  const int b = min(BK, si.nc - k0);
-  double (*P)[BK + 1] = reinterpret_cast<double (*)[BK + 1]>(smem);
-  double* rd = smem + BK * (BK + 1);   // 1 / L(r, r)
-  __shared__ int bad;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar tile bookkeeping
-  double* D = si.Ls + static_cast<int64_t>(k0) * si.f + k0;
-  // load the lower triangle (padded with the identity past b), all of a
-  // thread's entries in flight at once.  Every lane loads (entries past b or
-  // past the triangle read D[0] and are replaced), so the loads are not split
-  // by branches that would wait on each other.
-  constexpr int NL = BK * (BK + 1) / 2, PER = (NL + 255) / 256;
-  {
-    double v[PER];
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-      int r, col;
-      lower_entry<BK>(min(tid + u * 256, NL - 1), r, col);
-      const bool in = r < b;
-      const double t = D[in ? r + static_cast<int64_t>(col) * si.f : 0];
-      v[u] = in ? t : (r == col ? 1.0 : 0.0);
-    }
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-      int r, col;
-      lower_entry<BK>(min(tid + u * 256, NL - 1), r, col);
-      if (tid + u * 256 < NL) P[r][col] = v[u];
-    }
-  }
-  if (tid == 0) bad = INT_MAX;
-  __syncthreads();
-
   // ---- blocked Cholesky, one 16-column panel at a time ----
   // Each factoring wave takes the panel's 16 x 16 diagonal block in lanes
   // 0..15 (lane l holds row kb + l; every such wave the same) and 48 of the
@@ -696,7 +779,7 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
     const bool dg = lane < PW;
     const int prow_off = dg ? lane : PW + 48 * wave + (lane - PW);   // row - kb
 #pragma unroll 1
-    for (int p = 0; p < NPN; p++) {
+    for (int p = 0; p < panels; p++) {
       const int kb = p * PW;
       const int nf = max(1, (BK - kb - PW + 47) / 48);   // factoring waves
       if (wave < nf) {
@@ -744,11 +827,11 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
           // system is reported and kept out of the solve).  The first
           // failing column of the first failing panel is kept.
           const double lkk = P[kb + (lane & 15)][kb + (lane & 15)];
-          const uint64_t f = __builtin_amdgcn_ballot_w64(dg && kb + lane < b && !(lkk > c.pivot_tol));
-          if (f != 0 && tid == 0 && bad == INT_MAX) bad = si.a + k0 + kb + __builtin_ctzll(f);
+          const uint64_t f = __builtin_amdgcn_ballot_w64(dg && kb + lane < b && !(lkk > pivot_tol));
+          if (f != 0 && tid == 0 && *bad == INT_MAX) *bad = col0 + kb + __builtin_ctzll(f);
           if (dg) rd[kb + lane] = myinv;
         }
-      } else if (p > 0 && kb + PW < BK) {
+      } else if (p > 0 && p + 1 < panels) {
         // the next tile column (its tiles from the diagonal down) by the
         // panels before this one
         const int cb = kb + PW;
@@ -759,7 +842,7 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
                         });
       }
       __syncthreads();
-      if (kb + PW < BK) {
+      if (p + 1 < panels) {
         // and by this panel
         const int cb = kb + PW;
         panel_tiles<BK>(P, kb, 1, (BK - cb) / PW, 0, 4, wave, lane, [&](int e, int& r0, int& c0) {
@@ -770,19 +853,13 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
       }
     }
   }
+}
 
-  // L_kk back to the factor (the inverse below keeps P's lower part), the
-  // stores draining while the inverse is formed
-#pragma unroll
-  for (int u = 0; u < PER; u++) {
-    int r, col;
-    const int e = tid + u * 256;
-    lower_entry<BK>(min(e, NL - 1), r, col);
-    const double lv = P[r][col];
-    if (e < NL && r < b) D[r + static_cast<int64_t>(col) * si.f] = lv;
-  }
-
-  // ---- inverse: the 16x16 diagonal blocks (16 lanes each), then doubling ----
+// The inverses of the 16x16 diagonal blocks of the factor in P (16 lanes each),
+// stored above the diagonal and in column BK.  All threads, past a barrier.
+template <int BK>
+__device__ __forceinline__ void invert16(double (*P)[BK + 1], const double* rd, int tid)
+{
   if (tid < BK) {
     const int bb = (tid / PW) * PW, j = tid % PW;
     double x[PW];
@@ -803,6 +880,65 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
     }
   }
   __syncthreads();
+}
+
+// Diagonal block `step` of supernode s, by one workgroup of 256 threads with
+// smem >= potrf_smem<BK>().  BK: padded block edge (32, 64 or 128) >= b.
+// FULL: the whole inverse; otherwise only the inverses of its 16x16 diagonal
+// blocks (the blocked TRSM's), the rest formed after the level (k_inv_blocks).
+template <int BK, bool FULL>
+__device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double* dinv, int* pivot,
+                                            int s, int step, double* smem)
+{
+  const SnInfo si = sninfo(c, L, s);
+  const int k0 = step * BT;
+  if (k0 >= si.nc) return;
+  const int b = min(BK, si.nc - k0);
+  double (*P)[BK + 1] = reinterpret_cast<double (*)[BK + 1]>(smem);
+  double* rd = smem + BK * (BK + 1);   // 1 / L(r, r)
+  __shared__ int bad;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // scalar tile bookkeeping
+  double* D = si.Ls + static_cast<int64_t>(k0) * si.f + k0;
+  // load the lower triangle (padded with the identity past b), all of a
+  // thread's entries in flight at once.  Every lane loads (entries past b or
+  // past the triangle read D[0] and are replaced), so the loads are not split
+  // by branches that would wait on each other.
+  constexpr int NL = BK * (BK + 1) / 2, PER = (NL + 255) / 256;
+  {
+    double v[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      int r, col;
+      lower_entry<BK>(min(tid + u * 256, NL - 1), r, col);
+      const bool in = r < b;
+      const double t = D[in ? r + static_cast<int64_t>(col) * si.f : 0];
+      v[u] = in ? t : (r == col ? 1.0 : 0.0);
+    }
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      int r, col;
+      lower_entry<BK>(min(tid + u * 256, NL - 1), r, col);
+      if (tid + u * 256 < NL) P[r][col] = v[u];
+    }
+  }
+  if (tid == 0) bad = INT_MAX;
+  __syncthreads();
+
+  potrf_factor<BK>(P, rd, b, si.a + k0, c.pivot_tol, &bad, tid, lane, wave);
+
+  // L_kk back to the factor (the inverse below keeps P's lower part), the
+  // stores draining while the inverse is formed
+#pragma unroll
+  for (int u = 0; u < PER; u++) {
+    int r, col;
+    const int e = tid + u * 256;
+    lower_entry<BK>(min(e, NL - 1), r, col);
+    const double lv = P[r][col];
+    if (e < NL && r < b) D[r + static_cast<int64_t>(col) * si.f] = lv;
+  }
+
+  invert16<BK>(P, rd, tid);
   double* W = dinv + c.dinv_off[s] + static_cast<int64_t>(step) * BT * BT;
   if constexpr (FULL) {
     inverse_full<BK>(P, W, b, tid, wave, lane);
@@ -831,6 +967,175 @@ __global__ void __launch_bounds__(256) k_potrf_inv(CholDev c, const int* __restr
   if (step * BT >= c.sn_first[s + 1] - c.sn_first[s]) return;
   potrf_block<BK, (BK < 128)>(c, batch_at(c.L, sy, bt), batch_at(c.dinv, sy, bt), c.pivot + sy,
                               s, step, smem);
+}
+
+// The panel of supernodes with at most 32 columns, from the assembled entries to
+// the factor: the children's contributions, the diagonal block's factor and
+// inverse, and L21 = A21 Dinv^T for one tile of 128 rows per task.  Every tile forms
+// the diagonal block itself, and the first one writes its inverse; the block in the
+// panel stays as assembled, as other tiles may still have to read it: the sweeps
+// use the inverse alone.  In place of an extend-add, a diagonal-block and a TRSM
+// launch per tree level: these levels are bound by launches and latency, 13-25 us
+// each in one launch against 27-45 in three (1,000 buses).  Children's entries are
+// added in the order of the child list, with two children's loads in flight.
+// System blockIdx.y.
+constexpr int FP = 32;
+
+__global__ void __launch_bounds__(256) k_front_panel(CholDev c, const int* __restrict__ tsn,
+                                                     const int* __restrict__ ttr, Batch bt)
+{
+  __builtin_amdgcn_s_setprio(3);   // the critical chain: issue priority (see k_dense_nt)
+  __shared__ double Ps[FP * (FP + 1) + FP];
+  __shared__ double As[FP][BT + 2];   // the tile's rows of A21, column-major
+  __shared__ int bad;
+  double (*P)[FP + 1] = reinterpret_cast<double (*)[FP + 1]>(Ps);
+  double* rd = Ps + FP * (FP + 1);
+  const int sy = batch_sys(bt);
+  if (sy < 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+  const int s = uni(tsn[blockIdx.x]), tile = uni(ttr[blockIdx.x]);
+  const Sn sn = load_sn(c, s, lane);
+  const int a0 = sn.a, nc = sn.nc, f = sn.f;
+  double* Ls = batch_at(c.L, sy, bt) + sn.l_off;
+  const double* Ub = batch_at(c.U, sy, bt);
+  constexpr int NL = FP * (FP + 1) / 2, PER = (NL + 255) / 256;
+  constexpr int CPT = FP / 2, KB = 4;   // columns of a thread's row of the tile, per step
+  // thread: front row R, columns h, h + 2, .. of the tile; entries of the triangle
+  const int R = nc + tile * BT + (tid & (BT - 1)), h = uni(tid >> 7);
+  const bool live = R < f;
+  double va[CPT], vd[PER];
+#pragma unroll
+  for (int k = 0; k < CPT; k++) {
+    const int col = h + 2 * k;
+    va[k] = (live && col < nc) ? Ls[static_cast<int64_t>(col) * f + R] : 0.0;
+  }
+  int dr[PER], dc[PER];
+#pragma unroll
+  for (int u = 0; u < PER; u++) {
+    lower_entry<FP>(min(tid + u * 256, NL - 1), dr[u], dc[u]);
+    vd[u] = dr[u] < nc ? Ls[static_cast<int64_t>(dc[u]) * f + dr[u]] : (dr[u] == dc[u] ? 1.0 : 0.0);
+  }
+  // G children from t0 on, their loads in flight together
+  auto add_children = [&](auto count, int t0) {
+    constexpr int G = decltype(count)::value;
+    const int cw = child_words<G>(sn, t0, lane);
+    // their rows at this thread's front row, at the panel's columns (lane: column)
+    // and at its entries of the triangle
+    int ir[G], ic[G], dra[G][PER], dca[G][PER];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      const int* iv = sn.inv + static_cast<int64_t>(t0 + g) * sn.stride;
+      ir[g] = iv[live ? R : 0];
+      ic[g] = iv[min(lane, nc - 1)];
+#pragma unroll
+      for (int u = 0; u < PER; u++) {
+        dra[g][u] = iv[min(dr[u], nc - 1)];
+        dca[g][u] = iv[min(dc[u], nc - 1)];
+      }
+    }
+    double xd[G][PER], xa[G][CPT];
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+      const int n = rl32(cw, 4 * g + 2);
+      const double* uc = Ub + rl64(cw, 4 * g);
+      if (!live) ir[g] = -1;
+      // lane l: where the child's column for front column l starts
+      const int64_t cb = packed_lower(0, max(ic[g], 0), n);
+      const int clo = static_cast<int>(cb), chi = static_cast<int>(cb >> 32);
+#pragma unroll
+      for (int u = 0; u < PER; u++) {
+        if (dr[u] >= nc) dra[g][u] = -1;
+        const bool ok = dra[g][u] >= 0 && dca[g][u] >= 0;
+        xd[g][u] = uc[ok ? packed_lower(dra[g][u], dca[g][u], n) : 0];
+      }
+#pragma unroll
+      for (int k0 = 0; k0 < CPT; k0 += KB) {
+        if (h + 2 * k0 >= nc) break;   // uniform
+#pragma unroll
+        for (int k = k0; k < k0 + KB; k++) {   // past nc: a repeat, not added
+          const int l = h + 2 * k;
+          const int64_t at = static_cast<int64_t>(
+              (static_cast<uint64_t>(static_cast<uint32_t>(rl32(chi, l))) << 32) |
+              static_cast<uint32_t>(rl32(clo, l)));
+          xa[g][k] = uc[at + max(ir[g], max(rl32(ic[g], l), 0))];
+        }
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < G; g++) {
+#pragma unroll
+      for (int u = 0; u < PER; u++)
+        vd[u] = (dra[g][u] >= 0 && dca[g][u] >= 0) ? vd[u] + xd[g][u] : vd[u];
+#pragma unroll
+      for (int k0 = 0; k0 < CPT; k0 += KB) {
+        if (h + 2 * k0 >= nc) break;
+#pragma unroll
+        for (int k = k0; k < k0 + KB; k++) {
+          const bool has = h + 2 * k < nc && rl32(ic[g], h + 2 * k) >= 0;
+          va[k] = has && ir[g] >= 0 ? va[k] + xa[g][k] : va[k];
+        }
+      }
+    }
+  };
+  int t0 = 0;
+  for (; t0 + 2 <= sn.nch; t0 += 2) add_children(std::integral_constant<int, 2>{}, t0);
+  if (t0 < sn.nch) add_children(std::integral_constant<int, 1>{}, t0);
+#pragma unroll
+  for (int u = 0; u < PER; u++)
+    if (tid + u * 256 < NL) P[dr[u]][dc[u]] = vd[u];
+#pragma unroll
+  for (int k = 0; k < CPT; k++) As[h + 2 * k][tid & (BT - 1)] = va[k];
+  if (tid == 0) bad = INT_MAX;
+  __syncthreads();
+  // at most 16 columns: the second panel is the identity, and stays out of all below
+  const int panels = nc <= PW ? 1 : 2;
+  potrf_factor<FP>(P, rd, nc, a0, c.pivot_tol, &bad, tid, lane, wave, panels);
+  if (panels == 1 && tid < PW) rd[PW + tid] = 1.0;
+  if (panels == 1) __syncthreads();
+  invert16<FP>(P, rd, tid);
+  if (panels == 2) inverse_level<FP, 16>(P, wave, lane);
+  if (tile == 0) {
+    double* W = batch_at(c.dinv, sy, bt) + sn.dinv_off;
+#pragma unroll
+    for (int u = 0; u < PER; u++)
+      if (tid + u * 256 < NL && dr[u] < nc)
+        W[static_cast<int64_t>(dc[u]) * BT + dr[u]] = xinv<FP>(P, dr[u], dc[u]);
+    if (tid == 0 && bad != INT_MAX) atomicMin(c.pivot + sy, bad);
+  }
+  // L21: wave w takes rows 32 w .. 32 w + 31 of the tile, in two by two MFMA tiles
+  const int rows = f - (nc + tile * BT), r0 = 32 * wave;
+  if (r0 >= rows) return;   // no barrier follows
+  const int m16 = lane & 15, q4 = lane >> 4;
+  d4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k0 = 0; k0 < FP; k0 += 4) {
+    if (k0 >= nc) break;
+    double fa[2], fb[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      fa[i] = As[k0 + q4][r0 + 16 * i + m16];
+      fb[i] = xinv<FP>(P, 16 * i + m16, k0 + q4);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[j], fa[i], acc[i][j], 0, 0, 0);
+  }
+  double* C = Ls + nc + tile * BT + r0;
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+#pragma unroll
+    for (int j = 0; j < 2; j++)
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int row = 16 * i + m16, col = 16 * j + 4 * v + q4;
+        if (r0 + row < rows && col < nc) C[static_cast<int64_t>(col) * f + row] = acc[i][j][v];
+      }
 }
 
 // The whole inverse of 128-wide diagonal blocks whose factorization left only
@@ -1046,11 +1351,29 @@ void dense_nt(const CholDev& c, int ntasks, const int* tsn, const int* ttr, cons
   // `done` rides on the launch itself (its completion signal), so no marker
   // of its own sits between this kernel and the next one of the stream
   if (short_rows)
-    hipExtLaunchKernelGGL((k_dense_nt<32, 2, 1, 4, 8>), dim3(ntasks, b.count, BT / SHORT_TN),
+    hipExtLaunchKernelGGL((k_dense_nt<false, 32, 2, 1, 4, 8>), dim3(ntasks, b.count, BT / SHORT_TN),
                           dim3(256), 0, st, nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
   else
-    hipExtLaunchKernelGGL((k_dense_nt<128, 4, 4, 2, 2>), dim3(ntasks, b.count), dim3(256),
+    hipExtLaunchKernelGGL((k_dense_nt<false, 128, 4, 4, 2, 2>), dim3(ntasks, b.count), dim3(256),
                           alone ? ALONE_LDS : 0, st, nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
+  HIPCHK(hipGetLastError());
+}
+
+void update_matrices(const CholDev& c, int ntasks, const int* tsn, const int* ttr, const int* ttc,
+                     bool small, const Batch& b, hipStream_t st)
+{
+  if (ntasks <= 0 || b.count <= 0) return;
+  const dim3 grid(ntasks, b.count);
+  if (small) k_dense_nt<true, 64, 2, 2, 2, 4><<<grid, 256, 0, st>>>(c, tsn, ttr, ttc, 1, 0, b);
+  else k_dense_nt<true, 128, 4, 2, 4, 2><<<grid, 512, 0, st>>>(c, tsn, ttr, ttc, 1, 0, b);
+  HIPCHK(hipGetLastError());
+}
+
+void front_panel(const CholDev& c, int ntasks, const int* tsn, const int* ttr, const Batch& b,
+                 hipStream_t st)
+{
+  if (ntasks <= 0 || b.count <= 0) return;
+  k_front_panel<<<dim3(ntasks, b.count), 256, 0, st>>>(c, tsn, ttr, b);
   HIPCHK(hipGetLastError());
 }
 
