@@ -77,7 +77,7 @@ CholEngine::CholEngine(const Pattern& a, const CholOptions& opt, hipStream_t st)
       dpos[j] = pl_.l_off[s] + lj * f + lj;
     }
     uvo[s + 1] = uvo[s] + pl_.nr(s);
-    dvo[s + 1] = dvo[s] + static_cast<int64_t>(cdiv(pl_.nc(s), NB)) * NB * NB;
+    dvo[s + 1] = dvo[s] + dev::inv_size(pl_.nc(s));
   }
   diag_pos_.upload(dpos);
   uvec_off_.upload(uvo);
@@ -128,7 +128,7 @@ CholEngine::Sizes CholEngine::sizes() const
 {
   auto at_least1 = [](int64_t v) { return std::max<int64_t>(v, 1); };
   return Sizes{at_least1(pl_.l_off[pl_.ns]), at_least1(pl_.u_off[pl_.ns]), at_least1(n_dinv_),
-               at_least1(pl_.n), at_least1(n_ubuf_), at_least1(n_bpart_)};
+               at_least1(pl_.n), at_least1(n_ubuf_), at_least1(n_exch_)};
 }
 
 void CholEngine::set_tuning(const Tuning& t, int count)
@@ -149,10 +149,10 @@ void CholEngine::bind(const Storage& s, int64_t vs, int cap)
   cd_.pivot = s.pivot;
   ybuf_ = s.y;
   sd_.ubuf = s.ubuf;
-  sd_.bpart = s.bpart;
+  sd_.exch = s.exch;
   vs_ = vs;
   cap_ = cap;
-  // only the b x b lower part of an inverted diagonal block is ever written
+  // only the lower triangles of the inverses are ever written
   dev::fill(cd_.dinv, 0.0, n_dinv_, dev::Batch{cap, vs, nullptr}, st_);
 }
 
@@ -160,7 +160,7 @@ void CholEngine::own(int cap)
 {
   const Sizes z = sizes();
   auto al = [](int64_t v) { return (v + 31) / 32 * 32; };   // 256-byte slots
-  const int64_t vs = al(z.L) + al(z.U) + al(z.dinv) + al(z.y) + al(z.ubuf) + al(z.bpart);
+  const int64_t vs = al(z.L) + al(z.U) + al(z.dinv) + al(z.y) + al(z.ubuf) + al(z.exch);
   own_.alloc(static_cast<size_t>(vs) * cap);
   own_piv_.alloc(static_cast<size_t>(cap));
   double* p = own_.p;
@@ -175,7 +175,7 @@ void CholEngine::own(int cap)
   p += al(z.y);
   s.ubuf = p;
   p += al(z.ubuf);
-  s.bpart = p;
+  s.exch = p;
   s.pivot = own_piv_.p;
   bind(s, vs, cap);
 }
@@ -215,7 +215,7 @@ void CholEngine::build_fronts()
     }
     sr[s] = dev::SnRec{pl_.sn_first[s], nc, nr, pl_.child_ptr[s], nch, rows, {0, 0},
                        pl_.l_off[s], dinv, pl_.u_off[s], off};
-    dinv += static_cast<int64_t>(cdiv(nc, NB)) * NB * NB;
+    dinv += dev::inv_size(nc);
   }
   if (inv.empty()) inv.push_back(-1);
   child_rec_.upload(rec);
@@ -243,9 +243,10 @@ void CholEngine::build_tasks()
   const int gmax = std::clamp(tun_.group_max, 1, GMAX);
   const int nlev = static_cast<int>(pl_.level_ptr.size()) - 1;
   lv_.assign(nlev, Level{});
+  inv_blk_ = inv_grp_ = Launch{};
   std::vector<int> eap, eacol, eacptr{0}, eacc, eaccol;
   std::vector<int> potrf, trsm_sn, trsm_tr, upd_sn, upd_tr, upd_tc;
-  std::vector<int> syrk_sn, syrk_tr, syrk_tc, inv_sn, inv_step;
+  std::vector<int> syrk_sn, syrk_tr, syrk_tc, inv_sn, inv_step, grp_sn, grp_ix;
   std::vector<int> fp_sn, fp_tile;
   auto narrow = [&](int s) { return pl_.nc(s) <= dev::FRONT_NC; };
   struct Contrib {
@@ -480,7 +481,6 @@ void CholEngine::build_tasks()
     L.syrk.cnt = static_cast<int>(syrk_sn.size()) - L.syrk.off;
     // the whole inverses of the blocks of the steps factored without them
     // (128-wide launches): b^3/3 flops, the triangle read twice and written
-    L.inv.off = static_cast<int>(inv_sn.size());
     for (int j = 0; j < nsteps; j++) {
       if (L.potrf[j].maxb <= 64) continue;
       for (int q = b0; q < b1; q++) {
@@ -489,12 +489,30 @@ void CholEngine::build_tasks()
         const double db = std::min(NB, nc - j * NB);
         inv_sn.push_back(s);
         inv_step.push_back(j);
-        L.inv.flops += db * db * db / 3;
-        L.inv.bytes += 24.0 * db * (db + 1) / 2;
+        inv_blk_.flops += db * db * db / 3;
+        inv_blk_.bytes += 24.0 * db * (db + 1) / 2;
       }
     }
-    L.inv.cnt = static_cast<int>(inv_sn.size()) - L.inv.off;
+    // and of the groups' rest, the longest strips of each first: (n^3 - sum b^3)/3
+    // flops, the triangle read and written
+    for (int q = b0; q < b1; q++) {
+      const int s = pl_.level_sn[q], nc = pl_.nc(s);
+      for (int g0 = 0; g0 < nc; g0 += dev::INV_GROUP) {
+        const int n = std::min(dev::INV_GROUP, nc - g0);
+        if (n <= NB) continue;
+        for (int k = 0; k < (cdiv(n, NB) - 1) * (NB / 16); k++) {
+          grp_sn.push_back(s);
+          grp_ix.push_back(g0 / dev::INV_GROUP * 32 + k);
+        }
+        const double dn = n, full = n / NB, tail = n % NB;
+        const double db = full * NB * NB * NB + tail * tail * tail;
+        inv_grp_.flops += (dn * dn * dn - db) / 3;
+        inv_grp_.bytes += 16.0 * (dn * dn - (full * NB * NB + tail * tail)) / 2;
+      }
+    }
   }
+  inv_blk_.cnt = static_cast<int>(inv_sn.size());
+  inv_grp_.cnt = static_cast<int>(grp_sn.size());
   auto up = [](DevBuf<int>& b, std::vector<int>& v) {
     if (v.empty()) v.push_back(0);
     b.upload(v);
@@ -517,6 +535,8 @@ void CholEngine::build_tasks()
   up(t_syrk_tc_, syrk_tc);
   up(t_inv_sn_, inv_sn);
   up(t_inv_step_, inv_step);
+  up(t_grp_sn_, grp_sn);
+  up(t_grp_ix_, grp_ix);
 }
 
 void CholEngine::build_solve()
@@ -539,8 +559,20 @@ void CholEngine::build_solve()
     solve_lower_[top[s]] += nc * (nc + 1) / 2 + nr * nc;
     solve_n_[top[s]] += pl_.nc(s);
     if (!top[s]) continue;
-    for (int b = 0; b < cdiv(pl_.nc(s), NB); b++) fwd_top.insert(fwd_top.end(), {s, 0, b});
-    for (int u = 0; u < cdiv(pl_.nr(s), NB); u++) fwd_top.insert(fwd_top.end(), {s, 1, u});
+    // per group of pivot columns: the group before's chunk of its rows, its values,
+    // that chunk of the later groups' rows; then the rows below
+    const int n = pl_.nc(s), R = dev::TOP_ROWS, G = dev::INV_GROUP;
+    for (int g = 0; g * G < n; g++) {
+      const int i0 = g * G / R, i1 = cdiv(std::min(n, (g + 1) * G), R);
+      if (g > 0)
+        for (int i = i0; i < i1; i++) fwd_top.insert(fwd_top.end(), {s, dev::TOP_CHUNK, i, g - 1});
+      for (int i = i0; i < i1; i++) fwd_top.insert(fwd_top.end(), {s, dev::TOP_PIVOT, i, 0});
+      if (g > 0)
+        for (int i = i1; i < cdiv(n, R); i++)
+          fwd_top.insert(fwd_top.end(), {s, dev::TOP_CHUNK, i, g - 1});
+    }
+    for (int u = 0; u < cdiv(pl_.nr(s), 2048 / dev::top_waves(n)); u++)
+      fwd_top.insert(fwd_top.end(), {s, dev::TOP_BELOW, u, 0});
   }
   // forest items, by tree level (leaves first): a tall supernode, or up to four
   // short ones of the level
@@ -550,7 +582,7 @@ void CholEngine::build_solve()
   for (int s = 0; s < ns; s++) {
     foff[s + 1] = foff[s] + pl_.nc(s) + pl_.nr(s);
     uvo[s + 1] = uvo[s] + pl_.nr(s);
-    dvo[s + 1] = dvo[s] + static_cast<int64_t>(cdiv(pl_.nc(s), NB)) * NB * NB;
+    dvo[s + 1] = dvo[s] + dev::inv_size(pl_.nc(s));
   }
   for (size_t l = 0; l + 1 < pl_.level_ptr.size(); l++) {
     int open = 0;   // waves left in the level's last item
@@ -575,16 +607,22 @@ void CholEngine::build_solve()
   }
   for (size_t k = fwd.size(); k >= 4; k -= 4)   // parents first
     bwd.insert(bwd.end(), fwd.begin() + (k - 4), fwd.begin() + k);
-  std::vector<int64_t> bpo(ns + 1, 0);
-  for (int s = ns - 1; s >= 0; s--) {   // parents first: row chunks, then pivot blocks
+  for (int s = ns - 1; s >= 0; s--) {   // parents first
     if (!top[s]) continue;
-    const int np = cdiv(pl_.nc(s), NB), nu = cdiv(pl_.nr(s), NB);
-    for (int u = 0; u < nu; u++)
-      for (int k = 0; k < np; k++) bwd_top.insert(bwd_top.end(), {s, 0, u * np + k});
-    for (int k = np - 1; k >= 0; k--) bwd_top.insert(bwd_top.end(), {s, 1, k});
+    const int n = pl_.nc(s), f = n + pl_.nr(s);
+    for (int g0 = (n - 1) / dev::INV_GROUP * dev::INV_GROUP; g0 >= 0; g0 -= dev::INV_GROUP) {
+      const int g1 = std::min(n, g0 + dev::INV_GROUP);
+      for (int kind : {dev::TOP_RHS, dev::TOP_PIVOT}) {
+        const int rows = kind == dev::TOP_RHS ? f - g1 : g1 - g0;
+        if (rows == 0) continue;
+        for (int k = g0; k < g1; k += 16 << dev::top_shape(rows))
+          bwd_top.insert(bwd_top.end(), {s, kind, k, 0});
+      }
+    }
   }
-  for (int s = 0; s < ns; s++)   // the forest has no chunk partials
-    bpo[s + 1] = bpo[s] + (top[s] ? static_cast<int64_t>(cdiv(pl_.nr(s), NB)) * pl_.nc(s) : 0);
+  std::vector<int64_t> exo(ns + 1, pl_.n);
+  for (int s = 0; s < ns; s++)
+    exo[s + 1] = exo[s] + (top[s] ? static_cast<int64_t>((pl_.nc(s) - 1) / dev::INV_GROUP) * pl_.nc(s) : 0);
   // pull lists: front row of a parent <- entries of its children's update vectors
   std::vector<int> cnt(static_cast<size_t>(foff[ns]) + 1, 0);
   for (int c = 0; c < ns; c++) {
@@ -610,8 +648,8 @@ void CholEngine::build_solve()
   if (fsn.empty()) fsn.push_back(dev::ForestSn{});
   forest_.upload(fsn);
   sd_.forest = forest_.p;
-  sd_.n_fwd_top = static_cast<int>(fwd_top.size() / 3);
-  sd_.n_bwd_top = static_cast<int>(bwd_top.size() / 3);
+  sd_.n_fwd_top = static_cast<int>(fwd_top.size() / 4);
+  sd_.n_bwd_top = static_cast<int>(bwd_top.size() / 4);
   upi(fwd_items_, fwd);
   upi(bwd_items_, bwd);
   upi(fwd_top_items_, fwd_top);
@@ -619,7 +657,7 @@ void CholEngine::build_solve()
   upi(pull_ptr_, cnt);
   upi(pull_src_, src);
   front_off_.upload(foff);
-  bpart_off_.upload(bpo);
+  exch_off_.upload(exo);
   flags_.alloc(5);   // wait-bound error word, four sweep item counters
   sd_.fwd_items = fwd_items_.p;
   sd_.bwd_items = bwd_items_.p;
@@ -629,12 +667,12 @@ void CholEngine::build_solve()
   sd_.pull_ptr = pull_ptr_.p;
   sd_.pull_src = pull_src_.p;
   sd_.front_off = front_off_.p;
-  sd_.bpart_off = bpart_off_.p;
+  sd_.exch_off = exch_off_.p;
+  n_exch_ = exo[ns];
   sd_.err = flags_.p;
   sd_.ticket = flags_.p + 1;
   forest_full_ = n_cu_ * dev::forest_blocks_per_cu();
   share_ = 1;
-  n_bpart_ = bpo[ns];
   dev::fill_i(flags_.p, 0, 1, st_);
 }
 
@@ -755,14 +793,18 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
       }
     }
     if (rest_pending) HIPCHK(hipStreamWaitEvent(st_, ev_rest_, 0));
-    timed(PK_INV_BLOCKS, L.inv, [&] {
-      dev::inv_blocks(cd_, L.inv.cnt, t_inv_sn_.p + L.inv.off, t_inv_step_.p + L.inv.off, b, st_);
-    });
     timed(PK_DENSE_NT, L.syrk, [&] {
       dev::update_matrices(cd_, L.syrk.cnt, t_syrk_sn_.p + L.syrk.off, t_syrk_tr_.p + L.syrk.off,
                            t_syrk_tc_.p + L.syrk.off, L.small_u, b, st_);
     });
   }
+  // the solves' inverses, all levels at once
+  timed(PK_INV_BLOCKS, inv_blk_, [&] {
+    dev::inv_blocks(cd_, inv_blk_.cnt, t_inv_sn_.p, t_inv_step_.p, b, st_);
+  });
+  timed(PK_INV_BLOCKS, inv_grp_, [&] {
+    dev::inv_groups(cd_, inv_grp_.cnt, t_grp_sn_.p, t_grp_ix_.p, b, st_);
+  });
 }
 
 std::vector<int> CholEngine::pivots(int count)
@@ -810,8 +852,8 @@ dev::SweepFill CholEngine::sweep_fill(double* x) const
   f.n[1] = pl_.n;
   f.p[2] = sd_.ubuf;
   f.n[2] = n_ubuf_;
-  f.p[3] = sd_.bpart;
-  f.n[3] = n_bpart_;
+  f.p[3] = sd_.exch;
+  f.n[3] = n_exch_;
   f.ticket = sd_.ticket;
   return f;
 }

@@ -91,11 +91,11 @@ class CholEngine {
  public:
   // Doubles of per-system storage, by kind.
   struct Sizes {
-    int64_t L, U, dinv, y, ubuf, bpart;
+    int64_t L, U, dinv, y, ubuf, exch;
   };
   // Per-system storage of system 0 (pivot: one int per system).
   struct Storage {
-    double *L, *U, *dinv, *y, *ubuf, *bpart;
+    double *L, *U, *dinv, *y, *ubuf, *exch;
     int* pivot;
   };
   // Launch shapes of the numeric factorization (tile counts are over all the
@@ -179,7 +179,7 @@ class CholEngine {
     double flops = 0.0, bytes = 0.0;   // algorithmic, for the profiler
   };
   struct Level {
-    Launch front, ea_panel, syrk, inv;
+    Launch front, ea_panel, syrk;
     bool small_u = false;   // update matrices in 64 x 64 tiles
     std::vector<Launch> potrf, trsm, upd_next, upd_rest;
     // per step: its position in its group of consecutive steps and the
@@ -210,15 +210,16 @@ class CholEngine {
   dev::CholDev cd_{};
   dev::SolveDev sd_{};
   DevBuf<int> sn_first_, rows_ptr_, rows_, rel_, child_ptr_, child_list_, post_, sn_parent_;
-  DevBuf<int64_t> l_off_, u_off_, a_dst_, diag_pos_, uvec_off_, dinv_off_, front_off_;
+  DevBuf<int64_t> l_off_, u_off_, a_dst_, diag_pos_, uvec_off_, dinv_off_, front_off_, exch_off_;
   DevBuf<int> a_src_;
-  int64_t n_ubuf_ = 0, n_dinv_ = 0;
+  int64_t n_ubuf_ = 0, n_dinv_ = 0, n_exch_ = 0;
   // task lists
   std::vector<Level> lv_;
+  Launch inv_blk_, inv_grp_;   // the solves' inverses, all levels
   DevBuf<int> t_ea_p_, t_ea_col_, t_ea_cptr_, t_ea_cc_, t_ea_ccol_;
   DevBuf<int> t_potrf_, t_trsm_sn_, t_trsm_tr_, t_upd_sn_, t_upd_tr_, t_upd_tc_;
   DevBuf<int> t_syrk_sn_, t_syrk_tr_, t_syrk_tc_;
-  DevBuf<int> t_inv_sn_, t_inv_step_;
+  DevBuf<int> t_inv_sn_, t_inv_step_, t_grp_sn_, t_grp_ix_;
   DevBuf<int> t_fp_sn_, t_fp_tile_;
   DevBuf<dev::ChildRec> child_rec_;
   DevBuf<dev::SnRec> sn_rec_;
@@ -226,11 +227,9 @@ class CholEngine {
   int n_cu_ = 1;   // compute units: persistent-launch width
   // solve items
   DevBuf<int> fwd_items_, bwd_items_, pull_ptr_, pull_src_, flags_;
-  DevBuf<int64_t> bpart_off_;
   DevBuf<dev::ForestSn> forest_;
   DevBuf<int> fwd_top_items_, bwd_top_items_;
   double* ybuf_ = nullptr;   // forward-sweep output (bound storage)
-  int64_t n_bpart_ = 0;
   double solve_lower_[2] = {0.0, 0.0};   // stored lower-trapezoid entries: forest, top
   int64_t solve_n_[2] = {0, 0};          // columns: forest, top
 };

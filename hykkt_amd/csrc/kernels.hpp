@@ -281,6 +281,30 @@ struct SnRec {
 // Widest supernode that front_panel() takes.
 constexpr int FRONT_NC = 32;
 
+// Inverses of the factor's diagonal blocks, in groups of INV_GROUP columns: group g
+// of a supernode is a column-major inv_ld x inv_ld matrix at g * INV_GROUP^2 from
+// the supernode's slot, its lower triangle the inverse of L's (supernodes of at most
+// FRONT_NC columns: one 32 x 32 matrix).
+constexpr int INV_GROUP = 512;
+__host__ __device__ inline int inv_ld(int nc, int g)
+{
+  if (nc <= FRONT_NC) return FRONT_NC;
+  const int n = nc - g * INV_GROUP;
+  return n >= INV_GROUP ? INV_GROUP : (n + 127) / 128 * 128;
+}
+__host__ __device__ inline int64_t inv_size(int nc)
+{
+  const int g = (nc - 1) / INV_GROUP, ld = inv_ld(nc, g);
+  return static_cast<int64_t>(g) * INV_GROUP * INV_GROUP + static_cast<int64_t>(ld) * ld;
+}
+// Its diagonal block `step` (128 columns).
+__host__ __device__ inline int64_t inv_at(int nc, int step)
+{
+  const int g = step / (INV_GROUP / 128), i = step - g * (INV_GROUP / 128);
+  return static_cast<int64_t>(g) * INV_GROUP * INV_GROUP +
+         static_cast<int64_t>(i) * 128 * (inv_ld(nc, g) + 1);
+}
+
 // The factor storage of system 0 (system k's at + k*vs, vs of the Batch).
 struct CholDev {
   int n, ns;
@@ -300,8 +324,8 @@ struct CholDev {
   double* U;
   int* pivot;               // one int per system: first failing pivot (min), INT_MAX if none
   double pivot_tol;
-  double* dinv;             // inverted 128x128 diagonal blocks (column-major)
-  const int64_t* dinv_off;  // ns+1, offset of supernode s's first block in dinv
+  double* dinv;             // inverses of the diagonal blocks (see inv_ld)
+  const int64_t* dinv_off;  // ns+1, supernode s's slot in dinv
 };
 
 // Extend-add tasks: task t = (parent p, parent front column col);
@@ -314,7 +338,7 @@ void extend_add(const CholDev& c, int ntasks, const int* task_p, const int* task
 // dinv slots must be zero-initialized once (only the b x b lower part is written).
 // Blocks wider than 64 (max_b > 64) leave only the inverses of their 16x16
 // diagonal blocks in the slot: their TRSM is trsm(), the whole inverse comes
-// from inv_blocks() after the level.
+// from inv_blocks() after the last level.
 void potrf_inv(const CholDev& c, int nsn, const int* sns, int step, int max_b, const Batch& b,
                hipStream_t st);
 // L21 = A21 L_kk^{-T} below the 128-wide diagonal blocks of step `step` by blocked
@@ -325,6 +349,10 @@ void trsm(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr, 
 // inside potrf_inv.
 void inv_blocks(const CholDev& c, int ntasks, const int* task_sn, const int* task_step,
                 const Batch& b, hipStream_t st);
+// The groups' inverses below those blocks (tasks: supernode, 32 * group + strip of 16
+// columns).
+void inv_groups(const CholDev& c, int ntasks, const int* tsn, const int* tix, const Batch& b,
+                hipStream_t st);
 
 // MFMA update tiles over (supernode, tile row, tile col) tasks.  mode 0: trailing
 // panel update after block `step`; mode m >= 3: after blocks `step` .. `step`+m-2
@@ -355,8 +383,8 @@ void trsm_inv(const CholDev& c, int ntasks, const int* task_sn, const int* task_
 // memory.
 bool streams_overlap(hipStream_t a, hipStream_t b, int* words);
 
-// Single-launch supernodal solves over the whole tree.  Work items are
-// 128-row blocks of the fronts, dispatched in a dependency-respecting order;
+// Single-launch supernodal solves over the whole tree.  Work items are parts
+// of the fronts, dispatched in a dependency-respecting order;
 // items synchronise on the values they exchange, whose buffers are filled
 // with a sentinel (fill_sentinel) before each sweep.  With several systems,
 // launch item i*count + k is item i of system k.
@@ -374,12 +402,27 @@ struct ForestSn {
   int64_t pad2;
 };
 
+// Items of the top of the tree (see kernels_trsv.hip): their kinds, the rows of a
+// pivot or chunk item, the waves that share a column set of an item of rows below
+// nc columns (16 columns each; the other waves take further sets of 128 rows), and
+// how many times a backward item's 1024 rows (16 columns) halve (its columns
+// double) for so many rows.
+constexpr int TOP_RHS = 0, TOP_PIVOT = 1, TOP_CHUNK = 2, TOP_BELOW = 3;
+constexpr int TOP_ROWS = 64;
+__host__ __device__ inline int top_waves(int nc)
+{
+  return nc > 128 ? 16 : nc > 64 ? 8 : nc > 32 ? 4 : 2;
+}
+__host__ __device__ inline int top_shape(int rows)
+{
+  return rows > 512 ? 0 : rows > 256 ? 1 : rows > 128 ? 2 : 3;
+}
+
 struct SolveDev {
   // Items of the small-supernode forest (fwd_items, bwd_items: 4 ints each, indices
-  // into `forest`; see kernels_forest.hip) and of the top of the tree (*_top: 3 ints
+  // into `forest`; see kernels_forest.hip) and of the top of the tree (*_top: 4 ints
   // per item) are separate launches: forward forest then top, backward top then
-  // forest.  Top items: supernode, kind, index (forward: 0 pivot, 1 update, block;
-  // backward: 0 row chunk, chunk * blocks + column block; 1 pivot, block).
+  // forest.  Top items: supernode, kind, index, group (forward chunks).
   const ForestSn* forest;
   const int* fwd_items;
   int n_fwd;
@@ -394,8 +437,10 @@ struct SolveDev {
   const int* pull_src;
   const int64_t* front_off; // ns+1: offset of s's front rows in the pull_ptr index
   double* ubuf;             // forward update vectors (sentinel-filled per sweep; per system)
-  double* bpart;            // backward chunk partials: chunk u of s at bpart_off[s] + u*nc
-  const int64_t* bpart_off;
+  double* exch;             // the top's other exchanged values (sentinel-filled per sweep):
+                            // n backward right-hand sides, then forward chunks, chunk j of
+                            // s's pivot rows at exch_off[s] + j * nc
+  const int64_t* exch_off;
   int* err;                 // 1: a wait hit its bound (sticky until the host clears it)
   int* ticket;              // 4 item counters (forward forest, forward top, backward top,
                             // backward forest), zeroed with the first sentinel fill of a solve
@@ -412,7 +457,7 @@ void solve_forward_forest(const CholDev& c, const SolveDev& sd, const double* rh
                           const Batch& b, hipStream_t st);
 void solve_forward_top(const CholDev& c, const SolveDev& sd, const double* rhs, double* y,
                        const Batch& b, hipStream_t st);
-// L^T x = y (x and bpart sentinel-filled): the top of the tree, then the forest.
+// L^T x = y (x and exch sentinel-filled): the top of the tree, then the forest.
 void solve_backward_top(const CholDev& c, const SolveDev& sd, const double* y, double* x,
                         const Batch& b, hipStream_t st);
 void solve_backward_forest(const CholDev& c, const SolveDev& sd, const double* y, double* x,

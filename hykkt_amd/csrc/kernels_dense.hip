@@ -511,9 +511,8 @@ __global__ void __launch_bounds__(256, 2) k_trsm_inv(CholDev c, const int* __res
   GemmArgs g;
   g.A = panel + R0;
   g.lda = si.f;
-  g.B = batch_at(c.dinv, sy, bt) + c.dinv_off[tsn[blockIdx.x]] +
-        static_cast<int64_t>(step) * BT * BT;
-  g.ldb = BT;
+  g.B = batch_at(c.dinv, sy, bt) + c.dinv_off[tsn[blockIdx.x]] + inv_at(si.nc, step);
+  g.ldb = inv_ld(si.nc, k0 / INV_GROUP);
   g.C = panel + R0;
   g.ldc = si.f;
   g.M = min(TM, si.f - R0);
@@ -673,12 +672,12 @@ __device__ __forceinline__ void lower_entry(int e, int& r, int& col)
 
 // The doubling levels and the store of the whole inverse, from P holding L
 // in its lower part and the inverses of the 16x16 diagonal blocks (see
-// potrf_block), into the 128 x 128 dinv slot W (column-major; entries
-// outside the b x b lower triangle stay at the zeros written when the slot
-// was created).  All threads of the workgroup.
+// potrf_block), into the dinv slot at W (column-major, ldw; entries outside
+// the b x b lower triangle stay at the zeros written when the slot was
+// created).  All threads of the workgroup.
 template <int BK>
-__device__ __forceinline__ void inverse_full(double (*P)[BK + 1], double* W, int b, int tid,
-                                             int wave, int lane)
+__device__ __forceinline__ void inverse_full(double (*P)[BK + 1], double* W, int ldw, int b,
+                                             int tid, int wave, int lane)
 {
   constexpr int NL = BK * (BK + 1) / 2, PER = (NL + 255) / 256;
   if constexpr (BK >= 32) inverse_level<BK, 16>(P, wave, lane);
@@ -700,7 +699,7 @@ __device__ __forceinline__ void inverse_full(double (*P)[BK + 1], double* W, int
       int r, col;
       const int e = tid + (u0 + u) * 256;
       lower_entry<BK>(min(e, NL - 1), r, col);
-      if (u0 + u < PER && e < NL && r < b) W[static_cast<int64_t>(col) * BT + r] = xv[u];
+      if (u0 + u < PER && e < NL && r < b) W[static_cast<int64_t>(col) * ldw + r] = xv[u];
     }
   }
 }
@@ -939,9 +938,10 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
   }
 
   invert16<BK>(P, rd, tid);
-  double* W = dinv + c.dinv_off[s] + static_cast<int64_t>(step) * BT * BT;
+  double* W = dinv + c.dinv_off[s] + inv_at(si.nc, step);
+  const int ldw = inv_ld(si.nc, k0 / INV_GROUP);
   if constexpr (FULL) {
-    inverse_full<BK>(P, W, b, tid, wave, lane);
+    inverse_full<BK>(P, W, ldw, b, tid, wave, lane);
   } else {
     // the 16x16 diagonal blocks of the inverse, at their places in the slot
     constexpr int NE = (BK / PW) * (PW * (PW + 1) / 2);
@@ -949,7 +949,7 @@ __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double*
       const int bb = (e / (PW * (PW + 1) / 2)) * PW;
       int r, col;
       lower_entry<PW>(e % (PW * (PW + 1) / 2), r, col);
-      if (bb + r < b) W[static_cast<int64_t>(bb + col) * BT + bb + r] = xinv<BK>(P, bb + r, bb + col);
+      if (bb + r < b) W[static_cast<int64_t>(bb + col) * ldw + bb + r] = xinv<BK>(P, bb + r, bb + col);
     }
   }
   if (tid == 0 && bad != INT_MAX) atomicMin(pivot, bad);
@@ -980,6 +980,7 @@ __global__ void __launch_bounds__(256) k_potrf_inv(CholDev c, const int* __restr
 // added in the order of the child list, with two children's loads in flight.
 // System blockIdx.y.
 constexpr int FP = 32;
+static_assert(FP == FRONT_NC, "a narrow panel's slot is FP x FP");
 
 __global__ void __launch_bounds__(256) k_front_panel(CholDev c, const int* __restrict__ tsn,
                                                      const int* __restrict__ ttr, Batch bt)
@@ -1099,7 +1100,7 @@ __global__ void __launch_bounds__(256) k_front_panel(CholDev c, const int* __res
 #pragma unroll
     for (int u = 0; u < PER; u++)
       if (tid + u * 256 < NL && dr[u] < nc)
-        W[static_cast<int64_t>(dc[u]) * BT + dr[u]] = xinv<FP>(P, dr[u], dc[u]);
+        W[static_cast<int64_t>(dc[u]) * FP + dr[u]] = xinv<FP>(P, dr[u], dc[u]);
     if (tid == 0 && bad != INT_MAX) atomicMin(c.pivot + sy, bad);
   }
   // L21: wave w takes rows 32 w .. 32 w + 31 of the tile, in two by two MFMA tiles
@@ -1161,7 +1162,8 @@ __global__ void __launch_bounds__(256) k_inv_blocks(CholDev c, const int* __rest
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const double* D = si.Ls + static_cast<int64_t>(k0) * si.f + k0;
-  double* W = batch_at(c.dinv, sy, bt) + c.dinv_off[s] + static_cast<int64_t>(step) * BT * BT;
+  double* W = batch_at(c.dinv, sy, bt) + c.dinv_off[s] + inv_at(si.nc, step);
+  const int ldw = inv_ld(si.nc, k0 / INV_GROUP);
   {
     double v[PER];
 #pragma unroll
@@ -1183,13 +1185,92 @@ __global__ void __launch_bounds__(256) k_inv_blocks(CholDev c, const int* __rest
     const int bb = (e / T16) * PW;
     int r, col;
     lower_entry<PW>(e % T16, r, col);
-    const double x = (bb + r < b) ? W[static_cast<int64_t>(bb + col) * BT + bb + r]
+    const double x = (bb + r < b) ? W[static_cast<int64_t>(bb + col) * ldw + bb + r]
                                   : (r == col ? 1.0 : 0.0);
     if (r == col) P[bb + col][BK] = x;
     else P[bb + col][bb + r] = x;
   }
   __syncthreads();
-  inverse_full<BK>(P, W, b, tid, wave, lane);
+  inverse_full<BK>(P, W, ldw, b, tid, wave, lane);
+}
+
+// The inverses of groups of two to four 128-column diagonal blocks, below their
+// diagonal blocks' (which the launches before left): X = L^{-1} by columns,
+//   X(i, j) = -X(i, i) (L(i, j) X(j, j) + .. + L(i, i-1) X(i-1, j)),
+// a workgroup per strip of 16 columns, wave w rows 16 w .. 16 w + 15 of each block,
+// operands read straight into MFMA fragments, the strip and the sums through LDS.
+// With them a sweep passes a group of up to 512 columns in one product in place of a
+// chain of four, at 28 us per factorization at 1,000 buses, 34 at 5,000 (one
+// workgroup takes 15 us of matrix instructions for the first strip of a whole group).  Task: supernode, 32 group + strip; system
+// blockIdx.y.
+constexpr int IG_LD = PW + 1;   // row of the strip in LDS
+constexpr size_t IG_SMEM = INV_GROUP * IG_LD * sizeof(double);   // two workgroups per CU
+
+__global__ void __launch_bounds__(512, 4) k_inv_group(CholDev c, const int* __restrict__ tsn,
+                                                   const int* __restrict__ tix, Batch bt)
+{
+  extern __shared__ double smem[];
+  double (*Xs)[IG_LD] = reinterpret_cast<double (*)[IG_LD]>(smem);
+  double (*Ts)[IG_LD] = Xs + (INV_GROUP - BT);   // the last block's X is not read again
+  const int sy = batch_sys(bt);
+  if (sy < 0) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m16 = lane & 15, q4 = lane >> 4;
+  const int s = tsn[blockIdx.x], ix = tix[blockIdx.x], g = ix >> 5, cs = (ix & 31) * PW;
+  const SnInfo si = sninfo(c, batch_at(c.L, sy, bt), s);
+  const int g0 = g * INV_GROUP, ng = min(INV_GROUP, si.nc - g0), nb = (ng + BT - 1) / BT;
+  const int jb = cs / BT;
+  const int64_t ld = inv_ld(si.nc, g), f = si.f;
+  double* W = batch_at(c.dinv, sy, bt) + c.dinv_off[s] + static_cast<int64_t>(g) * INV_GROUP * INV_GROUP;
+#pragma unroll
+  for (int u = 0; u < BT * PW / 512; u++) {
+    const int r = BT * jb + (tid & (BT - 1)), cc = (tid >> 7) + 4 * u;
+    Xs[r][cc] = W[(cs + cc) * ld + r];
+  }
+  // acc += A X: this lane's row `row` of A (column-major, columns lda bytes apart) times
+  // X (K x 16, in LDS; K a multiple of 16), D steps' loads in flight
+  constexpr int D = 16;
+  auto product = [&](d4& acc, const double* A, int row, uint32_t lda, const double (*X)[IG_LD],
+                     int K) {
+    const rsrc_t ra = view(A, static_cast<int64_t>(K) * lda);
+    const uint32_t vo = static_cast<uint32_t>(row) * 8u + static_cast<uint32_t>(q4) * lda;
+    auto load = [&](int k) {
+      return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(
+                                            ra, vo, static_cast<uint32_t>(min(k, K - 4)) * lda, 0));
+    };
+    double a[D];
+#pragma unroll
+    for (int u = 0; u < D; u++) a[u] = load(4 * u);
+    for (int k0 = 0; k0 < K; k0 += 4 * D) {
+#pragma unroll
+      for (int u = 0; u < D; u++) {
+        const int k = k0 + 4 * u;
+        if (k >= K) break;
+        const double v = a[u];
+        a[u] = load(k + 4 * D);
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(X[k + q4][m16], v, acc, 0, 0, 0);
+      }
+    }
+  };
+  __syncthreads();
+  for (int ib = jb + 1; ib < nb; ib++) {
+    // rows past the supernode's columns repeat the last one; their X is 0
+    const int row = BT * ib + PW * w + m16;
+    d4 t = {0.0, 0.0, 0.0, 0.0};
+    product(t, si.Ls + (g0 + BT * jb) * f, min(g0 + row, si.nc - 1), static_cast<uint32_t>(f) * 8u,
+            Xs + BT * jb, BT * (ib - jb));
+#pragma unroll
+    for (int v = 0; v < 4; v++) Ts[PW * w + m16][4 * v + q4] = t[v];
+    __syncthreads();
+    d4 x = {0.0, 0.0, 0.0, 0.0};
+    product(x, W + BT * ib * ld, row, static_cast<uint32_t>(ld) * 8u, Ts, PW * (w + 1));
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      if (ib + 1 < nb) Xs[row][4 * v + q4] = -x[v];
+      if (row < ng) W[(cs + 4 * v + q4) * ld + row] = -x[v];
+    }
+    __syncthreads();
+  }
 }
 
 // L21 = A21 L_kk^{-T} for the rows below 128-wide diagonal block `step`, by
@@ -1230,7 +1311,8 @@ __global__ void __launch_bounds__(256) k_trsm(CholDev c, const int* __restrict__
   const int64_t f = si.f;
   const double* Lkk = si.Ls + static_cast<int64_t>(k0) * f + k0;   // L(k0 + r, k0 + c) at c*f + r
   double* A = si.Ls + static_cast<int64_t>(k0) * f + R0;            // A(row, col) at col*f + row
-  const double* W = batch_at(c.dinv, sy, bt) + c.dinv_off[s] + static_cast<int64_t>(step) * BT * BT;
+  const double* W = batch_at(c.dinv, sy, bt) + c.dinv_off[s] + inv_at(si.nc, step);
+  const int ldw = inv_ld(si.nc, k0 / INV_GROUP);
   const int np = (b + PW - 1) / PW;
   // stage: thread t holds entry (row t % 16, column t / 16) of every block;
   // rows at or past b (the panel rows below a partial block) read as 0.  All
@@ -1253,7 +1335,7 @@ __global__ void __launch_bounds__(256) k_trsm(CholDev c, const int* __restrict__
         v[t - t0] = in ? w : 0.0;
       } else {
         const int p = t - TRSM_NB;
-        v[t - t0] = W[static_cast<int64_t>(PW * p + cc) * BT + PW * p + rr];
+        v[t - t0] = W[static_cast<int64_t>(PW * p + cc) * ldw + PW * p + rr];
       }
     }
 #pragma unroll
@@ -1400,6 +1482,21 @@ void inv_blocks(const CholDev& c, int ntasks, const int* tsn, const int* tstep, 
   }();
   (void)attr;
   k_inv_blocks<<<dim3(ntasks, b.count), 256, SM, st>>>(c, tsn, tstep, b);
+  HIPCHK(hipGetLastError());
+}
+
+void inv_groups(const CholDev& c, int ntasks, const int* tsn, const int* tix, const Batch& b,
+                hipStream_t st)
+{
+  if (ntasks <= 0 || b.count <= 0) return;
+  static const bool attr = [] {
+    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_inv_group),
+                               hipFuncAttributeMaxDynamicSharedMemorySize,
+                               static_cast<int>(IG_SMEM)));
+    return true;
+  }();
+  (void)attr;
+  k_inv_group<<<dim3(ntasks, b.count), 512, IG_SMEM, st>>>(c, tsn, tix, b);
   HIPCHK(hipGetLastError());
 }
 

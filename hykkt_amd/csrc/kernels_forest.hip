@@ -28,7 +28,7 @@ namespace dev {
 namespace {
 
 constexpr int NT = 256;
-constexpr int SB = 128;          // edge of an inverted diagonal block's slot
+constexpr int SB = FRONT_NC;     // edge of an inverted diagonal block's slot
 constexpr int NC = FOREST_NC;
 constexpr int G = 8;             // columns per step of the unrolled loops
 
@@ -44,7 +44,7 @@ __device__ __forceinline__ double rl(double v, int j)
 struct Sn {
   int a, nc, nr, f;
   const double* L;   // panel, column-major, f rows
-  const double* W;   // inverted diagonal block, 128 rows
+  const double* W;   // inverted diagonal block, SB rows
   double* u;         // its forward update vector
   const int* pull_ptr;
   const int* rows;

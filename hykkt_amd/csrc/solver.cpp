@@ -29,7 +29,7 @@ struct Solver::Slots {
   int64_t dx = 0, dsv = 0, dyc = 0, dyd = 0;
   int64_t e_x = 0, e_s = 0, e_y = 0, e_d = 0, e_rxt = 0, e_ysc = 0, e_rxp = 0, e_schur = 0;
   int64_t e_cx = 0, c_dx = 0, c_dsv = 0, c_dyc = 0, c_dyd = 0;
-  int64_t L = 0, U = 0, dinv = 0, y = 0, ubuf = 0, bpart = 0;
+  int64_t L = 0, U = 0, dinv = 0, y = 0, ubuf = 0, exch = 0;
   int64_t stride = 0;
 };
 
@@ -446,7 +446,7 @@ void Solver::analyze()
   z.dinv = slot(cz.dinv);
   z.y = slot(cz.y);
   z.ubuf = slot(cz.ubuf);
-  z.bpart = slot(cz.bpart);
+  z.exch = slot(cz.exch);
   z.stride = at;
   S->cap = cap_;
   S->arena.alloc(static_cast<size_t>(z.stride) * cap_);
@@ -455,7 +455,7 @@ void Solver::analyze()
   S->flag_host.ensure(2 * static_cast<size_t>(cap_));
   double* base = S->arena.p;
   S->chol->bind(CholEngine::Storage{base + z.L, base + z.U, base + z.dinv, base + z.y,
-                                    base + z.ubuf, base + z.bpart, S->flags.p + FL_PIVOT * cap_},
+                                    base + z.ubuf, base + z.exch, S->flags.p + FL_PIVOT * cap_},
                 z.stride, cap_);
   HIPCHK(hipStreamSynchronize(st_));
 

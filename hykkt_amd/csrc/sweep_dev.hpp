@@ -31,7 +31,7 @@ struct SysBufs {
   const double* L;
   const double* dinv;
   double* ubuf;
-  double* bpart;
+  double* exch;
   const double* in;    // right-hand side (forward) or y (backward)
   double* out;         // y (forward) or x (backward)
 };
@@ -40,7 +40,7 @@ __device__ __forceinline__ SysBufs sys_bufs(const CholDev& c, const SolveDev& sd
                                             const Batch& bt, const double* in, double* out)
 {
   const int64_t o = static_cast<int64_t>(sy) * bt.vs;
-  return SysBufs{c.L + o, c.dinv + o, sd.ubuf + o, sd.bpart + o, in + o, out + o};
+  return SysBufs{c.L + o, c.dinv + o, sd.ubuf + o, sd.exch + o, in + o, out + o};
 }
 
 __device__ __forceinline__ double xload(const double* p)
@@ -78,15 +78,11 @@ __device__ double spin_load(const double* p, int* err)
 }
 
 // acc + (minus, NEG) the values at(0), .., at(n - 1), in that order, each once
-// its producer has written it.  Eight loads are in flight at a time: one after
-// the other they cost a round trip to the coherent level each (0.7 us), and a
-// pivot block of the backward sweep sums up to 60 row chunks' partials before
-// its chain can go on (top of the tree, backward: 10,000 buses 291 -> 269 us a
-// sweep, 20,000 650 -> 586).
-template <bool NEG, class AT>
+// its producer has written it.  U loads are in flight at a time: one after the
+// other they cost a round trip to the coherent level each (0.7 us).
+template <bool NEG, int U = 8, class AT>
 __device__ __forceinline__ double spin_sum(double acc, int n, AT at, int* err)
 {
-  constexpr int U = 8;
   for (int p0 = 0; p0 < n; p0 += U) {
     double v[U];
 #pragma unroll
@@ -131,6 +127,13 @@ __device__ __forceinline__ rsrc_t view(const double* base, uint32_t bytes)
 __device__ __forceinline__ double ld(rsrc_t r, uint32_t voff, uint32_t soff)
 {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
+}
+
+// Two consecutive values (any multiple of 8 bytes).
+typedef double d2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ d2v ld2(rsrc_t r, uint32_t voff, uint32_t soff)
+{
+  return __builtin_bit_cast(d2v, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
 }
 
 // Cross-lane sums of several values per lane.  Each exchange halves the values a
