@@ -25,6 +25,7 @@ namespace hykkt {
 namespace {
 constexpr int NB = 128;   // panel step, MFMA tile edge, solve block
 constexpr int SR = 32;    // rows of a short tile
+constexpr int TR = 64;    // rows of a short tile of the blocked TRSM
 constexpr int GMAX = 8;   // most steps one grouped trailing update can cover
 constexpr int U_SMALL_NC = 512;   // update matrices of at most so many columns take 64 x 64 tiles
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -230,8 +231,8 @@ void CholEngine::build_tasks()
 {
   // Launch shapes (see Tuning), counted over the tcount_ systems a launch
   // covers: a step whose TRSM has at most short_max tiles of 128 rows runs
-  // its TRSM and next-column update in 32-row tiles (four times the
-  // workgroups, each with a quarter of the work, for launches on the critical
+  // its TRSM in 64-row tiles and its next-column update in 32-row ones (more
+  // workgroups, each with less of the work, for launches on the critical
   // path); up to group_max consecutive steps share one trailing update with
   // K = G * NB (each C tile read and written once for the group) while that
   // update has at least pair_min * G^2 / 4 tiles of 128 x 128 beyond the G
@@ -346,14 +347,16 @@ void CholEngine::build_tasks()
       const bool last = gi == G - 1;   // the group's update of the columns after it
       L.potrf[j].off = static_cast<int>(potrf.size());
       L.trsm[j].off = static_cast<int>(trsm_sn.size());
-      int full_tiles = 0;
+      int full_tiles = 0, widest = 0;
       for (int q = b0; q < b1; q++) {
         const int s = pl_.level_sn[q];
         const int nc = pl_.nc(s), f = nc + pl_.nr(s), k0 = j * NB;
-        if (k0 < nc && !narrow(s)) full_tiles += cdiv(f - (k0 + std::min(NB, nc - k0)), NB);
+        if (k0 >= nc || narrow(s)) continue;
+        full_tiles += cdiv(f - (k0 + std::min(NB, nc - k0)), NB);
+        widest = std::max(widest, std::min(NB, nc - k0));
       }
       const bool shrt = full_tiles * tc <= tun_.short_max;
-      const int rows_unit = shrt ? SR : NB;
+      const int rows_unit = shrt ? (widest > 64 ? TR : SR) : NB;
       L.trsm[j].short_rows = shrt;
       L.upd_next[j].short_rows = shrt && !(last && G > 1);
       for (int q = b0; q < b1; q++) {
@@ -738,6 +741,15 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
     // enqueued.
     bool rest_pending = false;
     int rest_lo = INT_MAX;
+    // an update of up to five tiles of 128 x 128 per compute unit and K <= 512 takes
+    // 64 x 64 ones: more waves cover the loads of C, and the last ones end together
+    // (K = 128, 435 tiles: 50 -> 46 us; factor at 5,000 buses 2.99 -> 2.94 ms, 10,000
+    // 10.2 -> 9.8, 20,000 49.8 -> 48.8, 40,000 518 -> 516).  A larger one is better
+    // off with fewer operand loads (64 x 64 throughout, 20,000 buses: 53.4; for these
+    // launches at any K, 40,000: 520)
+    auto quarters = [&](const Launch& la, int kblk) {
+      return kblk <= 4 && static_cast<int64_t>(la.cnt) * b.count <= 5 * static_cast<int64_t>(n_cu_);
+    };
     for (size_t j = 0; j < L.potrf.size(); j++) {
       const int step = static_cast<int>(j);
       // in a group of G starting at step a: step a+i updates block column
@@ -777,7 +789,8 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
       timed(L.upd_next[j].short_rows ? PK_DENSE_NT_SHORT : PK_DENSE_NT, L.upd_next[j], [&] {
         dev::dense_nt(cd_, L.upd_next[j].cnt, t_upd_sn_.p + L.upd_next[j].off,
                       t_upd_tr_.p + L.upd_next[j].off, t_upd_tc_.p + L.upd_next[j].off, umode,
-                      ustep, b, st_, L.upd_next[j].short_rows, on_launch ? ev_main_ : nullptr);
+                      ustep, b, st_, L.upd_next[j].short_rows, on_launch ? ev_main_ : nullptr, false,
+                      quarters(L.upd_next[j], kblk));
       });
       if (rest) {
         if (!on_launch) HIPCHK(hipEventRecord(ev_main_, st_));
@@ -786,7 +799,8 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
           dev::dense_nt(cd_, L.upd_rest[j].cnt, t_upd_sn_.p + L.upd_rest[j].off,
                         t_upd_tr_.p + L.upd_rest[j].off, t_upd_tc_.p + L.upd_rest[j].off, umode,
                         ustep, b, st2_, false, ev_rest_,
-                        L.upd_rest[j].cnt * b.count <= 2 * n_cu_);   // all resident at once
+                        L.upd_rest[j].cnt * b.count <= 2 * n_cu_,   // all resident at once
+                        quarters(L.upd_rest[j], kblk));
         });
         rest_pending = true;
         rest_lo = std::min(rest_lo, upd_hi + 1);   // the rest starts after the columns just updated

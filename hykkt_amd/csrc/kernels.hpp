@@ -342,7 +342,7 @@ void extend_add(const CholDev& c, int ntasks, const int* task_p, const int* task
 void potrf_inv(const CholDev& c, int nsn, const int* sns, int step, int max_b, const Batch& b,
                hipStream_t st);
 // L21 = A21 L_kk^{-T} below the 128-wide diagonal blocks of step `step` by blocked
-// substitution (tasks: supernode, tile row of TM = 32 (short_rows) or 128 rows).
+// substitution (tasks: supernode, tile row of TM = 64 (short_rows) or 128 rows).
 void trsm(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr, int step,
           const Batch& b, hipStream_t st, bool short_rows);
 // The whole inverses of those blocks (tasks: supernode, step), same bits as formed
@@ -357,12 +357,13 @@ void inv_groups(const CholDev& c, int ntasks, const int* tsn, const int* tix, co
 // MFMA update tiles over (supernode, tile row, tile col) tasks.  mode 0: trailing
 // panel update after block `step`; mode m >= 3: after blocks `step` .. `step`+m-2
 // (K = (m-1) blocks).  Tiles of 128 x 128, or of 32 rows x 128 columns
-// (short_rows).  done: optional event
-// recorded by the launch's own completion.  alone: 128 x 128 tiles keep off a
-// compute unit that factors a 128-wide diagonal block.
+// (short_rows), or each 128 x 128 tile as four of 64 x 64 (quarters).  done: optional
+// event recorded by the launch's own completion.  alone: tiles keep off a compute
+// unit that factors a 128-wide diagonal block.
 void dense_nt(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr,
               const int* task_tc, int mode, int step, const Batch& b, hipStream_t st,
-              bool short_rows = false, hipEvent_t done = nullptr, bool alone = false);
+              bool short_rows = false, hipEvent_t done = nullptr, bool alone = false,
+              bool quarters = false);
 // The update matrices U = -L21 L21^T + the children's, tasks as above with tiles of
 // 128 x 128 (small: 64 x 64) entries of U.
 void update_matrices(const CholDev& c, int ntasks, const int* task_sn, const int* task_tr,

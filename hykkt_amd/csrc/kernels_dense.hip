@@ -261,8 +261,9 @@ __device__ __forceinline__ int child_words(const Sn& r, int t0, int lane)
 // in the panel, or return 0 past its end); K steps past K read 0 for both
 // operands.
 //
-// WN waves along the columns, TM / (16 IM) along the rows, on TM rows; a tile's 128 columns are
-// split over gridDim.z workgroups of 16 JN WN columns.  System blockIdx.y.
+// WN waves along the columns, TM / (16 IM) along the rows, on TM rows; a tile's 128
+// columns are split over gridDim.z workgroups of 16 JN WN columns (64 x 64 tiles: its
+// four quarters).  System blockIdx.y.
 // U: mode 1 (a kernel of its own, so that the others keep their registers).
 template <bool U, int TM, int IM, int JN, int WN, int D>
 __global__ void __launch_bounds__(TM / IM * WN * 4, TM / IM * WN / 32)
@@ -286,7 +287,10 @@ __global__ void __launch_bounds__(TM / IM * WN * 4, TM / IM * WN / 32)
   // end of the views: the panel's last entry and the one after it (the second
   // row of a pair; the storage goes on there)
   const double* panel_end = Ls + static_cast<int64_t>(f) * nc + 1;
-  const int zc = static_cast<int>(blockIdx.z) * TN;
+  // a workgroup's part of the task's tile: 64 x 64 tiles a quarter of 128 x 128
+  constexpr bool QUARTER = !U && TM == 64;
+  const int z = static_cast<int>(blockIdx.z);
+  const int zc = (QUARTER ? z & 1 : z) * TN, zr = QUARTER ? (z >> 1) * TM : 0;
   // this workgroup's rows and columns of the front (R0, C0), the first column
   // of the K range and K; M, N: valid rows and columns
   int R0, C0, ka, K, M, N;
@@ -300,12 +304,12 @@ __global__ void __launch_bounds__(TM / IM * WN * 4, TM / IM * WN / 32)
   } else {
     ka = step * BT;
     K = min(mode >= 3 ? (mode - 1) * BT : BT, nc - ka);
-    R0 = ka + K + tr * TM;
+    R0 = ka + K + tr * (QUARTER ? BT : TM) + zr;
     C0 = ka + K + tc * BT + zc;
     M = min(TM, f - R0);
     N = min(TN, nc - C0);
   }
-  if (M <= 0 || N <= 0) return;
+  if (M <= 0 || N <= 0 || (QUARTER && R0 + M <= C0)) return;
   const int m16 = lane & 15, q4 = lane >> 4;
   const int wr = (wave / WN) * QM, wc = (wave % WN) * QN;
   const uint32_t f8 = static_cast<uint32_t>(f) * 8u;
@@ -1279,19 +1283,21 @@ __global__ void __launch_bounds__(512, 4) k_inv_group(CholDev c, const int* __re
 // A wave owns 16-row groups; a group's X_q^T live in MFMA accumulators, whose
 // lane layout (element v = D[4v + l/16][l%16]) is the B operand's of k-step
 // v, so they feed the later panels' products without going through LDS.  The
-// 28 blocks L_pq (p > q) and the 8 inverses inv16(L_pp) are staged in LDS
-// first (each 16 x 16, column-major, in batches of loads), each panel's A
-// values are loaded while the one before is computed.  Few registers: a
-// 32-row tile fits beside two workgroups of the trailing update on one CU,
-// so the critical path's TRSM does not wait for them to drain.  TM rows per tile (32 or 128: 2 or 8
-// groups); every row takes the same operations in the same order whatever
-// the tile, so both shapes give the same bits.  In place.  System blockIdx.y.
+// 28 blocks L_pq (p > q) and the 8 inverses inv16(L_pp) are staged in LDS first (each
+// 16 x 16, column-major), and A is loaded panels ahead of its use: beside a trailing
+// update a load takes several times its time alone.  Few registers: a 64-row tile
+// fits beside two workgroups of the trailing update on one CU, so the critical path's
+// TRSM does not wait for them to drain.  TM rows per tile (64 or 128: 4 or 8 groups);
+// every row takes the same operations in the same order whatever the tile, so both
+// shapes give the same bits.  One 4,284-column supernode (5,000 buses), mean of its
+// steps beside the trailing updates: 32-row tiles with one panel ahead 19.2 us, now
+// 15.7.  In place.  System blockIdx.y.
 constexpr int TRSM_NB = (BT / PW) * (BT / PW - 1) / 2;   // blocks L_pq, p > q
 constexpr size_t TRSM_SMEM = (TRSM_NB + BT / PW) * PW * PW * sizeof(double);
 
 template <int TM>
-__global__ void __launch_bounds__(256) k_trsm(CholDev c, const int* __restrict__ tsn,
-                                              const int* __restrict__ ttr, int step, Batch bt)
+__global__ void __launch_bounds__(256, TM == 64 ? 4 : 1)
+    k_trsm(CholDev c, const int* __restrict__ tsn, const int* __restrict__ ttr, int step, Batch bt)
 {
   __builtin_amdgcn_s_setprio(3);   // the critical chain: issue priority (see k_dense_nt)
   constexpr int NG = TM / 16, NGW = (NG + 3) / 4;   // groups, groups per wave
@@ -1314,67 +1320,75 @@ __global__ void __launch_bounds__(256) k_trsm(CholDev c, const int* __restrict__
   const double* W = batch_at(c.dinv, sy, bt) + c.dinv_off[s] + inv_at(si.nc, step);
   const int ldw = inv_ld(si.nc, k0 / INV_GROUP);
   const int np = (b + PW - 1) / PW;
-  // stage: thread t holds entry (row t % 16, column t / 16) of every block;
-  // rows at or past b (the panel rows below a partial block) read as 0.  All
-  // loads are issued before the first LDS store.
-  {
-    const int rr = threadIdx.x % PW, cc = threadIdx.x / PW;
-    constexpr int NBAT = 9;   // loads in flight per batch
-#pragma unroll
-    for (int t0 = 0; t0 < TRSM_NB + NPN; t0 += NBAT) {
-    double v[NBAT];
-#pragma unroll
-    for (int t = t0; t < t0 + NBAT; t++) {
-      if (t < TRSM_NB) {
-        int p = 1;
-        while ((p + 1) * p / 2 <= t) p++;   // compile-time after unrolling
-        const int q = t - p * (p - 1) / 2;
-        const int row = PW * p + rr;
-        const bool in = p < np && row < b;
-        const double w = Lkk[in ? static_cast<int64_t>(PW * q + cc) * f + row : 0];
-        v[t - t0] = in ? w : 0.0;
-      } else {
-        const int p = t - TRSM_NB;
-        v[t - t0] = W[static_cast<int64_t>(PW * p + cc) * ldw + PW * p + rr];
-      }
-    }
-#pragma unroll
-    for (int t = t0; t < t0 + NBAT; t++) smem[t * PW * PW + threadIdx.x] = v[t - t0];
-    }
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
   const int i16 = lane & 15, k4 = lane >> 4;
-  int grow[NGW];   // first row of each of this wave's groups (-1: none)
+  const uint32_t f8 = static_cast<uint32_t>(f) * 8u, w8 = static_cast<uint32_t>(ldw) * 8u;
+  auto load = [](rsrc_t v, uint32_t vo, uint32_t so) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(v, vo, so, 0));
+  };
+  // A_p^T of each group, into the place of X_p^T: element v = A(row i16, column 16p + 4v
+  // + k4), at byte va of view(A) and the column quadruple's uniform offset; rows and
+  // columns past the end are off the view (they read 0 and are not stored)
+  d4 x[NGW][NPN];
+  const rsrc_t av = view(A, static_cast<int64_t>(b) * f8);
+  const int last4 = (b - 1) / 4;   // the last column quadruple, perhaps partial
+  uint32_t va[NGW], vlast[NGW];
 #pragma unroll
   for (int gi = 0; gi < NGW; gi++) {
-    const int g = wave + 4 * gi;
-    grow[gi] = (g < NG && g * 16 < M) ? g * 16 : -1;
+    const int g = wave + 4 * gi, row = 16 * g + i16;
+    va[gi] = g < NG && row < M
+                 ? static_cast<uint32_t>(row) * 8u + static_cast<uint32_t>(k4) * f8 : OFF_NONE;
+    vlast[gi] = 4 * last4 + k4 < b ? va[gi] : OFF_NONE;
   }
-  if (grow[0] < 0) return;   // no barrier follows
-  // A_p^T of each group: element v = A(row i16, column 16p + 4v + k4)
-  auto load_a = [&](int p, d4 (&a)[NGW]) {
+  auto off_a = [&](int gi, int q) { return q < last4 ? va[gi] : q == last4 ? vlast[gi] : OFF_NONE; };
+  // stage: thread t holds entry (row t % 16, column t / 16) of every block, NBAT loads in
+  // flight together; rows at or past b (the panel rows below a partial block) and blocks
+  // past it read as 0
+  {
+    const int rr = threadIdx.x % PW, cc = threadIdx.x / PW, nfull = b / PW;
+    const rsrc_t vl = view(Lkk, static_cast<int64_t>(b) * f8), vw = view(W, static_cast<int64_t>(BT) * w8);
+    const uint32_t full = static_cast<uint32_t>(rr) * 8u + static_cast<uint32_t>(cc) * f8;
+    const uint32_t part = rr < b - PW * nfull ? full : OFF_NONE;
+    const uint32_t wo = static_cast<uint32_t>(rr) * 8u + static_cast<uint32_t>(cc) * w8;
+    constexpr int NBAT = 18;
 #pragma unroll
-    for (int gi = 0; gi < NGW; gi++) {
-      const int row = grow[gi] + i16;
+    for (int t0 = 0; t0 < TRSM_NB + NPN; t0 += NBAT) {
+      double v[NBAT];
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int col = PW * p + 4 * v + k4;
-        a[gi][v] = (grow[gi] >= 0 && row < M && col < b) ? A[col * f + row] : 0.0;
+      for (int t = t0; t < t0 + NBAT; t++) {
+        int p = 1;
+        while ((p + 1) * p / 2 <= t) p++;   // compile-time after unrolling
+        const int q = t - p * (p - 1) / 2, pi = t - TRSM_NB;
+        v[t - t0] = t < TRSM_NB
+                        ? load(vl, p < nfull ? full : p == nfull ? part : OFF_NONE,
+                               static_cast<uint32_t>(PW * p) * 8u + static_cast<uint32_t>(PW * q) * f8)
+                        : load(vw, pi < np ? wo : OFF_NONE, static_cast<uint32_t>(PW * pi) * (8u + w8));
       }
+#pragma unroll
+      for (int t = t0; t < t0 + NBAT; t++) smem[t * PW * PW + threadIdx.x] = v[t - t0];
     }
+  }
+  // A of the panels ahead, in their X's registers: five for one group a wave (112
+  // registers in all), the next one for two
+  constexpr int AHEAD = NGW == 1 ? 5 : 1;
+  auto load_a = [&](int p) {
+#pragma unroll
+    for (int gi = 0; gi < NGW; gi++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        x[gi][p][v] = load(av, off_a(gi, 4 * p + v), static_cast<uint32_t>(PW * p + 4 * v) * f8);
   };
-  d4 x[NGW][NPN];
-  d4 an[NGW];
-  load_a(0, an);
+#pragma unroll
+  for (int p = 0; p < AHEAD; p++) load_a(p);
+  __syncthreads();
+  if (PW * wave >= M) return;   // no barrier follows
 #pragma unroll
   for (int p = 0; p < NPN; p++) {
     if (p >= np) break;
     d4 acc[NGW];
 #pragma unroll
-    for (int gi = 0; gi < NGW; gi++) acc[gi] = an[gi];
-    if (p + 1 < np) load_a(p + 1, an);
+    for (int gi = 0; gi < NGW; gi++) acc[gi] = x[gi][p];
+    if (p + AHEAD < NPN) load_a(p + AHEAD);
     // - sum_{q<p} L_pq X_q^T: A operand -L(16p + i16, 16q + 4 s4 + k4)
 #pragma unroll
     for (int q = 0; q < NPN; q++) {
@@ -1401,13 +1415,11 @@ __global__ void __launch_bounds__(256) k_trsm(CholDev c, const int* __restrict__
     }
 #pragma unroll
     for (int gi = 0; gi < NGW; gi++) {
-      if (p + 1 < NPN) x[gi][p] = r[gi];   // the last panel's X is not read again
-      const int row = grow[gi] + i16;
+      x[gi][p] = r[gi];
 #pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const int col = PW * p + 4 * v + k4;
-        if (grow[gi] >= 0 && row < M && col < b) A[col * f + row] = r[gi][v];
-      }
+      for (int v = 0; v < 4; v++)
+        if (off_a(gi, 4 * p + v) != OFF_NONE)
+          A[(PW * p + 4 * v + k4) * f + 16 * (wave + 4 * gi) + i16] = r[gi][v];
     }
   }
 }
@@ -1427,7 +1439,7 @@ constexpr size_t ALONE_LDS = 31 * 1024;
 
 void dense_nt(const CholDev& c, int ntasks, const int* tsn, const int* ttr, const int* ttc,
               int mode, int step, const Batch& b, hipStream_t st, bool short_rows, hipEvent_t done,
-              bool alone)
+              bool alone, bool quarters)
 {
   if (ntasks <= 0 || b.count <= 0) return;
   // `done` rides on the launch itself (its completion signal), so no marker
@@ -1435,6 +1447,9 @@ void dense_nt(const CholDev& c, int ntasks, const int* tsn, const int* ttr, cons
   if (short_rows)
     hipExtLaunchKernelGGL((k_dense_nt<false, 32, 2, 1, 4, 8>), dim3(ntasks, b.count, BT / SHORT_TN),
                           dim3(256), 0, st, nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
+  else if (quarters)
+    hipExtLaunchKernelGGL((k_dense_nt<false, 64, 2, 2, 2, 4>), dim3(ntasks, b.count, 4), dim3(256),
+                          alone ? ALONE_LDS : 0, st, nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
   else
     hipExtLaunchKernelGGL((k_dense_nt<false, 128, 4, 4, 2, 2>), dim3(ntasks, b.count), dim3(256),
                           alone ? ALONE_LDS : 0, st, nullptr, done, 0, c, tsn, ttr, ttc, mode, step, b);
@@ -1505,7 +1520,7 @@ void trsm(const CholDev& c, int ntasks, const int* tsn, const int* ttr, int step
 {
   if (ntasks <= 0 || b.count <= 0) return;
   static const bool attr = [] {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_trsm<32>),
+    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_trsm<64>),
                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                static_cast<int>(TRSM_SMEM)));
     HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_trsm<128>),
@@ -1515,7 +1530,7 @@ void trsm(const CholDev& c, int ntasks, const int* tsn, const int* ttr, int step
   }();
   (void)attr;
   const dim3 grid(ntasks, b.count);
-  if (short_rows) k_trsm<32><<<grid, 256, TRSM_SMEM, st>>>(c, tsn, ttr, step, b);
+  if (short_rows) k_trsm<64><<<grid, 256, TRSM_SMEM, st>>>(c, tsn, ttr, step, b);
   else k_trsm<128><<<grid, 256, TRSM_SMEM, st>>>(c, tsn, ttr, step, b);
   HIPCHK(hipGetLastError());
 }
