@@ -430,7 +430,10 @@ __global__ void __launch_bounds__(TM / IM * WN * 4, TM / IM * WN / 32)
             double x[VG][IM];
 #pragma unroll
             for (int v = 0; v < VG; v++) {
-              const int b = ib[g][j][v0 + v];
+              int b = ib[g][j][v0 + v];
+              // 128 x 128: a column's address is formed in its turn, and its sums before the
+              // next one's loads; held beside the accumulators they spilled 31 registers
+              if constexpr (CG == 1) asm volatile("" : "+v"(b));
               const double* col = uc + packed_lower(0, b < n ? b : 0, n);
               // on or below the child's diagonal; the others read the column's first
 #pragma unroll
@@ -442,6 +445,9 @@ __global__ void __launch_bounds__(TM / IM * WN * 4, TM / IM * WN / 32)
               for (int i = 0; i < IM; i++)
                 acc[i][j][v0 + v] = ia[g][i] >= ib[g][j][v0 + v] ? acc[i][j][v0 + v] + x[v][i]
                                                                  : acc[i][j][v0 + v];
+            if constexpr (CG == 1)
+#pragma unroll
+              for (int i = 0; i < IM; i++) asm volatile("" : "+v"(acc[i][j]) : : "memory");
           }
       }
     }
@@ -1340,7 +1346,10 @@ __global__ void __launch_bounds__(256, TM == 64 ? 4 : 1)
                  ? static_cast<uint32_t>(row) * 8u + static_cast<uint32_t>(k4) * f8 : OFF_NONE;
     vlast[gi] = 4 * last4 + k4 < b ? va[gi] : OFF_NONE;
   }
-  auto off_a = [&](int gi, int q) { return q < last4 ? va[gi] : q == last4 ? vlast[gi] : OFF_NONE; };
+  auto off_a = [&](int gi, int q) {
+    const uint32_t full = va[gi], last = vlast[gi];   // values: chosen by address they are in scratch
+    return q < last4 ? full : q == last4 ? last : OFF_NONE;
+  };
   // stage: thread t holds entry (row t % 16, column t / 16) of every block, NBAT loads in
   // flight together; rows at or past b (the panel rows below a partial block) and blocks
   // past it read as 0

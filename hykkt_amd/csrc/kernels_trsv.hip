@@ -214,12 +214,12 @@ __device__ __forceinline__ void fwd_below(const CholDev& c, const SolveDev& sd, 
         l[k] = ld2(L, static_cast<uint32_t>(r) * 8u,
                    static_cast<uint32_t>(min(at + k, si.nc - 1) - c0) * f8);
     };
-    if (wk * FC < si.nc) load(0);
+    load(0);
     // the children's entries in the item's rows, a row a thread (from this set's first on)
     const int t = threadIdx.x;
     if (t < NW / wc * RW && i0 + t < si.f) pull[t] = pulled(sd, B, s, 0.0, i0 + t);
-    for (int c0 = 0; c0 + wk * FC < si.nc; c0 += wc * FC) {
-      const int at = c0 + wk * FC, kv = min(si.nc - at, FC);
+    for (int c0 = 0, at = wk * FC; at < si.nc;) {
+      const int kv = min(si.nc - at, FC);
       const double yv = lane < kv ? spin_load(B.out + si.a + at + lane, sd.err) : 0.0;
 #pragma unroll
       for (int k = 0; k < FC; k++) {
@@ -228,7 +228,13 @@ __device__ __forceinline__ void fwd_below(const CholDev& c, const SolveDev& sd, 
         acc[0] += l[k][0] * yk;
         acc[1] += l[k][1] * yk;
       }
-      if (at + wc * FC < si.nc) load(c0 + wc * FC);
+      // the sums before the next slice's loads: after them they would keep both slices
+      // in registers (and 84 bytes a lane in scratch)
+      asm volatile("" : "+v"(acc[0]), "+v"(acc[1]) : : "memory");
+      c0 += wc * FC;
+      at += wc * FC;
+      if (at >= si.nc) break;
+      load(c0);
     }
   }
   *reinterpret_cast<d2v*>(&part[w][2 * lane]) = acc;
