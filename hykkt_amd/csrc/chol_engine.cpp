@@ -322,6 +322,7 @@ void CholEngine::build_tasks()
     // column update).  Single steps (G = 1) update after their own block.
     L.gpos.assign(nsteps, 0);
     L.gsize.assign(nsteps, 1);
+    L.upd_whole.assign(nsteps, 0);
     for (int j = 0; j < nsteps;) {
       int G = 1;
       for (int g = std::min(gmax, nsteps - j); g >= 2 && G == 1; g--) {
@@ -348,17 +349,30 @@ void CholEngine::build_tasks()
       L.potrf[j].off = static_cast<int>(potrf.size());
       L.trsm[j].off = static_cast<int>(trsm_sn.size());
       int full_tiles = 0, widest = 0;
+      int64_t upd_tiles = 0;   // of 128 x 128
       for (int q = b0; q < b1; q++) {
         const int s = pl_.level_sn[q];
         const int nc = pl_.nc(s), f = nc + pl_.nr(s), k0 = j * NB;
         if (k0 >= nc || narrow(s)) continue;
-        full_tiles += cdiv(f - (k0 + std::min(NB, nc - k0)), NB);
+        const int rt = cdiv(f - (k0 + std::min(NB, nc - k0)), NB);
+        const int ct = cdiv(nc - (k0 + std::min(NB, nc - k0)), NB);
+        full_tiles += rt;
+        upd_tiles += static_cast<int64_t>(ct) * rt - static_cast<int64_t>(ct) * (ct - 1) / 2;
         widest = std::max(widest, std::min(NB, nc - k0));
       }
       const bool shrt = full_tiles * tc <= tun_.short_max;
       const int rows_unit = shrt ? (widest > 64 ? TR : SR) : NB;
       L.trsm[j].short_rows = shrt;
-      L.upd_next[j].short_rows = shrt && !(last && G > 1);
+      // A step whose whole update is at most a tile of 128 x 128 per four compute units
+      // takes it in one launch on the main stream: beside the diagonal block the rest
+      // costs an event on each stream, 11 us a step, more than this update's own time
+      // (1,000 buses: 1222 -> 1176 us a solve, 500 1125 -> 1098, 5,000 3738 -> 3707; up
+      // to one tile per compute unit 5,000 takes 3797).  32-row tiles up to one per
+      // eight (64 x 64 tiles instead: 1185, 1113).
+      const bool whole = G == 1 && upd_tiles * tc <= n_cu_ / 4;
+      L.upd_whole[j] = whole;
+      const bool ushrt = whole ? upd_tiles * tc <= n_cu_ / 8 : shrt && !(last && G > 1);
+      L.upd_next[j].short_rows = ushrt;
       for (int q = b0; q < b1; q++) {
         const int s = pl_.level_sn[q];
         const int nc = pl_.nc(s), f = nc + pl_.nr(s);
@@ -377,7 +391,7 @@ void CholEngine::build_tasks()
         L.potrf[j].bytes += 16.0 * tri;
         L.trsm[j].flops += r * db * db;
         L.trsm[j].bytes += 8.0 * (2 * r * db + tri);
-        // the update splits into the next block column (tile column 0) and
+        // the update, unless whole, splits into the next block column (tile column 0) and
         // the rest, so the next step can start before the rest is done.  In a
         // group, an inner step updates the next block column by the group's
         // blocks so far (K = kw) and the last step the columns after the group
@@ -399,7 +413,10 @@ void CholEngine::build_tasks()
           const double pn = cn * r - cn * (cn - 1) / 2;
           L.upd_next[j].flops += 2.0 * dk * pn;
           L.upd_next[j].bytes += 8.0 * (r * dk + 2 * pn);
-          if (G == 1) {
+          if (whole) {
+            L.upd_next[j].flops += 2.0 * db * (pairs - pn);
+            L.upd_next[j].bytes += 8.0 * 2 * (pairs - pn);
+          } else if (G == 1) {
             L.upd_rest[j].flops += 2.0 * db * (pairs - pn);
             L.upd_rest[j].bytes += 8.0 * 2 * (pairs - pn);
           }
@@ -433,18 +450,12 @@ void CholEngine::build_tasks()
             continue;
           }
           const int b = std::min(NB, nc - k0);
-          const int rtiles = cdiv(f - (k0 + b), NB), ctiles = cdiv(nc - (k0 + b), NB);
-          if (part == 0 && shrt) {   // next block column in 32-row tiles
-            if (ctiles > 0)
-              for (int tr = 0; tr < cdiv(f - (k0 + b), SR); tr++) {
-                upd_sn.push_back(s);
-                upd_tr.push_back(tr);
-                upd_tc.push_back(0);
-              }
-            continue;
-          }
-          for (int tc = part == 0 ? 0 : 1; tc < (part == 0 ? std::min(1, ctiles) : ctiles); tc++)
-            for (int tr = tc; tr < rtiles; tr++) {
+          const int ctiles = cdiv(nc - (k0 + b), NB);
+          const int tc0 = part == 0 ? 0 : whole ? ctiles : 1;
+          const int tc1 = part == 0 && !whole ? std::min(1, ctiles) : ctiles;
+          const int unit = part == 0 && ushrt ? SR : NB;   // 32-row tiles
+          for (int tc = tc0; tc < tc1; tc++)
+            for (int tr = tc * (NB / unit); tr < cdiv(f - (k0 + b), unit); tr++) {
               upd_sn.push_back(s);
               upd_tr.push_back(tr);
               upd_tc.push_back(tc);
@@ -760,7 +771,7 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
       const bool last = gi == G - 1;
       const int kblk = last ? G : gi + 1;
       const int umode = kblk == 1 ? 0 : kblk + 1, ustep = a;
-      const int upd_hi = (last && G > 1) ? step + G : step + 1;
+      const int upd_hi = L.upd_whole[j] ? INT_MAX : (last && G > 1) ? step + G : step + 1;
       timed(PK_POTRF, L.potrf[j], [&] {
         dev::potrf_inv(cd_, L.potrf[j].cnt, t_potrf_.p + L.potrf[j].off, step, L.potrf[j].maxb, b,
                        st_);

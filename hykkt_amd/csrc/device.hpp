@@ -185,6 +185,7 @@ class CholEngine {
     // per step: its position in its group of consecutive steps and the
     // group's size (1: the step updates after its own block; see build_tasks)
     std::vector<int> gpos, gsize;
+    std::vector<char> upd_whole;   // upd_next has all the step's columns, upd_rest none
   };
   void build_fronts();
   void build_tasks();
