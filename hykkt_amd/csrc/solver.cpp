@@ -27,7 +27,8 @@ struct Solver::Slots {
   int64_t cx = 0, cr = 0, cw = 0, cp = 0, cs = 0, schur = 0, sc = 0, part = 0, part2 = 0, rpart = 0;
   int64_t h0 = 0, cq = 0, cz = 0;
   int64_t dx = 0, dsv = 0, dyc = 0, dyd = 0;
-  int64_t e_x = 0, e_s = 0, e_y = 0, e_d = 0, e_rxt = 0, e_ysc = 0, e_rxp = 0, e_schur = 0;
+  Rows e[2];   // residual rows: a pass's, and the ones the next pass corrects
+  int64_t e_rxt = 0, e_ysc = 0, e_rxp = 0, e_schur = 0;
   int64_t e_cx = 0, c_dx = 0, c_dsv = 0, c_dyc = 0, c_dyd = 0;
   int64_t L = 0, U = 0, dinv = 0, y = 0, ubuf = 0, exch = 0;
   int64_t stride = 0;
@@ -427,10 +428,7 @@ void Solver::analyze()
   z.dsv = slot(d);
   z.dyc = slot(m);
   z.dyd = slot(d);
-  z.e_x = slot(n);
-  z.e_s = slot(d);
-  z.e_y = slot(m);
-  z.e_d = slot(d);
+  for (Rows& e : z.e) e = Rows{slot(n), slot(d), slot(m), slot(d)};
   z.e_rxt = slot(n);
   z.e_ysc = slot(m);
   z.e_rxp = slot(n);
@@ -778,7 +776,7 @@ std::vector<int> Solver::run(int count, bool from_setters)
   // CG start y_host, or zero when none is bound (then no start-residual solve)
   const Solution sol{z.dx, z.dsv, z.dyc, z.dyd}, none{-1, -1, -1, -1};
   solve_pass(Pass{z.rxp, z.schur, z.cx}, z.rx_til, z.ry_s, z.in[IN_RS], z.in[IN_RYD], any_y0, sol,
-             none, dev::masked(b, S.flag(FL_OK)), b, last_iters_, true);
+             none, z.e[0], dev::masked(b, S.flag(FL_OK)), b, last_iters_, true);
   std::vector<int> zrow(count), piv(count);
   std::vector<int> rc(count, HYKKT_OK);
   std::vector<double> nb(count);
@@ -835,24 +833,25 @@ std::vector<int> Solver::run(int count, bool from_setters)
                             st_));
       ba = dev::masked(b, S.flag(FL_ACT));
     }
+    const Rows& e = z.e[pass & 1];
     if (S.has_jd) {
-      dev::row_scale(d, S.jd_rp.p, in[IN_JD], in[IN_DS], P(z.e_d), P(z.e_s), nullptr, P(z.ryd_s),
-                     ba, st_);
+      dev::row_scale(d, S.jd_rp.p, in[IN_JD], in[IN_DS], P(e.d), P(e.s), nullptr, P(z.ryd_s), ba,
+                     st_);
       timed(PK_SPMV, 2.0 * S.nnz_jd, spmv_bytes(n, d, S.nnz_jd, true, true, false), ba, [&] {
         dev::spmv(n, S.jdt_rp.p, S.jdt_ci.p, S.jdt_map.p, in[IN_JD], 1.0, nullptr, P(z.ryd_s),
-                  1.0, P(z.e_x), P(z.e_rxt), S.jdt_blk.p, S.jdt_nblk, ba, st_);
+                  1.0, P(e.x), P(z.e_rxt), S.jdt_blk.p, S.jdt_nblk, ba, st_);
       });
     } else {
-      dev::copy(P(z.e_rxt), P(z.e_x), n, ba, st_);
+      dev::copy(P(z.e_rxt), P(e.x), n, ba, st_);
     }
     dev::vec_scale(P(z.e_rxt), P(z.max_d), n, ba, st_);
-    dev::copy(P(z.e_ysc), P(z.e_y), m, ba, st_);
+    dev::copy(P(z.e_ysc), P(e.y), m, ba, st_);
     dev::vec_scale(P(z.e_ysc), P(z.max_d) + n, m, ba, st_);
     // the correction's right-hand side is small: its CG usually stops within
     // an iteration or two, so its first look at the live flags comes from
     // the last refinement pass, not the first pass
-    solve_pass(corr, z.e_rxt, z.e_ysc, z.e_s, z.e_d, false, csol, sol, ba, ba, last_ref_iters_,
-               false);
+    solve_pass(corr, z.e_rxt, z.e_ysc, e.s, e.d, false, csol, sol, z.e[(pass + 1) & 1], ba, ba,
+               last_ref_iters_, false);
     int rit = 0;
     for (int k = 0; k < count; k++)
       if (act[k]) rit = std::max(rit, cg_result(fin(k)).iters);
@@ -930,8 +929,8 @@ std::vector<int> Solver::run(int count, bool from_setters)
 // the usual pass has one host round trip and no iteration that nobody needs.  If
 // a system is still live, the CG goes on and they run again.
 void Solver::solve_pass(const Pass& w, int64_t rxt, int64_t ysc, int64_t rs, int64_t ryd, bool x0,
-                        const Solution& out, const Solution& base, const dev::Batch& bs,
-                        const dev::Batch& br, int hint, bool first)
+                        const Solution& out, const Solution& base, const Rows& rows,
+                        const dev::Batch& bs, const dev::Batch& br, int hint, bool first)
 {
   Sym& S = *sym_;
   const Slots& z = S.z;
@@ -1026,10 +1025,10 @@ void Solver::solve_pass(const Pass& w, int64_t rxt, int64_t ysc, int64_t rs, int
   res.dsv = rec.dsv;
   res.dyc = rec.dyc;
   res.dyd = rec.dyd;
-  res.e_x = P(z.e_x);
-  res.e_s = P(z.e_s);
-  res.e_y = P(z.e_y);
-  res.e_d = P(z.e_d);
+  res.e_x = P(rows.x);
+  res.e_s = P(rows.s);
+  res.e_y = P(rows.y);
+  res.e_d = P(rows.d);
   res.part = P(z.rpart);
   dev::Finish fin{};
   fin.out = S.fin.p;

@@ -92,11 +92,15 @@ class Solver {
   struct Solution {
     int64_t dx, dsv, dyc, dyd;
   };
-  // CG, recovery (into out, onto base unless its offsets are -1) and residual;
-  // synchronizes and leaves each system's FIN_SLOTS results in Sym::fin.
+  struct Rows {
+    int64_t x = 0, s = 0, y = 0, d = 0;
+  };
+  // CG, recovery (into out, onto base unless its offsets are -1) and residual (into
+  // rows, which may not be rs or ryd: both may run several times); synchronizes and
+  // leaves each system's FIN_SLOTS results in Sym::fin.
   void solve_pass(const Pass& w, int64_t rxt, int64_t ysc, int64_t rs, int64_t ryd, bool x0,
-                  const Solution& out, const Solution& base, const dev::Batch& bs,
-                  const dev::Batch& br, int hint, bool first);
+                  const Solution& out, const Solution& base, const Rows& rows,
+                  const dev::Batch& bs, const dev::Batch& br, int hint, bool first);
   double* P(int64_t off) const;   // system 0's address of an arena slot
   // Run the launch in fn bracketed for the profiler, charged with the work
   // of the b.count systems it covers.
