@@ -743,10 +743,17 @@ void CholEngine::build_solve()
   dev::fill_i(flags_.p, 0, 1, st_);
 }
 
+// Zeros in the factor storage of b's systems.  The first clean_ ones have them from
+// prezero_L, whose fill may still be in flight on the second stream: whatever
+// follows waits for it, also when this call has more systems, or it would zero
+// entries that were assembled meanwhile.
 void CholEngine::zero_L(const dev::Batch& b)
 {
-  if (b.count <= clean_) HIPCHK(hipStreamWaitEvent(st_, ev_zero_, 0));
-  else dev::fill(cd_.L, 0.0, pl_.l_off[pl_.ns], b, st_);
+  const int have = std::min(clean_, b.count);
+  if (clean_ > 0) HIPCHK(hipStreamWaitEvent(st_, ev_zero_, 0));
+  if (have < b.count)
+    dev::fill(cd_.L + have * b.vs, 0.0, pl_.l_off[pl_.ns],
+              dev::Batch{b.count - have, b.vs, b.mask ? b.mask + have : nullptr}, st_);
   clean_ = 0;
 }
 
