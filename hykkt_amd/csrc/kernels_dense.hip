@@ -791,13 +791,19 @@ __device__ __forceinline__ void potrf_factor(double (*P)[BK + 1], double* rd, in
     for (int p = 0; p < panels; p++) {
       const int kb = p * PW;
       const int nf = max(1, (BK - kb - PW + 47) / 48);   // factoring waves
+      double v[PW];
+      const int r = kb + prow_off;
       if (wave < nf) {
-        const int r = kb + prow_off;
-        const bool mine = r < BK && (dg ? wave == 0 : true);   // this lane stores row r
         const int rr = min(r, BK - 1);
-        double v[PW];
 #pragma unroll
         for (int q = 0; q < PW; q++) v[q] = P[rr][kb + q];
+      }
+      // every factoring wave has read the diagonal block before wave 0 stores its factor
+      // there: a wave may lag the others by more than a pass where work of other
+      // streams shares its SIMD
+      if (nf > 1) __syncthreads();
+      if (wave < nf) {
+        const bool mine = r < BK && (dg ? wave == 0 : true);   // this lane stores row r
         double myinv = 1.0;   // 1 / L(kb + lane, kb + lane), taken at step k == lane
 #pragma unroll
         for (int k = 0; k < PW; k++) {
