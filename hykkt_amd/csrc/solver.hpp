@@ -122,10 +122,10 @@ class Solver {
   int vec_n_[8] = {};
   std::vector<SystemIn> sys_in_;
   std::vector<hykkt_stats> st_k_;
-  // CG iterations of the last first pass and of the last refinement pass:
-  // where the host first looks at the live flags in the next such pass
-  int last_iters_ = 0;
-  int last_ref_iters_ = 0;
+  // CG iterations of the last first pass and of the last refinement pass (-1: none
+  // yet): where the host first looks at the live flags in the next such pass
+  int last_iters_ = -1;
+  int last_ref_iters_ = -1;
   hykkt_tuning tuning_{};
   // file-path storage (read_matrix_files)
   CsrHost fblk_[4];

@@ -64,3 +64,36 @@ def test_batch_of_unequal_iterations(every):
             assert rc[k] == ref[0] == H.HYKKT_OK
             same(b.stats_k(k), np.concatenate(b.solution_k(k)), ref)
         rc = b.execute_batch(len(systems))
+
+
+@pytest.mark.parametrize("every", [0, 1])
+def test_early_looks_run_no_recovery(every):
+    """Looks at a CG that is not done read its live flags alone: at most two recoveries
+    and residuals a pass (k_spmv in the profile has both, and the products)."""
+    g = GridPattern(203, 263, seed=11)
+    sy = g.system(0, ds_range=(1e-4, 1e8))
+    sy.gamma = 1e1
+    opts = dict(refine_max=0, cg_check_every=every)
+    _, st, _, s = alone(g, sy, **opts)
+    assert st["cg_iters"] > 10
+    for _ in range(2):
+        s.profile(True)
+        s.execute()
+        n = s.kernel_times()["k_spmv"]["launches"]
+        # Jd^T, Jc^T and Jc once, and both Jc products per iteration
+        assert 2 <= n - (3 + 2 * s.stats()["cg_iters"]) <= 4
+        s.profile(False)
+    # a fresh pattern, whose iteration count is not known
+    s = H.HykktSolver(sy.gamma)
+    s.options(**opts)
+    s.profile(True)
+    d = g.d
+    s.set_H(sy.H.rp, sy.H.ci, sy.H.v, g.n, g.n, g.H.nnz)
+    s.set_Ds(np.arange(d + 1), np.arange(d), sy.Ds.v, d, d, d)
+    s.set_Jc(sy.Jc.rp, sy.Jc.ci, sy.Jc.v, g.m, g.n, g.Jc.nnz)
+    s.set_Jd(sy.Jd.rp, sy.Jd.ci, sy.Jd.v, g.d, g.n, g.Jd.nnz)
+    for name in ("rx", "rs", "ry", "ryd"):
+        v = getattr(sy, name)
+        getattr(s, "set_" + name)(v, len(v))
+    s.execute()
+    assert s.kernel_times()["k_spmv"]["launches"] == 3 + 2 * s.stats()["cg_iters"] + 2
