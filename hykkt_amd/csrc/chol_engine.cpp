@@ -7,10 +7,10 @@
 //   blocked right-looking panel factorization in 128-column steps
 //     (factor + invert the diagonal block; TRSM of the rows below with the
 //      inverted block on the matrix cores -- for 128-wide blocks by blocked
-//      substitution with the inverses of the 16x16 diagonal blocks, the
-//      whole inverse formed after the level for the solves; MFMA update of
-//      the panel's trailing columns),
-//   U = -L21 L21^T on the matrix cores plus the children's update matrices.
+//      substitution with the inverses of the 16x16 diagonal blocks; MFMA
+//      update of the panel's trailing columns),
+//   U = -L21 L21^T on the matrix cores plus the children's update matrices;
+// after the last level the inverses of groups of columns, for the solves.
 // Solves: one forward and one backward sweep over the whole tree.
 #include <algorithm>
 #include <queue>
@@ -295,10 +295,10 @@ void CholEngine::build_tasks()
   const int gmax = std::clamp(tun_.group_max, 1, GMAX);
   const int nlev = static_cast<int>(pl_.level_ptr.size()) - 1;
   lv_.assign(nlev, Level{});
-  inv_blk_ = inv_grp_ = Launch{};
+  inv_grp_ = Launch{};
   std::vector<int> eap, eacol, eacptr{0}, eacc, eaccol;
   std::vector<int> potrf, trsm_sn, trsm_tr, upd_sn, upd_tr, upd_tc;
-  std::vector<int> syrk_sn, syrk_tr, syrk_tc, inv_sn, inv_step, grp_sn, grp_ix;
+  std::vector<int> syrk_sn, syrk_tr, syrk_tc, grp_sn, grp_ix;
   std::vector<int> fp_sn, fp_tile;
   auto narrow = [&](int s) { return pl_.nc(s) <= dev::FRONT_NC; };
   struct Contrib {
@@ -546,39 +546,24 @@ void CholEngine::build_tasks()
     }
     L.syrk.cnt = static_cast<int>(syrk_sn.size()) - L.syrk.off;
     xcd_order(syrk_sn, syrk_tr, syrk_tc, L.syrk.off, XCD_BLOCK / ut);
-    // the whole inverses of the blocks of the steps factored without them
-    // (128-wide launches): b^3/3 flops, the triangle read twice and written
-    for (int j = 0; j < nsteps; j++) {
-      if (L.potrf[j].maxb <= 64) continue;
-      for (int q = b0; q < b1; q++) {
-        const int s = pl_.level_sn[q], nc = pl_.nc(s);
-        if (j * NB >= nc || narrow(s)) continue;
-        const double db = std::min(NB, nc - j * NB);
-        inv_sn.push_back(s);
-        inv_step.push_back(j);
-        inv_blk_.flops += db * db * db / 3;
-        inv_blk_.bytes += 24.0 * db * (db + 1) / 2;
-      }
-    }
-    // and of the groups' rest, the longest strips of each first: (n^3 - sum b^3)/3
-    // flops, the triangle read and written
+    // the groups' inverses, the longest strips of each first (whole from the 16 x 16
+    // ones: (n^3 - 256 n)/3 flops, the triangle read and written).  A block of at most
+    // 64 columns that its factorization inverted stays as it is.
     for (int q = b0; q < b1; q++) {
       const int s = pl_.level_sn[q], nc = pl_.nc(s);
+      if (narrow(s) || (nc <= 64 && L.potrf[0].maxb <= 64)) continue;
       for (int g0 = 0; g0 < nc; g0 += dev::INV_GROUP) {
         const int n = std::min(dev::INV_GROUP, nc - g0);
-        if (n <= NB) continue;
-        for (int k = 0; k < (cdiv(n, NB) - 1) * (NB / 16); k++) {
+        for (int k = 0; k < cdiv(n, 16) - 1; k++) {
           grp_sn.push_back(s);
           grp_ix.push_back(g0 / dev::INV_GROUP * 32 + k);
         }
-        const double dn = n, full = n / NB, tail = n % NB;
-        const double db = full * NB * NB * NB + tail * tail * tail;
-        inv_grp_.flops += (dn * dn * dn - db) / 3;
-        inv_grp_.bytes += 16.0 * (dn * dn - (full * NB * NB + tail * tail)) / 2;
+        const double dn = n;
+        inv_grp_.flops += (dn * dn * dn - 256 * dn) / 3;
+        inv_grp_.bytes += 16.0 * (dn * dn - 16 * dn) / 2;
       }
     }
   }
-  inv_blk_.cnt = static_cast<int>(inv_sn.size());
   inv_grp_.cnt = static_cast<int>(grp_sn.size());
   auto up = [](DevBuf<int>& b, std::vector<int>& v) {
     if (v.empty()) v.push_back(0);
@@ -600,8 +585,6 @@ void CholEngine::build_tasks()
   up(t_syrk_sn_, syrk_sn);
   up(t_syrk_tr_, syrk_tr);
   up(t_syrk_tc_, syrk_tc);
-  up(t_inv_sn_, inv_sn);
-  up(t_inv_step_, inv_step);
   up(t_grp_sn_, grp_sn);
   up(t_grp_ix_, grp_ix);
 }
@@ -884,10 +867,7 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
     });
   }
   // the solves' inverses, all levels at once
-  timed(PK_INV_BLOCKS, inv_blk_, [&] {
-    dev::inv_blocks(cd_, inv_blk_.cnt, t_inv_sn_.p, t_inv_step_.p, b, st_);
-  });
-  timed(PK_INV_BLOCKS, inv_grp_, [&] {
+  timed(PK_INV_GROUP, inv_grp_, [&] {
     dev::inv_groups(cd_, inv_grp_.cnt, t_grp_sn_.p, t_grp_ix_.p, b, st_);
   });
 }

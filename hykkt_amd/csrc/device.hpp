@@ -216,11 +216,11 @@ class CholEngine {
   int64_t n_ubuf_ = 0, n_dinv_ = 0, n_exch_ = 0;
   // task lists
   std::vector<Level> lv_;
-  Launch inv_blk_, inv_grp_;   // the solves' inverses, all levels
+  Launch inv_grp_;   // the solves' inverses, all levels
   DevBuf<int> t_ea_p_, t_ea_col_, t_ea_cptr_, t_ea_cc_, t_ea_ccol_;
   DevBuf<int> t_potrf_, t_trsm_sn_, t_trsm_tr_, t_upd_sn_, t_upd_tr_, t_upd_tc_;
   DevBuf<int> t_syrk_sn_, t_syrk_tr_, t_syrk_tc_;
-  DevBuf<int> t_inv_sn_, t_inv_step_, t_grp_sn_, t_grp_ix_;
+  DevBuf<int> t_grp_sn_, t_grp_ix_;
   DevBuf<int> t_fp_sn_, t_fp_tile_;
   DevBuf<dev::ChildRec> child_rec_;
   DevBuf<dev::SnRec> sn_rec_;

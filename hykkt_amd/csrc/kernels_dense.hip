@@ -692,7 +692,6 @@ __device__ __forceinline__ void inverse_full(double (*P)[BK + 1], double* W, int
   constexpr int NL = BK * (BK + 1) / 2, PER = (NL + 255) / 256;
   if constexpr (BK >= 32) inverse_level<BK, 16>(P, wave, lane);
   if constexpr (BK >= 64) inverse_level<BK, 32>(P, wave, lane);
-  if constexpr (BK >= 128) inverse_level<BK, 64>(P, wave, lane);
   // over the folded lower triangle, LDS reads first so they overlap
   constexpr int SB2 = (PER + 1) / 2;   // entries per batch
 #pragma unroll
@@ -900,7 +899,7 @@ __device__ __forceinline__ void invert16(double (*P)[BK + 1], const double* rd, 
 // Diagonal block `step` of supernode s, by one workgroup of 256 threads with
 // smem >= potrf_smem<BK>().  BK: padded block edge (32, 64 or 128) >= b.
 // FULL: the whole inverse; otherwise only the inverses of its 16x16 diagonal
-// blocks (the blocked TRSM's), the rest formed after the level (k_inv_blocks).
+// blocks (the blocked TRSM's); k_inv_group forms the rest.
 template <int BK, bool FULL>
 __device__ __forceinline__ void potrf_block(const CholDev& c, double* L, double* dinv, int* pivot,
                                             int s, int step, double* smem)
@@ -1155,70 +1154,25 @@ __global__ void __launch_bounds__(256) k_front_panel(CholDev c, const int* __res
       }
 }
 
-// The whole inverse of 128-wide diagonal blocks whose factorization left only
-// the 16x16 diagonal blocks' inverses (potrf_block<128, false>): L_kk from
-// the panel, those inverses from the dinv slot, then the doubling levels.
-// Task (s, step); system blockIdx.y.  Same arithmetic as the in-kernel
-// inverse, so the same bits.
-__global__ void __launch_bounds__(256) k_inv_blocks(CholDev c, const int* __restrict__ tsn,
-                                                    const int* __restrict__ tstep, Batch bt)
-{
-  constexpr int BK = BT;
-  constexpr int NL = BK * (BK + 1) / 2, PER = (NL + 255) / 256;
-  constexpr int T16 = PW * (PW + 1) / 2;
-  extern __shared__ double smem[];
-  const int sy = batch_sys(bt);
-  if (sy < 0) return;
-  const int s = tsn[blockIdx.x], step = tstep[blockIdx.x];
-  const SnInfo si = sninfo(c, batch_at(c.L, sy, bt), s);
-  const int k0 = step * BT;
-  if (k0 >= si.nc) return;
-  const int b = min(BK, si.nc - k0);
-  double (*P)[BK + 1] = reinterpret_cast<double (*)[BK + 1]>(smem);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const double* D = si.Ls + static_cast<int64_t>(k0) * si.f + k0;
-  double* W = batch_at(c.dinv, sy, bt) + c.dinv_off[s] + inv_at(si.nc, step);
-  const int ldw = inv_ld(si.nc, k0 / INV_GROUP);
-  {
-    double v[PER];
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-      int r, col;
-      lower_entry<BK>(min(tid + u * 256, NL - 1), r, col);
-      const bool in = r < b;
-      const double t = D[in ? r + static_cast<int64_t>(col) * si.f : 0];
-      v[u] = in ? t : (r == col ? 1.0 : 0.0);
-    }
-#pragma unroll
-    for (int u = 0; u < PER; u++) {
-      int r, col;
-      lower_entry<BK>(min(tid + u * 256, NL - 1), r, col);
-      if (tid + u * 256 < NL) P[r][col] = v[u];
-    }
-  }
-  for (int e = tid; e < (BK / PW) * T16; e += 256) {
-    const int bb = (e / T16) * PW;
-    int r, col;
-    lower_entry<PW>(e % T16, r, col);
-    const double x = (bb + r < b) ? W[static_cast<int64_t>(bb + col) * ldw + bb + r]
-                                  : (r == col ? 1.0 : 0.0);
-    if (r == col) P[bb + col][BK] = x;
-    else P[bb + col][bb + r] = x;
-  }
-  __syncthreads();
-  inverse_full<BK>(P, W, ldw, b, tid, wave, lane);
-}
-
-// The inverses of groups of two to four 128-column diagonal blocks, below their
-// diagonal blocks' (which the launches before left): X = L^{-1} by columns,
-//   X(i, j) = -X(i, i) (L(i, j) X(j, j) + .. + L(i, i-1) X(i-1, j)),
-// a workgroup per strip of 16 columns, wave w rows 16 w .. 16 w + 15 of each block,
-// operands read straight into MFMA fragments, the strip and the sums through LDS.
+// The inverses of groups of up to four 128-column diagonal blocks, from the factor and
+// the inverses of its 16 x 16 diagonal blocks (which the factorization left): a
+// workgroup per strip of 16 columns solves L X = E, 128 rows at a time, wave w rows
+// 16 w .. 16 w + 15 of them. First all the blocks before, in one product (operands read
+// straight into MFMA fragments, X from LDS); then the block's eight panels by
+// substitution, each wave's sums staying in its accumulators, whose lane layout
+// (element v = D[4 v + l/16][l%16]) is the B operand's of k-step v.
+// By substitution, and not with products of the 128-wide blocks' own inverses (doubled
+// from the 16 x 16 ones), which lose the square of a block's condition number: backward
+// error of a solve with a Gaussian kernel matrix (condition 1e11) of 512 / 1,024: 2.6e-13
+// / 1.7e-13, with products 2.3e-10 / 9.5e-12, sweeps through 128-wide inverses 1.5e-11 /
+// 3.6e-14. On the grids' H_gamma, gamma 1e4 to 1e6 and Ds spread 1e-2..1e2 to 1e-4..1e8,
+// backward and forward errors are those of 128-wide inverses; on dense matrices of random
+// eigenvectors up to 7 times theirs, and below the unit roundoff.
 // With them a sweep passes a group of up to 512 columns in one product in place of a
-// chain of four, at 28 us per factorization at 1,000 buses, 34 at 5,000 (one
-// workgroup takes 15 us of matrix instructions for the first strip of a whole group).  Task: supernode, 32 group + strip; system
-// blockIdx.y.
+// chain of four. Bound by the first strip's chain: 36 us a factorization at 1,000 buses,
+// 125 at 20,000, 217 at eight systems of 5,000 (products: 48, 128, 209 in two launches).
+// Loads four K-steps ahead: with 8 and 16 the kernel spills (217 and 275 us, eight of
+// 5,000). Task: supernode, 32 group + strip; system blockIdx.y.
 constexpr int IG_LD = PW + 1;   // row of the strip in LDS
 constexpr size_t IG_SMEM = INV_GROUP * IG_LD * sizeof(double);   // two workgroups per CU
 
@@ -1227,65 +1181,98 @@ __global__ void __launch_bounds__(512, 4) k_inv_group(CholDev c, const int* __re
 {
   extern __shared__ double smem[];
   double (*Xs)[IG_LD] = reinterpret_cast<double (*)[IG_LD]>(smem);
-  double (*Ts)[IG_LD] = Xs + (INV_GROUP - BT);   // the last block's X is not read again
   const int sy = batch_sys(bt);
   if (sy < 0) return;
-  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int NP = BT / PW;   // panels of a block, a wave each
+  const int lane = threadIdx.x & 63, w = uni(threadIdx.x >> 6);
   const int m16 = lane & 15, q4 = lane >> 4;
-  const int s = tsn[blockIdx.x], ix = tix[blockIdx.x], g = ix >> 5, cs = (ix & 31) * PW;
+  const int s = uni(tsn[blockIdx.x]), ix = uni(tix[blockIdx.x]), g = ix >> 5, cs = (ix & 31) * PW;
   const SnInfo si = sninfo(c, batch_at(c.L, sy, bt), s);
-  const int g0 = g * INV_GROUP, ng = min(INV_GROUP, si.nc - g0), nb = (ng + BT - 1) / BT;
-  const int jb = cs / BT;
-  const int64_t ld = inv_ld(si.nc, g), f = si.f;
-  double* W = batch_at(c.dinv, sy, bt) + c.dinv_off[s] + static_cast<int64_t>(g) * INV_GROUP * INV_GROUP;
+  const int nc = uni(si.nc), f = uni(si.f);
+  const int g0 = g * INV_GROUP, ng = min(INV_GROUP, nc - g0), nb = (ng + BT - 1) / BT;
+  const int jb = cs / BT, pj = (cs - BT * jb) / PW;   // the strip's block and panel
+  const int ld = inv_ld(nc, g);
+  const uint32_t f8 = static_cast<uint32_t>(f) * 8u;
+  double* W = batch_at(c.dinv, sy, bt) + uni64(c.dinv_off[s]) +
+              static_cast<int64_t>(g) * INV_GROUP * INV_GROUP;
+  const double* Lg = batch_at(c.L, sy, bt) + uni64(c.l_off[s]) + static_cast<int64_t>(g0) * f;
+  auto load = [](rsrc_t v, uint32_t vo, uint32_t so) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(v, vo, so, 0));
+  };
+  constexpr int D = 4;   // K-steps of the product whose loads are in flight
+  for (int ib = jb; ib < nb; ib++) {
+    // this lane's row of the factor (past the supernode's columns the last one: its X is
+    // 0, as the inverses past them hold zeros), its columns in this block
+    const int row = BT * ib + PW * w, cols = min(BT, nc - g0 - BT * ib);
+    const uint32_t vr = static_cast<uint32_t>(min(g0 + row + m16, nc - 1)) * 8u;
+    const int p0 = ib == jb ? pj : 0;   // rows above are 0
+    // L(row, 16 q + 4 v + q4) of the block, q < w, and inv16 of the wave's own panel
+    // (a quadruple of columns that ends past the block's is another one: rows that
+    // would use it are past the supernode's columns)
+    double lw[NP - 1][4], iw[4];
+    {
+      const rsrc_t rl = view(Lg + static_cast<int64_t>(BT * ib) * f, static_cast<int64_t>(cols) * f8);
+      const uint32_t vo = vr + static_cast<uint32_t>(min(q4, cols - 1)) * f8;
 #pragma unroll
-  for (int u = 0; u < BT * PW / 512; u++) {
-    const int r = BT * jb + (tid & (BT - 1)), cc = (tid >> 7) + 4 * u;
-    Xs[r][cc] = W[(cs + cc) * ld + r];
-  }
-  // acc += A X: this lane's row `row` of A (column-major, columns lda bytes apart) times
-  // X (K x 16, in LDS; K a multiple of 16), D steps' loads in flight
-  constexpr int D = 16;
-  auto product = [&](d4& acc, const double* A, int row, uint32_t lda, const double (*X)[IG_LD],
-                     int K) {
-    const rsrc_t ra = view(A, static_cast<int64_t>(K) * lda);
-    const uint32_t vo = static_cast<uint32_t>(row) * 8u + static_cast<uint32_t>(q4) * lda;
-    auto load = [&](int k) {
-      return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(
-                                            ra, vo, static_cast<uint32_t>(min(k, K - 4)) * lda, 0));
-    };
-    double a[D];
+      for (int q = 0; q < NP - 1; q++)
 #pragma unroll
-    for (int u = 0; u < D; u++) a[u] = load(4 * u);
-    for (int k0 = 0; k0 < K; k0 += 4 * D) {
+        for (int v = 0; v < 4; v++)
+          lw[q][v] = q >= p0 && q < w
+                         ? load(rl, vo, static_cast<uint32_t>(min(PW * q + 4 * v, max(cols - 4, 0))) * f8)
+                         : 0.0;
 #pragma unroll
-      for (int u = 0; u < D; u++) {
-        const int k = k0 + 4 * u;
-        if (k >= K) break;
-        const double v = a[u];
-        a[u] = load(k + 4 * D);
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(X[k + q4][m16], v, acc, 0, 0, 0);
+      for (int v = 0; v < 4; v++) iw[v] = W[static_cast<int64_t>(row + 4 * v + q4) * ld + row + m16];
+    }
+    // E - L X over the blocks before: element v is row 4 v + q4, column m16
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    if (ib == jb) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        acc[v] = w == pj && 4 * v + q4 == m16 ? 1.0 : 0.0;
+        if (w < pj) Xs[row + 4 * v + q4][m16] = 0.0;
+      }
+    } else {
+      const int K = BT * (ib - jb);
+      const rsrc_t ra = view(Lg + static_cast<int64_t>(BT * jb) * f, static_cast<int64_t>(K) * f8);
+      const double (*X)[IG_LD] = Xs + BT * jb;
+      const uint32_t vo = vr + static_cast<uint32_t>(q4) * f8;
+      auto at = [&](int k) { return load(ra, vo, static_cast<uint32_t>(min(k, K - 4)) * f8); };
+      double a[D];
+#pragma unroll
+      for (int u = 0; u < D; u++) a[u] = at(4 * u);
+      for (int k0 = 0; k0 < K; k0 += 4 * D) {
+#pragma unroll
+        for (int u = 0; u < D; u++) {
+          const int k = k0 + 4 * u;
+          const double v = -a[u];
+          a[u] = at(k + 4 * D);
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(v, X[k + q4][m16], acc, 0, 0, 0);
+        }
       }
     }
-  };
-  __syncthreads();
-  for (int ib = jb + 1; ib < nb; ib++) {
-    // rows past the supernode's columns repeat the last one; their X is 0
-    const int row = BT * ib + PW * w + m16;
-    d4 t = {0.0, 0.0, 0.0, 0.0};
-    product(t, si.Ls + (g0 + BT * jb) * f, min(g0 + row, si.nc - 1), static_cast<uint32_t>(f) * 8u,
-            Xs + BT * jb, BT * (ib - jb));
 #pragma unroll
-    for (int v = 0; v < 4; v++) Ts[PW * w + m16][4 * v + q4] = t[v];
-    __syncthreads();
-    d4 x = {0.0, 0.0, 0.0, 0.0};
-    product(x, W + BT * ib * ld, row, static_cast<uint32_t>(ld) * 8u, Ts, PW * (w + 1));
+    for (int p = 0; p < NP; p++) {
+      if (p < p0) continue;
+      if (w == p) {
+        d4 x = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      if (ib + 1 < nb) Xs[row][4 * v + q4] = -x[v];
-      if (row < ng) W[(cs + 4 * v + q4) * ld + row] = -x[v];
+        for (int v = 0; v < 4; v++)
+          x = __builtin_amdgcn_mfma_f64_16x16x4f64(iw[v], acc[v], x, 0, 0, 0);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const int r = row + 4 * v + q4;
+          Xs[r][m16] = x[v];
+          if (r < ng && r >= cs + PW) W[static_cast<int64_t>(cs + m16) * ld + r] = x[v];
+        }
+      }
+      __syncthreads();
+      if (p + 1 < NP && w > p) {
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-lw[p < NP - 1 ? p : 0][v],
+                                                     Xs[BT * ib + PW * p + 4 * v + q4][m16], acc, 0, 0, 0);
+      }
     }
-    __syncthreads();
   }
 }
 
@@ -1497,21 +1484,6 @@ void trsm_inv(const CholDev& c, int ntasks, const int* tsn, const int* ttr, int 
   const dim3 grid(ntasks, b.count);
   if (short_rows) k_trsm_inv<32><<<grid, 256, SM, st>>>(c, tsn, ttr, step, b);
   else k_trsm_inv<128><<<grid, 256, SM, st>>>(c, tsn, ttr, step, b);
-  HIPCHK(hipGetLastError());
-}
-
-void inv_blocks(const CholDev& c, int ntasks, const int* tsn, const int* tstep, const Batch& b,
-                hipStream_t st)
-{
-  if (ntasks <= 0 || b.count <= 0) return;
-  constexpr size_t SM = (BT * (BT + 1) + BT) * sizeof(double);
-  static const bool attr = [] {
-    HIPCHK(hipFuncSetAttribute(reinterpret_cast<const void*>(k_inv_blocks),
-                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(SM)));
-    return true;
-  }();
-  (void)attr;
-  k_inv_blocks<<<dim3(ntasks, b.count), 256, SM, st>>>(c, tsn, tstep, b);
   HIPCHK(hipGetLastError());
 }
 

@@ -26,7 +26,7 @@ enum ProfKind {
   PK_SPGEMM_SCATTER,
   PK_TRSM,               // blocked-substitution TRSM, 128-row tiles
   PK_TRSM_SHORT,         // the same, 32-row tiles
-  PK_INV_BLOCKS,
+  PK_INV_GROUP,
   PK_COUNT
 };
 
