@@ -29,6 +29,7 @@ constexpr int TR = 64;    // rows of a short tile of the blocked TRSM
 constexpr int GMAX = 8;   // most steps one grouped trailing update can cover
 constexpr int XCD_BLOCK = 1024;   // rows and columns of a block of tiles of one XCD
 constexpr int U_SMALL_NC = 512;   // update matrices of at most so many columns take 64 x 64 tiles
+static_assert(CholOptions{}.index_narrow == dev::FRONT_NC, "front_panel's index has the columns' rows");
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // Tiles `from` .. of a launch's list (by supernode, column, row) in the order that keeps
@@ -241,8 +242,7 @@ CholEngine::~CholEngine()
   if (st2_) (void)hipStreamDestroy(st2_);
 }
 
-// The supernodes' records, and where each child's rows are among its parent's
-// front rows.
+// The supernodes' records.
 void CholEngine::build_fronts()
 {
   const int ns = pl_.ns;
@@ -252,27 +252,18 @@ void CholEngine::build_fronts()
     rec[t] = dev::ChildRec{pl_.u_off[ch], pl_.nr(ch), 0};
   }
   std::vector<dev::SnRec> sr(std::max(ns, 1));
-  std::vector<int> inv;
   int64_t dinv = 0;
   for (int s = 0; s < ns; s++) {
-    const int nc = pl_.nc(s), nr = pl_.nr(s), first = nc <= dev::FRONT_NC ? 0 : nc;
-    const int rows = nc + nr - first, nch = pl_.child_ptr[s + 1] - pl_.child_ptr[s];
-    const int64_t at = static_cast<int64_t>(inv.size()), off = at - first;
-    inv.resize(at + static_cast<int64_t>(nch) * rows, -1);
-    for (int t = 0; t < nch; t++) {
-      const int ch = pl_.child_list[pl_.child_ptr[s] + t];
-      for (int q = pl_.rows_ptr[ch]; q < pl_.rows_ptr[ch + 1]; q++)
-        if (pl_.rel[q] >= first)
-          inv[off + static_cast<int64_t>(t) * rows + pl_.rel[q]] = q - pl_.rows_ptr[ch];
-    }
-    sr[s] = dev::SnRec{pl_.sn_first[s], nc, nr, pl_.child_ptr[s], nch, rows, {0, 0},
-                       pl_.l_off[s], dinv, pl_.u_off[s], off};
+    const int nc = pl_.nc(s);
+    const int nch = pl_.pulls[s] ? pl_.child_ptr[s + 1] - pl_.child_ptr[s] : 0;
+    sr[s] = dev::SnRec{pl_.sn_first[s], nc, pl_.nr(s), pl_.child_ptr[s], nch, pl_.inv_rows[s],
+                       {0, 0}, pl_.l_off[s], dinv, pl_.u_off[s], pl_.inv_off[s]};
     dinv += dev::inv_size(nc);
   }
-  if (inv.empty()) inv.push_back(-1);
   child_rec_.upload(rec);
   sn_rec_.upload(sr);
-  inv_.upload(inv);
+  if (pl_.inv.empty()) inv_.upload(std::vector<int>{-1});
+  else inv_.upload(pl_.inv);
   cd_.child_rec = child_rec_.p;
   cd_.sn_rec = sn_rec_.p;
   cd_.inv = inv_.p;
@@ -308,18 +299,20 @@ void CholEngine::build_tasks()
   for (int l = 0; l < nlev; l++) {
     Level& L = lv_[l];
     const int b0 = pl_.level_ptr[l], b1 = pl_.level_ptr[l + 1];
-    {
-      Launch& la = L.ea_panel;
+    // part 0: panels whose kernels do not add the children themselves; 1: update
+    // matrices of the supernodes without an index of their children's rows
+    for (int part = 0; part < 2; part++) {
+      Launch& la = part == 0 ? L.ea_panel : L.ea_u;
       la.off = static_cast<int>(eap.size());
       for (int q = b0; q < b1; q++) {
         const int p = pl_.level_sn[q], ncp = pl_.nc(p);
-        if (narrow(p)) continue;   // front_panel adds its children itself
+        if (pl_.pulls[p] && (part == 1 || narrow(p))) continue;
         con.clear();
         for (int t = pl_.child_ptr[p]; t < pl_.child_ptr[p + 1]; t++) {
           const int c = pl_.child_list[t];
           for (int k = pl_.rows_ptr[c]; k < pl_.rows_ptr[c + 1]; k++) {
             int col = pl_.rel[k];
-            if (col < ncp) con.push_back({col, c, k - pl_.rows_ptr[c]});
+            if ((col < ncp) == (part == 0)) con.push_back({col, c, k - pl_.rows_ptr[c]});
           }
         }
         std::stable_sort(con.begin(), con.end(),
@@ -530,7 +523,7 @@ void CholEngine::build_tasks()
       const double nr = pl_.nr(s), nc = pl_.nc(s), pairs = nr * (nr + 1) / 2;
       L.syrk.flops += 2.0 * nc * pairs;
       L.syrk.bytes += 8.0 * (nr * nc + pairs);
-      for (int t = pl_.child_ptr[s]; t < pl_.child_ptr[s + 1]; t++) {
+      for (int t = pl_.child_ptr[s]; pl_.pulls[s] && t < pl_.child_ptr[s + 1]; t++) {
         const int ch = pl_.child_list[t];
         double below = 0;   // the child's rows below s's columns
         for (int k = pl_.rows_ptr[ch]; k < pl_.rows_ptr[ch + 1]; k++) below += pl_.rel[k] >= pl_.nc(s);
@@ -776,14 +769,16 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
   };
   auto timed = [&](int kind, const Launch& la, auto&& launch) { timed_on(st_, kind, la, launch); };
   for (const Level& L : lv_) {
+    auto add_children = [&](const Launch& la) {
+      timed(PK_EXTEND_ADD, la, [&] {
+        dev::extend_add(cd_, la.cnt, t_ea_p_.p + la.off, t_ea_col_.p + la.off, t_ea_cptr_.p + la.off,
+                        t_ea_cc_.p, t_ea_ccol_.p, b, st_);
+      });
+    };
+    add_children(L.ea_panel);
     timed(PK_POTRF, L.front, [&] {
       dev::front_panel(cd_, L.front.cnt, t_fp_sn_.p + L.front.off, t_fp_tile_.p + L.front.off, b,
                        st_);
-    });
-    timed(PK_EXTEND_ADD, L.ea_panel, [&] {
-      dev::extend_add(cd_, L.ea_panel.cnt, t_ea_p_.p + L.ea_panel.off,
-                      t_ea_col_.p + L.ea_panel.off, t_ea_cptr_.p + L.ea_panel.off, t_ea_cc_.p,
-                      t_ea_ccol_.p, b, st_);
     });
     // Blocked steps with look-ahead.  Main stream: diagonal blocks, TRSM,
     // update of the next block column(s); second stream: the rest of the
@@ -865,6 +860,7 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
       dev::update_matrices(cd_, L.syrk.cnt, t_syrk_sn_.p + L.syrk.off, t_syrk_tr_.p + L.syrk.off,
                            t_syrk_tc_.p + L.syrk.off, L.small_u, b, st_);
     });
+    add_children(L.ea_u);
   }
   // the solves' inverses, all levels at once
   timed(PK_INV_GROUP, inv_grp_, [&] {

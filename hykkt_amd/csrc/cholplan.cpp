@@ -363,7 +363,33 @@ CholPlan chol_analyze(const Pattern& a, const CholOptions& opt)
     }
   }
 
-  // ---- 9. assembly targets of the input's lower-triangle entries ----
+  // ---- 9. where each child's rows are among its parent's front rows ----
+  pl.pulls.assign(ns, 1);
+  pl.inv_off.assign(ns, 0);
+  pl.inv_rows.assign(ns, 0);
+  for (int s = 0; s < ns; s++) {
+    const int first = pl.inv_first(s, opt.index_narrow), nch = pl.child_ptr[s + 1] - pl.child_ptr[s];
+    const int rows = pl.nc(s) + pl.nr(s) - first;
+    int64_t child_rows = 0;
+    for (int t = pl.child_ptr[s]; t < pl.child_ptr[s + 1]; t++) child_rows += pl.nr(pl.child_list[t]);
+    const int64_t size = static_cast<int64_t>(nch) * rows, at = static_cast<int64_t>(pl.inv.size());
+    pl.inv_off[s] = at - first;
+    pl.inv_rows[s] = rows;
+    if (nch > opt.index_children + pl.nc(s) / opt.index_per_cols ||
+        static_cast<double>(size) > opt.index_max * static_cast<double>(child_rows)) {
+      pl.pulls[s] = 0;
+      continue;
+    }
+    pl.inv.resize(at + size, -1);
+    for (int t = 0; t < nch; t++) {
+      const int ch = pl.child_list[pl.child_ptr[s] + t];
+      for (int q = pl.rows_ptr[ch]; q < pl.rows_ptr[ch + 1]; q++)
+        if (pl.rel[q] >= first)
+          pl.inv[pl.inv_off[s] + static_cast<int64_t>(t) * rows + pl.rel[q]] = q - pl.rows_ptr[ch];
+    }
+  }
+
+  // ---- 10. assembly targets of the input's lower-triangle entries ----
   pl.a_src.resize(nlow);
   pl.a_dst.resize(nlow);
   for (int c = 0; c < n; c++) {

@@ -179,7 +179,7 @@ class CholEngine {
     double flops = 0.0, bytes = 0.0;   // algorithmic, for the profiler
   };
   struct Level {
-    Launch front, ea_panel, syrk;
+    Launch front, ea_panel, ea_u, syrk;
     bool small_u = false;   // update matrices in 64 x 64 tiles
     std::vector<Launch> potrf, trsm, upd_next, upd_rest;
     // per step: its position in its group of consecutive steps and the

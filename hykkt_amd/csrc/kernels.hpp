@@ -270,7 +270,8 @@ struct ChildRec {
 };
 // What a workgroup needs to know of a supernode.  Child t's row of its update matrix
 // at front row r, or -1: inv[inv_off + t * inv_rows + r] (the rows below the
-// supernode's columns; for at most FRONT_NC columns those, too).
+// supernode's columns; for at most FRONT_NC columns those, too).  nch = 0: no children,
+// or extend_add() adds them.
 struct SnRec {
   int a, nc, nr;      // first column, columns, rows below them
   int child0, nch;    // its children in child_rec
@@ -328,7 +329,7 @@ struct CholDev {
   const int64_t* dinv_off;  // ns+1, supernode s's slot in dinv
 };
 
-// Extend-add tasks: task t = (parent p, parent front column col);
+// Extend-add tasks: task t = (parent p, front column col: of the panel or below it);
 // contributions [cptr[t], cptr[t+1]) are (child, child-local column) pairs.
 void extend_add(const CholDev& c, int ntasks, const int* task_p, const int* task_col,
                 const int* cptr, const int* contrib_child, const int* contrib_col,

@@ -34,8 +34,9 @@ __device__ __forceinline__ SnInfo sninfo(const CholDev& c, double* L, int s)
 }
 
 // ----------------------------------------------------------------- extend-add
-// One workgroup per column of a parent's panel and system (its update matrix takes
-// its children's in k_dense_nt).  Children are added one
+// One workgroup per front column of a parent and system: columns of panels, and of the
+// update matrices whose tiles do not take the children's themselves (k_dense_nt: the
+// parents with an index of their children's rows).  Children are added one
 // after the other (fixed order => deterministic sums); within one child the
 // relative index map is injective.
 __global__ void __launch_bounds__(256) k_extend_add(CholDev c, const int* __restrict__ task_p,
@@ -47,11 +48,14 @@ __global__ void __launch_bounds__(256) k_extend_add(CholDev c, const int* __rest
   const int sy = batch_sys(b);
   if (sy < 0) return;
   double* const L = batch_at(c.L, sy, b);
-  const double* const U = batch_at(c.U, sy, b);
+  double* const U = batch_at(c.U, sy, b);
   const int t = blockIdx.x;
   const int p = task_p[t], col = task_col[t];
   const SnInfo ip = sninfo(c, L, p);
-  double* const base = ip.Ls + static_cast<int64_t>(col) * ip.f;
+  // front row r of the column at base[r] (of U: rows >= col)
+  double* const base = col < ip.nc
+                           ? ip.Ls + static_cast<int64_t>(col) * ip.f
+                           : U + c.u_off[p] + packed_lower(0, col - ip.nc, ip.nr) - ip.nc;
   for (int k = cptr[t]; k < cptr[t + 1]; k++) {
     const int ch = cc[k], r2 = ccol[k];
     const int nrc = c.rows_ptr[ch + 1] - c.rows_ptr[ch];

@@ -73,6 +73,12 @@ struct CholPlan {
   std::vector<int> rel;         // per entry of rows: position in the parent's front
   std::vector<int> child_ptr;   // ns+1
   std::vector<int> child_list;  // children in increasing order
+  // Where the rows of s's children are in its front: row of child t's update matrix at
+  // front row r, or -1, at inv[inv_off[s] + t * inv_rows[s] + r] (r from inv_first(s)
+  // on).  Supernodes without it (pulls[s] = 0) have too many children (see CholOptions).
+  std::vector<char> pulls;      // ns
+  std::vector<int64_t> inv_off;
+  std::vector<int> inv_rows, inv;
   std::vector<int64_t> l_off;   // ns+1 (doubles)
   std::vector<int64_t> u_off;   // ns+1 (doubles): U(s) offsets (reused space), [ns] = pool size
   std::vector<int> level;       // height in the supernodal tree (leaves 0)
@@ -88,6 +94,7 @@ struct CholPlan {
   int max_front = 0;
   int nc(int s) const { return sn_first[s + 1] - sn_first[s]; }
   int nr(int s) const { return rows_ptr[s + 1] - rows_ptr[s]; }
+  int inv_first(int s, int narrow) const { return nc(s) <= narrow ? 0 : nc(s); }
 };
 
 struct CholOptions {
@@ -95,6 +102,19 @@ struct CholOptions {
   double relax_frac_mid = 0.5;  // zero fraction allowed up to relax_mid_cols columns
   int relax_mid_cols = 32;
   double relax_frac_big = 0.05; // zero fraction allowed beyond that
+  // Index of the children's rows, with the columns' rows for supernodes of at most
+  // index_narrow columns.  A tile of a front walks all the children in it, about 3 us
+  // each beside the tile's own work, which grows with the columns; without it they are
+  // added in passes of their own.  So it is for supernodes of at most index_children +
+  // nc / index_per_cols children: 20 columns on 600 rows, 16 / 64 / 256 / 4,000 children,
+  // with it 453 / 541 / 868 / 7628 us a factorization, without 432 / 430 / 438 / 777; 200
+  // on 1,500 1364 / 1392 / 1477 / 3265 against 1354 / 1352 / 1362 / 1546.  (The grids'
+  // fronts, 8 to 28 children up to 40,000 buses, are below the line: there the passes
+  // took longer than the walk.)  And with at most index_max entries for each row of the
+  // children, so its size is bounded by the factor's own structure.
+  int index_narrow = 32;
+  int index_children = 16, index_per_cols = 16;
+  double index_max = 64.0;
 };
 
 // Analyse the lower triangle of the n x n symmetric matrix `a` (CSR, sorted;
