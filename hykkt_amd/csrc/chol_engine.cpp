@@ -844,11 +844,15 @@ void CholEngine::factor(double pivot_tol, const dev::Batch& bt, bool pivots_clea
       if (rest) {
         if (!on_launch) HIPCHK(hipEventRecord(ev_main_, st_));
         HIPCHK(hipStreamWaitEvent(st2_, ev_main_, 0));
+        // off the diagonal block's compute unit (see dense_nt): up to two tiles of 128 x
+        // 128 a compute unit, which are then all resident; as quarters up to eight
+        // workgroups, of which the LDS lets five in at a time.  The line at those five
+        // takes longer (5,000 buses 3740 -> 3766 us, 10,000 and batches the same)
         timed_on(st2_, PK_DENSE_NT, L.upd_rest[j], [&] {
           dev::dense_nt(cd_, L.upd_rest[j].cnt, t_upd_sn_.p + L.upd_rest[j].off,
                         t_upd_tr_.p + L.upd_rest[j].off, t_upd_tc_.p + L.upd_rest[j].off, umode,
                         ustep, b, st2_, false, ev_rest_,
-                        L.upd_rest[j].cnt * b.count <= 2 * n_cu_,   // all resident at once
+                        L.upd_rest[j].cnt * b.count <= 2 * n_cu_,
                         quarters(L.upd_rest[j], kblk));
         });
         rest_pending = true;
