@@ -114,10 +114,7 @@ CholEngine::CholEngine(const Pattern& a, const CholOptions& opt, hipStream_t st)
   upi(rows_ptr_, pl_.rows_ptr);
   upi(rows_, pl_.rows);
   upi(rel_, pl_.rel);
-  upi(child_ptr_, pl_.child_ptr);
-  upi(child_list_, pl_.child_list);
   upi(post_, pl_.post);
-  upi(sn_parent_, pl_.sn_parent);
   l_off_.upload(pl_.l_off);
   u_off_.upload(pl_.u_off);
   upi(a_src_, pl_.a_src);
@@ -145,9 +142,6 @@ CholEngine::CholEngine(const Pattern& a, const CholOptions& opt, hipStream_t st)
   cd_.rel = rel_.p;
   cd_.l_off = l_off_.p;
   cd_.u_off = u_off_.p;
-  cd_.child_ptr = child_ptr_.p;
-  cd_.child_list = child_list_.p;
-  cd_.sn_parent = sn_parent_.p;
   cd_.dinv_off = dinv_off_.p;
   build_fronts();
   build_tasks();

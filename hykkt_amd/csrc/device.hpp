@@ -210,7 +210,7 @@ class CholEngine {
   Profiler* prof_ = nullptr;
   dev::CholDev cd_{};
   dev::SolveDev sd_{};
-  DevBuf<int> sn_first_, rows_ptr_, rows_, rel_, child_ptr_, child_list_, post_, sn_parent_;
+  DevBuf<int> sn_first_, rows_ptr_, rows_, rel_, post_;
   DevBuf<int64_t> l_off_, u_off_, a_dst_, diag_pos_, uvec_off_, dinv_off_, front_off_, exch_off_;
   DevBuf<int> a_src_;
   int64_t n_ubuf_ = 0, n_dinv_ = 0, n_exch_ = 0;

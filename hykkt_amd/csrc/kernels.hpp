@@ -315,10 +315,7 @@ struct CholDev {
   const int* rel;
   const int64_t* l_off;     // ns+1
   const int64_t* u_off;     // ns+1: U(s) offsets in the reused update space
-  const int* child_ptr;
-  const int* child_list;
-  const int* sn_parent;
-  const ChildRec* child_rec;   // by position in child_list
+  const ChildRec* child_rec;   // by position in the plan's child_list
   const SnRec* sn_rec;
   const int* inv;              // see SnRec
   double* L;

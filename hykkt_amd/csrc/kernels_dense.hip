@@ -140,7 +140,6 @@ __device__ __forceinline__ SnInfo sninfo(const CholDev& c, double* L, int s)
 // the gfx9-family raw-buffer setting).
 using rsrc_t = __amdgpu_buffer_rsrc_t;
 typedef double d2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t VIEW_MAX = 0x7fffffffu;
 constexpr uint32_t OFF_NONE = 0x80000000u;   // past every view: the load returns 0
 
