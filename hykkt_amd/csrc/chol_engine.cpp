@@ -114,7 +114,6 @@ CholEngine::CholEngine(const Pattern& a, const CholOptions& opt, hipStream_t st)
   upi(rows_ptr_, pl_.rows_ptr);
   upi(rows_, pl_.rows);
   upi(rel_, pl_.rel);
-  upi(post_, pl_.post);
   l_off_.upload(pl_.l_off);
   u_off_.upload(pl_.u_off);
   upi(a_src_, pl_.a_src);
@@ -164,7 +163,8 @@ void CholEngine::pick_second_stream()
   std::vector<hipStream_t> rejected;
   for (int t = 0; t < TRIES; t++) {
     HIPCHK(hipStreamCreate(&st2_));
-    if (t + 1 == TRIES || dev::streams_overlap(st_, st2_, words.p)) break;
+    overlap_ = dev::streams_overlap(st_, st2_, words.p);
+    if (overlap_ || t + 1 == TRIES) break;
     rejected.push_back(st2_);
     st2_ = nullptr;
   }

@@ -168,7 +168,8 @@ class CholEngine {
   const int* a_src() const { return a_src_.p; }
   const int64_t* a_dst() const { return a_dst_.p; }
   int n_assembled() const { return static_cast<int>(pl_.a_src.size()); }
-  const int* post_dev() const { return post_.p; }
+  // Whether the second stream was seen to run beside the solver's own when it was picked.
+  bool second_stream_overlaps() const { return overlap_; }
   // Time every factor/solve launch with `p` (nullptr: no timing).
   void set_profiler(Profiler* p) { prof_ = p; }
 
@@ -204,13 +205,14 @@ class CholEngine {
   DevBuf<double> own_;   // owned storage (own)
   DevBuf<int> own_piv_;
   hipStream_t st2_ = nullptr;   // look-ahead: the rest of each trailing update
+  bool overlap_ = false;        // seen to run beside st_ when it was picked
   hipEvent_t ev_main_ = nullptr, ev_rest_ = nullptr;
   hipEvent_t ev_zero_ = nullptr;   // prezero_L's fill done
   int clean_ = 0;                  // systems whose storage prezero_L zeroes, untouched since
   Profiler* prof_ = nullptr;
   dev::CholDev cd_{};
   dev::SolveDev sd_{};
-  DevBuf<int> sn_first_, rows_ptr_, rows_, rel_, post_;
+  DevBuf<int> sn_first_, rows_ptr_, rows_, rel_;
   DevBuf<int64_t> l_off_, u_off_, a_dst_, diag_pos_, uvec_off_, dinv_off_, front_off_, exch_off_;
   DevBuf<int> a_src_;
   int64_t n_ubuf_ = 0, n_dinv_ = 0, n_exch_ = 0;

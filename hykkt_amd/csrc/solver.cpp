@@ -1190,6 +1190,12 @@ long long Solver::debug_copy(int what, void* out, long long cap)
     case 20: return icopy(S.jctp_pat.rp);
     case 21: return icopy(S.jctp_pat.ci);
     case 22: return icopy(S.jctp_map);
+    case 23: {
+      DevBuf<int> words;
+      words.alloc(2);
+      return icopy({S.chol->second_stream_overlaps() ? 1 : 0,
+                    dev::streams_overlap(st_, st_, words.p) ? 1 : 0});
+    }
     default: throw Error(HYKKT_E_ARG, "debug_copy: unknown selector");
   }
 }

@@ -230,6 +230,8 @@ int hykkt_set_permutation(hykkt_solver s, const int* perm, int n);
  *  15 P*Hg*P^T rowptr (n+1)  16 its colidx (nnz_hgam)  17 its value map (nnz_hgam)
  *  18 Jc*P^T colidx (nnz Jc)  19 its map (nnz Jc)
  *  20 P*Jc^T rowptr (n+1)    21 its colidx (nnz Jc)   22 its map (nnz Jc)
+ *  23 two ints: 1 if the factorization's second stream was seen to run beside the
+ *     solver's when it was picked; the same test of one stream with itself (0)
  * Returns the number of elements copied or a negative error. */
 long long hykkt_debug_copy(hykkt_solver s, int what, void* host_out, long long capacity);
 
