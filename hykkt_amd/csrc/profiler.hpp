@@ -12,21 +12,26 @@
 
 namespace hykkt {
 
+// Groups of launches, each under one name (Profiler::name).  The names are an interface
+// that callers look groups up by; several are those of kernels since split or replaced,
+// so a group's kernels are listed here.
 enum ProfKind {
-  PK_DENSE_NT = 0,       // 128 x 128 tiles
-  PK_DENSE_NT_SHORT,     // 32 x 128 tiles (the short launches on the critical path)
-  PK_POTRF,
-  PK_EXTEND_ADD,
-  PK_SOLVE_FWD_FOREST,
-  PK_SOLVE_FWD_TOP,
-  PK_SOLVE_BWD_TOP,
-  PK_SOLVE_BWD_FOREST,
-  PK_SPMV,
-  PK_SPGEMM_VALUES,
-  PK_SPGEMM_SCATTER,
-  PK_TRSM,               // blocked-substitution TRSM, 128-row tiles
-  PK_TRSM_SHORT,         // the same, 32-row tiles
-  PK_INV_GROUP,
+  PK_DENSE_NT = 0,       // k_dense_nt with tiles of 128 x 128 and 64 x 64 (updates, update
+                         // matrices), k_trsm_inv<128>
+  PK_DENSE_NT_SHORT,     // k_dense_nt with 32-row tiles, k_trsm_inv<32> (the short launches
+                         // on the critical path)
+  PK_POTRF,              // k_potrf_inv<128, 64, 32>, k_front_panel
+  PK_EXTEND_ADD,         // k_extend_add
+  PK_SOLVE_FWD_FOREST,   // k_forest<true, ..>
+  PK_SOLVE_FWD_TOP,      // k_solve_fwd
+  PK_SOLVE_BWD_TOP,      // k_solve_bwd
+  PK_SOLVE_BWD_FOREST,   // k_forest<false, ..>
+  PK_SPMV,               // k_spmv, k_spmv_rows, k_cg_apply, k_recover, k_residual
+  PK_SPGEMM_VALUES,      // k_spgemm_values
+  PK_SPGEMM_SCATTER,     // k_spgemm_scatter
+  PK_TRSM,               // k_trsm<128>
+  PK_TRSM_SHORT,         // k_trsm<64>
+  PK_INV_GROUP,          // k_inv_group
   PK_COUNT
 };
 

@@ -263,24 +263,33 @@ int hykkt_device_mem_info(unsigned long long* free_bytes, unsigned long long* to
 
 /* Per-kernel timing of the factorization and triangular-solve launches
  * (no counterpart in the reference, which times whole phases with
- * std::chrono in its examples).  While enabled, every launch of the kernels
+ * std::chrono in its examples).  While enabled, every launch of the groups
  * below is bracketed by HIP events on the solver's stream and its duration
  * is summed with the algorithmic flops and HBM bytes it performs:
- *   k_dense_nt<128> / k_dense_nt<32>  MFMA tiles of 128 or 32 rows x 128
- *                 columns: TRSM (r*b^2), panel update and U = -L21 L21^T
- *                 (2*K per lower-triangle entry); the 32-row tiles for the
- *                 short launches on the factorization's critical path
- *   k_potrf_inv   128-column diagonal blocks (b^3/3)
- *   k_extend_add  update-matrix assembly (1 flop, 24 bytes per entry)
- *   k_solve_fwd / k_solve_bwd  one sweep each (2*nnz(L) flops, 8*nnz(L) bytes)
- *   k_spmv        CSR products with Jc, Jc^T, Jd^T (2*nnz flops; indices, values,
- *                 x and y each moved once)
+ *   k_dense_nt<128> / k_dense_nt<32>  panel updates and U = -L21 L21^T with the
+ *                 children's update matrices (2*K per lower-triangle entry, 1 per
+ *                 child entry), and TRSM by whole inverses (r*b^2): tiles of 128 x 128
+ *                 and 64 x 64, and of 32 rows for the short launches on the
+ *                 factorization's critical path
+ *   k_potrf_inv   diagonal blocks (b^3/3); panels of at most 32 columns with their
+ *                 children and TRSM in one launch
+ *   k_trsm<128> / k_trsm<32>  blocked-substitution TRSM (r*b^2) in tiles of 128 and of
+ *                 64 rows
+ *   k_extend_add  children added to the wider panels (1 flop, 24 bytes per entry)
+ *   k_inv_group   inverses of groups of columns, for the sweeps
+ *   k_fwd_forest / k_solve_bwd<256, false>  forward and backward sweep, part of the
+ *                 small supernodes
+ *   k_solve_fwd<1024, true> / k_solve_bwd<1024, true>  the rest of the tree (together
+ *                 2*nnz(L) flops, 8*nnz(L) bytes a sweep)
+ *   k_spmv        CSR products with Jc, Jc^T, Jd^T, recovery and residual rows (2*nnz
+ *                 flops; indices, values, x and y each moved once)
  *   k_spgemm_values / k_spgemm_scatter  H~ and H_gamma values (2 flops and 24
  *                 bytes per term, plus each output entry's indices, D term and
  *                 store)
+ * The names are groups of launches; some are of kernels that others have replaced.
  * hykkt_profile_enable clears the totals; hykkt_profile_get writes up to
- * `capacity` entries, one per kernel launched since, and sets *count to the
- * number of those kernels. */
+ * `capacity` entries, one per group launched since, and sets *count to the
+ * number of those groups. */
 typedef struct {
   char name[32];
   long long launches;
