@@ -25,9 +25,9 @@ sys.path.insert(0, ROOT)
 # Hardware queues.  The served stream runs one solver slot (two streams) per
 # resident pattern concurrently, 16 slots; with fewer queues than streams, slots
 # share queues and their kernels serialise (at 16 queues the served stream ran
-# at 585 solves/s, at 32 at 1,127).  The plain path, one solve at a time, is
-# slower with many queues (its short launches wait longer: 191 solves/s at 4
-# or 16, 96 at 32), and so is any process while another process on the GPU
+# at 887 solves/s, at 32 at 1,430).  The plain path, one solve at a time, is
+# slower with many queues (its short launches wait longer: 312 solves/s at 4
+# or 16, 147 at 32), and so is any process while another process on the GPU
 # holds many queues.  So the served and batched legs run first, in a child
 # process at CONCURRENT_QUEUES, before this process starts the HIP runtime;
 # the headline sequence and the plain legs then run here at HIP's default of

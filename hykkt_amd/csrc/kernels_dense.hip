@@ -532,19 +532,17 @@ __global__ void __launch_bounds__(256, 2) k_trsm_inv(CholDev c, const int* __res
 }
 
 // Factor the diagonal block of step `step` (b <= 128) in LDS, write L_kk back
-// and its inverse (lower triangular, zero-padded to 128 x 128, column-major)
-// to dinv.  LDS holds one BK x (BK+1) array P, padded to BK with the
+// and the inverses of its 16 x 16 diagonal blocks, or its whole inverse (b <= 64),
+// to dinv (lower part).  LDS holds one BK x (BK+1) array P, padded to BK with the
 // identity: L(r, c) (r >= c) at P[r][c], the inverse X(i, j) (i > j) at
 // P[j][i] and X(j, j) at P[j][BK]; and the reciprocals of L's diagonal.
 //
-// Cholesky, blocked by 16-column panels: wave 0 factors the whole panel in
-// registers (two rows per lane; the pivot row's entries reach every lane
-// through v_readlane; 1/sqrt of the pivot is v_rsq_f64 refined by two Newton
-// steps, so the chain carries no division or square root); the trailing
-// lower part takes the rank-16 update as FP64 MFMA 16x16x4 tiles spread over
-// the four waves.  Inverse: the 16x16 diagonal
-// blocks are inverted together (16 lanes per block, lane j computes column
-// j), then blocks of 16, 32 and 64 are doubled with
+// Cholesky, blocked by 16-column panels: one to three waves factor a panel in
+// registers (see potrf_factor; 1/sqrt of the pivot is v_rsq_f64 refined by two Newton
+// steps, so the chain carries no division or square root); the tile columns behind it
+// are updated as FP64 MFMA 16x16x4 tiles.  Inverse: the 16x16 diagonal blocks are
+// inverted together (16 lanes per block, lane j computes column j); for the whole one
+// blocks of 16 and 32 are then doubled with
 //   inv([L11 0; L21 L22]) = [X11 0; -X22 (L21 X11)  X22],
 // both products on the matrix cores; L21 X11 is parked in the slot that
 // -X22 (L21 X11) then overwrites.
